@@ -1,6 +1,7 @@
 import os
 import sys
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -34,4 +35,16 @@ def oracle():
     from oracle import pyoracle
     if not os.path.exists(pyoracle.ORACLE_SO):
         pyoracle.build()
+    if not os.path.exists(pyoracle.TRIREF_SO):
+        # no reference tree to build Triangle from: tests that only need an
+        # input CDT take it from the host builder, tests that compare with
+        # Triangle itself skip
+        pyoracle.triref = lambda: pytest.skip("the reference's Triangle is not built")
+        pyoracle.triangle_cdt = _host_cdt
     return pyoracle
+
+
+def _host_cdt(points, segments):
+    import gpu_cdt_refine_amd as g
+    P = np.ascontiguousarray(points, np.float64).reshape(-1, 2)
+    return (P,) + g.build_cdt(P, segments)
