@@ -615,7 +615,8 @@ enum { SS_PENDING = 0, SS_EXISTS = 1, SS_REGION = 2, SS_SPLIT_EDGE = 3, SS_ERROR
        SS_DEFER = 5, SS_OVER = 6 };
 constexpr int SLIT = -3;  // boundary entry whose far side is in the region
 
-// Triangles incident to each vertex: the smallest slot (deterministic).
+// A triangle incident to each vertex (the smallest slot; later passes keep it
+// up to date where regions are retriangulated).
 __global__ void k_vtri(MeshG m, int nt, int *vtri) {
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += gridDim.x * blockDim.x) {
     const int4 v = m.V[t];
@@ -643,7 +644,15 @@ struct SegOut {
 // triangles its interior crosses up to b or up to the first vertex z lying on
 // it.  Chains: left (vertices left of a->b) and right, in order from a.
 // Boundary edges of the region with their outer otri.
-__device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W, int kseg) {
+//
+// One wave per segment.  The walk is one chain of dependent loads, so every
+// lane follows it (the same addresses: one request each) and lane 0 writes;
+// the slit test at its end, a search of the region for every boundary edge,
+// runs a boundary edge per lane against the region's copy in LDS.
+constexpr int SEG_LDS = 128;  // regions held in LDS; larger ones stay in the workspace
+__device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W, int kseg,
+                           int *sR) {
+  const bool w0 = threadIdx.x == 0;
   SegOut o{SS_ERROR, -1, 0, 0, 0, 0, -1, -1};
   int *R = W;
   int *CL = R + kseg, *CR = CL + (kseg + 2);
@@ -661,8 +670,9 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
   }
   // rotate counterclockwise around a until b lies in the wedge of a triangle
   int x = -1, y = -1, t0 = -1;
+  int4 v0, n0;
   for (int guard = 0; guard < 65536; guard++) {
-    const int4 v = m.V[t];
+    const int4 v = m.V[t], nn = m.N[t];
     const int ia = index_of(v, a);
     if (ia < 0) {
       flag(m, E_TOPOLOGY);
@@ -704,10 +714,12 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
         x = xv;
         y = yv;
         t0 = t;
+        v0 = v;
+        n0 = nn;
         break;
       }
     }
-    const int nb = comp4(m.N[t], (ia + 1) % 3);  // across (a, y): the next triangle ccw
+    const int nb = comp4(nn, (ia + 1) % 3);  // across (a, y): the next triangle ccw
     if (nb < 0 || !tri_ok(m, nb >> 2)) {
       flag(m, E_TOPOLOGY);
       return o;
@@ -720,48 +732,57 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
   }
   // walk across the triangles the segment crosses; x right of a->b, y left
   int n = 0, nl = 0, nr = 0, nbnd = 0;
-  auto add_bnd = [&](int tt, int j) -> bool {
+  auto add_bnd = [&](const int4 &v, const int4 &nn, int j) -> bool {
     if (nbnd == kseg + 2) return false;
-    const int ob = comp4(m.N[tt], j);
+    const int ob = comp4(nn, j);
     if (ob >= 0 && !tri_ok(m, ob >> 2)) {
       flag(m, E_INDEX);
       return false;
     }
-    const int4 v = m.V[tt];
-    Bu[nbnd] = comp4(v, (j + 1) % 3);
-    Bv[nbnd] = comp4(v, (j + 2) % 3);
-    Bo[nbnd] = comp4(m.N[tt], j);
+    if (w0) {
+      Bu[nbnd] = comp4(v, (j + 1) % 3);
+      Bv[nbnd] = comp4(v, (j + 2) % 3);
+      Bo[nbnd] = ob;
+    }
     nbnd++;
     return true;
   };
-  {
-    const int ia = index_of(m.V[t0], a);
-    R[n++] = t0;
-    CR[nr++] = x;
-    CL[nl++] = y;
-    // edges (a, x) (opposite y) and (y, a) (opposite x)
-    if (!add_bnd(t0, (ia + 2) % 3) || !add_bnd(t0, (ia + 1) % 3)) {
-      flag(m, E_CAVITY);
-      return o;
+  auto add_tri = [&](int tt) {
+    if (w0) {
+      R[n] = tt;
+      if (n < SEG_LDS) sR[n] = tt;
     }
+    n++;
+  };
+  int jx = index_of(v0, a);  // crossed edge of the current triangle: opposite a
+  add_tri(t0);
+  if (w0) {
+    CR[0] = x;
+    CL[0] = y;
   }
-  int cur = t0, jx = (index_of(m.V[t0], a));  // crossed edge of cur: opposite a
+  nl = nr = 1;
+  // edges (a, x) (opposite y) and (y, a) (opposite x)
+  if (!add_bnd(v0, n0, (jx + 2) % 3) || !add_bnd(v0, n0, (jx + 1) % 3)) {
+    flag(m, E_CAVITY);
+    return o;
+  }
+  int4 nc = n0;  // neighbours of the current triangle
   int L = y, Rr = x;
   for (int guard = 0; guard < kseg + 8; guard++) {
-    const int nb = comp4(m.N[cur], jx);
+    const int nb = comp4(nc, jx);
     if (nb < 0 || !tri_ok(m, nb >> 2)) {
       flag(m, E_TOPOLOGY);
       return o;
     }
     const int u = nb >> 2, ju = nb & 3;  // in u, the crossed edge is opposite ju
-    const int4 vu = m.V[u];
+    const int4 vu = m.V[u], nu = m.N[u];
     const int z = comp4(vu, ju);
     if (z == m.np || !vert_ok(m, z)) {  // the segment cannot leave the hull
       flag(m, E_TOPOLOGY);
       return o;
     }
     if (n == kseg) return over;
-    R[n++] = u;
+    add_tri(u);
     // u = (z, ., .): the edge (L, z) and the edge (z, Rr) are its other edges
     const int iL = index_of(vu, L), iR = index_of(vu, Rr);
     if (iL < 0 || iR < 0) {
@@ -770,7 +791,7 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
     }
     // edge (z, Rr) is opposite L; edge (L, z) is opposite Rr
     if (z == b) {
-      if (!add_bnd(u, iL) || !add_bnd(u, iR)) return over;
+      if (!add_bnd(vu, nu, iL) || !add_bnd(vu, nu, iR)) return over;
       o.status = SS_REGION;
       o.z = b;
       break;
@@ -778,23 +799,25 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
     const double2 Z = m.P[z];
     const int oz = orient2d_sign(pa.x, pa.y, pb.x, pb.y, Z.x, Z.y, false, nullptr);
     if (oz == 0) {  // the segment passes through z: the region ends here
-      if (!add_bnd(u, iL) || !add_bnd(u, iR)) return over;
+      if (!add_bnd(vu, nu, iL) || !add_bnd(vu, nu, iR)) return over;
       o.status = SS_REGION;
       o.z = z;
       break;
     }
     if (oz > 0) {  // z left: (L, z) is a boundary edge, the segment leaves through (z, Rr)
-      if (!add_bnd(u, iR) || nl == kseg + 2) return over;
-      CL[nl++] = z;
+      if (!add_bnd(vu, nu, iR) || nl == kseg + 2) return over;
+      if (w0) CL[nl] = z;
+      nl++;
       L = z;
       jx = iL;
     } else {  // z right: (z, Rr) is a boundary edge, the segment leaves through (L, z)
-      if (!add_bnd(u, iL) || nr == kseg + 2) return over;
-      CR[nr++] = z;
+      if (!add_bnd(vu, nu, iL) || nr == kseg + 2) return over;
+      if (w0) CR[nr] = z;
+      nr++;
       Rr = z;
       jx = iR;
     }
-    cur = u;
+    nc = nu;
   }
   if (o.status != SS_REGION) {
     flag(m, E_CAVITY);
@@ -804,8 +827,11 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
   // triangles around a chain vertex of degree 3, so that vertex's chain
   // neighbour appears on both sides of it) is a slit of the pseudo-polygon,
   // not a boundary edge: its partner is found among the new triangles.
-  for (int e = 0; e < nbnd; e++)
-    if (Bo[e] >= 0 && in_list(R, n, Bo[e] >> 2)) Bo[e] = SLIT;
+  __syncthreads();  // the lists lane 0 wrote
+  for (int e = threadIdx.x; e < nbnd; e += 64) {
+    const int ob = Bo[e];
+    if (ob >= 0 && (n <= SEG_LDS ? in_list(sR, n, ob >> 2) : in_list(R, n, ob >> 2))) Bo[e] = SLIT;
+  }
   o.n = n;
   o.nl = nl;
   o.nr = nr;
@@ -814,55 +840,55 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
 }
 
 // Per pending segment: scan (above) and record the outcome.
-__global__ void k_seg_scan(MeshG m, const int2 *seg, const int *pend, int npend, const int *vtri,
-                           int *W, int kseg, int4 *info, int4 *info2, int *nover) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < npend; k += gridDim.x * blockDim.x) {
-    const int s = pend[k];
-    const int2 e = seg[s];
-    const SegOut o = seg_scan(m, e.x, e.y, vtri, W + (size_t)k * ws_seg(kseg), kseg);
-    if (o.status == SS_OVER) atomicAdd(nover, 1);
-    info[k] = make_int4(o.status, o.z, o.n, o.nbnd);
-    info2[k] = make_int4(o.nl, o.nr, o.t_edge, o.j_edge);
+__global__ __launch_bounds__(64) void k_seg_scan(MeshG m, const int2 *seg, const int *pend,
+                                                 int npend, const int *vtri, int *W, int kseg,
+                                                 int4 *info, int4 *info2, int *nover) {
+  __shared__ int sR[SEG_LDS];
+  for (int k = blockIdx.x; k < npend; k += gridDim.x) {
+    const int2 e = seg[pend[k]];
+    const SegOut o = seg_scan(m, e.x, e.y, vtri, W + (size_t)k * ws_seg(kseg), kseg, sR);
+    if (threadIdx.x == 0) {
+      if (o.status == SS_OVER) atomicAdd(nover, 1);
+      info[k] = make_int4(o.status, o.z, o.n, o.nbnd);
+      info2[k] = make_int4(o.nl, o.nr, o.t_edge, o.j_edge);
+    }
+    __syncthreads();  // sR is reused
   }
 }
 
-// Claims on the region and its ring; existing edges need none.
-__global__ void k_seg_claim(MeshG m, int npend, const int *W, int kseg, const int4 *info,
-                            unsigned long long ep) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < npend; k += gridDim.x * blockDim.x) {
+// Claims on the region and its ring (one wave per segment, an entry per
+// lane); existing edges need none.
+__global__ __launch_bounds__(64) void k_seg_claim(MeshG m, int npend, const int *W, int kseg,
+                                                  const int4 *info, unsigned long long ep) {
+  for (int k = blockIdx.x; k < npend; k += gridDim.x) {
     const int4 in = info[k];
     if (in.x != SS_REGION) continue;
     const int *Wk = W + (size_t)k * ws_seg(kseg);
     const int *R = Wk, *Bo = Wk + bo_off(kseg);
     const unsigned long long key = claim_key(ep, k);
-    for (int q = 0; q < in.z; q++) atomicMax(&m.claim[2 * (size_t)R[q]], key);
-    for (int q = 0; q < in.w; q++)
+    for (int q = threadIdx.x; q < in.z; q += 64) atomicMax(&m.claim[2 * (size_t)R[q]], key);
+    for (int q = threadIdx.x; q < in.w; q += 64)
       if (Bo[q] >= 0) atomicMax(&m.claim[2 * (size_t)(Bo[q] >> 2)], key);
   }
 }
 
-__global__ void k_seg_win(MeshG m, int npend, const int *W, int kseg, const int4 *info,
-                          unsigned long long ep, int *win) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < npend; k += gridDim.x * blockDim.x) {
+__global__ __launch_bounds__(64) void k_seg_win(MeshG m, int npend, const int *W, int kseg,
+                                                const int4 *info, unsigned long long ep,
+                                                int *win) {
+  for (int k = blockIdx.x; k < npend; k += gridDim.x) {
     const int4 in = info[k];
-    int w = 0;
-    if (in.x == SS_REGION) {
+    bool lose = in.x != SS_REGION;
+    if (!lose) {
       const int *Wk = W + (size_t)k * ws_seg(kseg);
       const int *R = Wk, *Bo = Wk + bo_off(kseg);
       const unsigned long long key = claim_key(ep, k);
-      w = 1;
-      for (int q = 0; q < in.z && w; q++) w = m.claim[2 * (size_t)R[q]] == key;
-      for (int q = 0; q < in.w && w; q++)
-        if (Bo[q] >= 0) w = m.claim[2 * (size_t)(Bo[q] >> 2)] == key;
+      for (int q = threadIdx.x; q < in.z; q += 64) lose |= m.claim[2 * (size_t)R[q]] != key;
+      for (int q = threadIdx.x; q < in.w; q += 64)
+        if (Bo[q] >= 0) lose |= m.claim[2 * (size_t)(Bo[q] >> 2)] != key;
     }
-    win[k] = w;
+    const bool w = __ballot(lose) == 0ull;
+    if (threadIdx.x == 0) win[k] = w;
   }
-}
-
-// exact-sign incircle of real vertices (filters, double-double, expansion)
-__device__ inline int incircle_v(const MeshG &m, int a, int b, int c, int d, double *ws) {
-  const double2 A = m.P[a], B = m.P[b], C = m.P[c], D = m.P[d];
-  return incircle_sign(A.x, A.y, B.x, B.y, C.x, C.y, D.x, D.y, ws, false, nullptr);
 }
 
 // The segment pieces recovered so far: (input segment, from, to).
@@ -878,157 +904,212 @@ struct Piece {
 // triangles take the region's slots in ascending order; their links are
 // matched edge by edge, inside the region or to the boundary's outer
 // triangles (whose back-links are repaired).
-__global__ void k_seg_apply(MeshG m, const int2 *seg_cur, const int *pend, int npend, int *W,
-                            int kseg, const int4 *info, const int4 *info2, const int *win, double *arena,
-                            Piece *pieces, int *npieces, int pcap, int2 *seg_next, int *done) {
-  const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-  double *ws = arena + (size_t)lane * GCDT_INCIRCLE_WS;
-  for (int k = lane; k < npend; k += gridDim.x * blockDim.x) {
+//
+// One wave per region, its chains, triangles and slots in LDS (regions of up
+// to SEG_LDS triangles; larger ones use the workspace).  The base of a
+// sub-problem (lo, hi) is (vertex lo - 1, vertex hi + 1) of its chain with
+// the end points at -1 and cnt, so a stack entry is two ints.  The scan for
+// the best vertex tests 64 chain vertices at a time against the current best
+// and restarts behind the first that replaces it: the sequential scan's
+// result.  Links are a search per edge, one edge per lane.  (One lane per
+// region through global memory was bound by its serial chain of loads:
+// 2.9 ms a pass at 4,000 points, regions of 18 to 77 triangles.)
+//
+// FAST: an incircle sign neither the filter nor the double-double stage
+// decides defers the region, before any write to the mesh, to the exact
+// kernel, whose grid the expansion arena covers.
+template <bool FAST>
+__global__ __launch_bounds__(64) void k_seg_apply(MeshG m, int2 *seg, const int *pend, int npend,
+                                                  int *W, int kseg, const int4 *info,
+                                                  const int4 *info2, const int *win,
+                                                  double *arena, Piece *pieces, int *npieces,
+                                                  int pcap, int *done, int *vtri, int *slow,
+                                                  int *nslow) {
+  __shared__ int s_id[SEG_LDS + 2], s_nt[3 * SEG_LDS], s_r[SEG_LDS], s_stk[2 * (SEG_LDS + 2)];
+  __shared__ double2 s_xy[SEG_LDS + 2];
+  const int lane = threadIdx.x;
+  double *ws = FAST ? nullptr : arena + ((size_t)blockIdx.x * 64 + lane) * GCDT_INCIRCLE_WS;
+  const int nwork = FAST ? npend : *nslow;
+  for (int it = blockIdx.x; it < nwork; it += gridDim.x) {
+    const int k = FAST ? it : slow[it];
     if (!win[k]) continue;
     const int s = pend[k];
-    const int a = seg_cur[s].x, b = seg_cur[s].y;
+    const int a = seg[s].x, b = seg[s].y;
     const int4 in = info[k], in2 = info2[k];
     const int z = in.y, n = in.z, nbnd = in.w, nl = in2.x, nr = in2.y;
     int *R = W + (size_t)k * ws_seg(kseg);
     int *CL = R + kseg, *CR = CL + (kseg + 2);
     int *Bu = CR + (kseg + 2), *Bv = Bu + (kseg + 2), *Bo = Bv + (kseg + 2);
-    int *NT = Bo + (kseg + 2);
-    int *STK = NT + 3 * (size_t)kseg;
+    const bool lds = n <= SEG_LDS;
+    int *NT = lds ? s_nt : Bo + (kseg + 2);
+    int *STK = lds ? s_stk : Bo + (kseg + 2) + 3 * (size_t)kseg;
     if (nl + nr != n || n > kseg || nl < 1 || nr < 1) {
       flag(m, E_TOPOLOGY);
       continue;
     }
     int ne = 0;
-    bool bad = false;
-    for (int side = 0; side < 2 && !bad; side++) {
+    bool bad = false, undecided = false;
+    for (int side = 0; side < 2 && !bad && !undecided; side++) {
       // side 0: base (a, z), chain CL in order; side 1: base (z, a), chain CR reversed
       const int cnt = side == 0 ? nl : nr;
-      int sp = 0;
-      STK[0] = side == 0 ? a : z;
-      STK[1] = side == 0 ? z : a;
-      STK[2] = 0;
-      STK[3] = cnt - 1;
-      sp = 1;
-      while (sp > 0) {
-        sp--;
-        const int x = STK[4 * sp], y = STK[4 * sp + 1], lo = STK[4 * sp + 2], hi = STK[4 * sp + 3];
-        if (lo > hi) continue;
-        int best = lo;
-        for (int i = lo + 1; i <= hi; i++) {
-          const int cb = side == 0 ? CL[best] : CR[nr - 1 - best];
-          const int ci = side == 0 ? CL[i] : CR[nr - 1 - i];
-          if (incircle_v(m, x, y, cb, ci, ws) > 0) best = i;
+      const int ex = side == 0 ? a : z, ey = side == 0 ? z : a;
+      auto chain = [&](int i) {  // vertex i of the chain, end points at -1 and cnt
+        return i < 0 ? ex : (i >= cnt ? ey : (side == 0 ? CL[i] : CR[nr - 1 - i]));
+      };
+      __syncthreads();  // the previous side's (or region's) LDS use has ended
+      if (lds)
+        for (int i = lane - 1; i <= cnt; i += 64) {
+          const int c = chain(i);
+          s_id[i + 1] = c;
+          s_xy[i + 1] = m.P[c];
         }
-        const int c = side == 0 ? CL[best] : CR[nr - 1 - best];
-        if (ne == n || sp + 2 > kseg + 2) {
+      auto id = [&](int i) { return lds ? s_id[i + 1] : chain(i); };
+      auto xy = [&](int i) { return lds ? s_xy[i + 1] : m.P[chain(i)]; };
+      int sp = 1;
+      if (lane == 0) {
+        STK[0] = 0;
+        STK[1] = cnt - 1;
+      }
+      while (sp > 0) {
+        __syncthreads();  // the stack's top
+        sp--;
+        const int lo = STK[2 * sp], hi = STK[2 * sp + 1];
+        const double2 X = xy(lo - 1), Y = xy(hi + 1);
+        int best = lo;
+        for (int pos = lo + 1; pos <= hi && !undecided;) {
+          const double2 Cb = xy(best);
+          const int i = pos + lane;
+          bool in_c = false, und = false;
+          if (i <= hi) {
+            const double2 D = xy(i);
+            int sg = incircle_filtered(X.x, X.y, Y.x, Y.y, Cb.x, Cb.y, D.x, D.y, false, nullptr);
+            if (sg == PRED_UNSURE) {
+              if (FAST) {
+                sg = incircle_dd_sign(X.x, X.y, Y.x, Y.y, Cb.x, Cb.y, D.x, D.y);
+                und = sg == 0;
+              } else {
+                sg = incircle_sign(X.x, X.y, Y.x, Y.y, Cb.x, Cb.y, D.x, D.y, ws, false, nullptr);
+              }
+            }
+            in_c = sg > 0;
+          }
+          if (__ballot(und) != 0ull) {
+            undecided = true;
+            break;
+          }
+          const unsigned long long bal = __ballot(in_c);
+          if (bal == 0ull) {
+            pos += 64;
+          } else {
+            best = pos + __builtin_ctzll(bal);
+            pos = best + 1;
+          }
+        }
+        if (undecided) break;
+        if (ne == n) {
           bad = true;
           break;
         }
-        NT[3 * ne] = x;
-        NT[3 * ne + 1] = y;
-        NT[3 * ne + 2] = c;
+        if (lane == 0) {
+          NT[3 * ne] = id(lo - 1);
+          NT[3 * ne + 1] = id(hi + 1);
+          NT[3 * ne + 2] = id(best);
+        }
         ne++;
-        STK[4 * sp] = x;
-        STK[4 * sp + 1] = c;
-        STK[4 * sp + 2] = lo;
-        STK[4 * sp + 3] = best - 1;
-        sp++;
-        STK[4 * sp] = c;
-        STK[4 * sp + 1] = y;
-        STK[4 * sp + 2] = best + 1;
-        STK[4 * sp + 3] = hi;
-        sp++;
+        __syncthreads();  // everyone has read the entry its successor overwrites
+        if (lo <= best - 1) {
+          if (lane == 0) {
+            STK[2 * sp] = lo;
+            STK[2 * sp + 1] = best - 1;
+          }
+          sp++;
+        }
+        if (best + 1 <= hi) {
+          if (lane == 0) {
+            STK[2 * sp] = best + 1;
+            STK[2 * sp + 1] = hi;
+          }
+          sp++;
+        }
       }
+    }
+    if (undecided) {
+      if (lane == 0) slow[atomicAdd(nslow, 1)] = k;
+      continue;
     }
     if (bad || ne != n) {
       flag(m, E_TOPOLOGY);
       continue;
     }
-    // region slots in ascending order
-    for (int i = 1; i < n; i++) {
-      const int x = R[i];
-      int j = i - 1;
-      while (j >= 0 && R[j] > x) {
-        R[j + 1] = R[j];
-        j--;
-      }
-      R[j + 1] = x;
+    // region slots in ascending order (distinct: the rank is the position)
+    __syncthreads();
+    int *SR = lds ? s_r : STK;
+    for (int e = lane; e < n; e += 64) {
+      const int v = R[e];
+      int rank = 0;
+      for (int x = 0; x < n; x++) rank += R[x] < v;
+      SR[rank] = v;
     }
-    // links: first find every edge's partner, then write
+    __syncthreads();
     bool ok = true;
-    for (int q = 0; q < n && ok; q++) {
-      const int st = R[q];
-      int nn[3];
-      for (int j = 0; j < 3 && ok; j++) {
-        const int u = NT[3 * q + (j + 1) % 3], v = NT[3 * q + (j + 2) % 3];
-        int link = -2;
-        for (int q2 = 0; q2 < n && link == -2; q2++) {
-          if (q2 == q) continue;
-          for (int j2 = 0; j2 < 3; j2++)
-            if (NT[3 * q2 + (j2 + 1) % 3] == v && NT[3 * q2 + (j2 + 2) % 3] == u) {
-              link = (R[q2] << 2) | j2;
-              break;
-            }
-        }
-        if (link == -2)
-          for (int e = 0; e < nbnd; e++)
-            if (Bu[e] == u && Bv[e] == v && Bo[e] != SLIT) {
-              link = Bo[e];
-              break;
-            }
-        if (link == -2) ok = false;
-        nn[j] = link;
+    for (int it3 = lane; it3 < 3 * n; it3 += 64) {
+      const int q = it3 / 3, j = it3 % 3, st = SR[q];
+      const int u = NT[3 * q + (j + 1) % 3], v = NT[3 * q + (j + 2) % 3];
+      int link = -2;
+      for (int q2 = 0; q2 < n && link == -2; q2++) {
+        const int A = NT[3 * q2], B = NT[3 * q2 + 1], C = NT[3 * q2 + 2];
+        const int j2 = (B == v && C == u) ? 0 : ((C == v && A == u) ? 1 : ((A == v && B == u) ? 2 : -1));
+        if (j2 >= 0) link = (SR[q2] << 2) | j2;
       }
-      if (!ok) break;
-      m.V[st] = make_int4(NT[3 * q], NT[3 * q + 1], NT[3 * q + 2], 0);
-      m.N[st] = make_int4(nn[0], nn[1], nn[2], 0);
+      if (link == -2)
+        for (int e = 0; e < nbnd; e++)
+          if (Bu[e] == u && Bv[e] == v && Bo[e] != SLIT) {
+            link = Bo[e];
+            // the outer triangle's back-link
+            if (link >= 0) reinterpret_cast<int *>(&m.N[link >> 2])[link & 3] = (st << 2) | j;
+            break;
+          }
+      if (link == -2) {
+        ok = false;
+        continue;
+      }
+      reinterpret_cast<int *>(&m.N[st])[j] = link;
+      reinterpret_cast<int *>(&m.V[st])[j] = NT[it3];
+      vtri[NT[it3]] = st;  // any triangle at the vertex serves the next pass's scans
     }
-    if (!ok) {
+    if (__ballot(!ok) != 0ull) {
       flag(m, E_TOPOLOGY);
       continue;
     }
-    // back-links of the outer triangles
-    for (int q = 0; q < n; q++) {
-      const int st = R[q];
-      for (int j = 0; j < 3; j++) {
-        const int u = NT[3 * q + (j + 1) % 3], v = NT[3 * q + (j + 2) % 3];
-        for (int e = 0; e < nbnd; e++)
-          if (Bu[e] == u && Bv[e] == v && Bo[e] >= 0) {
-            const int o = Bo[e];
-            int *slot = reinterpret_cast<int *>(&m.N[o >> 2]) + (o & 3);
-            *slot = (st << 2) | j;
-            break;
-          }
+    if (lane == 0) {
+      const int pi = atomicAdd(npieces, 1);
+      if (pi >= pcap) {
+        flag(m, E_CAVITY);
+      } else {
+        pieces[pi] = Piece{s, a, z, 0};
+        seg[s] = make_int2(z, b);
+        done[s] = z == b;
       }
     }
-    const int pi = atomicAdd(npieces, 1);
-    if (pi >= pcap) {
-      flag(m, E_CAVITY);
-      continue;
-    }
-    pieces[pi] = Piece{s, a, z, 0};
-    seg_next[s] = make_int2(z, b);
-    done[s] = z == b;
   }
 }
 
 // Segments that are (or begin with) an existing edge: record the piece and
 // continue from its end.
-__global__ void k_seg_edges(MeshG m, const int2 *seg_cur, const int *pend, int npend,
-                            const int4 *info, Piece *pieces, int *npieces, int pcap,
-                            int2 *seg_next, int *done) {
+__global__ void k_seg_edges(MeshG m, int2 *seg, const int *pend, int npend, const int4 *info,
+                            Piece *pieces, int *npieces, int pcap, int *done) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < npend; k += gridDim.x * blockDim.x) {
     const int4 in = info[k];
     if (in.x != SS_EXISTS && in.x != SS_SPLIT_EDGE) continue;
     const int s = pend[k];
-    const int a = seg_cur[s].x, b = seg_cur[s].y, z = in.y;
+    const int a = seg[s].x, b = seg[s].y, z = in.y;
     const int pi = atomicAdd(npieces, 1);
     if (pi >= pcap) {
       flag(m, E_CAVITY);
       continue;
     }
     pieces[pi] = Piece{s, a, z, 0};
-    seg_next[s] = make_int2(z, b);
+    seg[s] = make_int2(z, b);
     done[s] = z == b;
   }
 }
@@ -1395,7 +1476,7 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
   }
   if (tbase != cap) throw std::runtime_error("CDT insertion left unused slots (duplicate points?)");
   // ---- phase 2: constraint recovery ----
-  int2 *seg_cur = B.alloc<int2>(ns), *seg_next = B.alloc<int2>(ns);
+  int2 *seg = B.alloc<int2>(ns);
   int *done = B.alloc<int>(ns);
   int *pend = B.alloc<int>(ns), *pend2 = B.alloc<int>(ns);
   int *vtri = B.alloc<int>(np);
@@ -1406,7 +1487,7 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
   int *swin = nullptr, *W2 = nullptr;
   int seg_passes = 0, npieces_total = 0;
   if (ns > 0) {
-    CC(hipMemcpyAsync(seg_cur, segs, sizeof(int2) * ns, hipMemcpyHostToDevice, B.st));
+    CC(hipMemcpyAsync(seg, segs, sizeof(int2) * ns, hipMemcpyHostToDevice, B.st));
     CC(hipMemsetAsync(done, 0, sizeof(int) * ns, B.st));
     CC(hipMemsetAsync(npieces, 0, sizeof(int), B.st));
     std::vector<int> hp(ns);
@@ -1416,31 +1497,32 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
     info = B.alloc<int4>(SBATCH);
     info2 = B.alloc<int4>(SBATCH);
     swin = B.alloc<int>(SBATCH);
+    int *sslow = B.alloc<int>(SBATCH);
     int kseg = KSEG0;
     size_t w2_ints = (size_t)SBATCH * ws_seg(kseg);
     W2 = B.alloc<int>(w2_ints);
-    int *nover = B.alloc<int>(1);
+    int *nover = B.alloc<int>(2);  // regions over capacity; regions left to the exact kernel
     int npend = ns;
     int last_pieces = -1;
+    CC(hipMemsetAsync(vtri, 0x7f, sizeof(int) * np, B.st));
+    k_vtri<<<Builder::grid(cap), BLK, 0, B.st>>>(m, cap, vtri);
     while (npend > 0) {
       if (++seg_passes > 1000000) throw std::runtime_error("segment recovery did not finish");
       const int batch = (int)std::min<size_t>(SBATCH, w2_ints / ws_seg(kseg));
       const int nb = std::min(npend, batch);
-      CC(hipMemsetAsync(nover, 0, sizeof(int), B.st));
-      CC(hipMemsetAsync(vtri, 0x7f, sizeof(int) * np, B.st));
-      k_vtri<<<Builder::grid(cap), BLK, 0, B.st>>>(m, cap, vtri);
-      k_seg_scan<<<Builder::grid(nb, 64), 64, 0, B.st>>>(m, seg_cur, pend, nb, vtri, W2, kseg,
-                                                          info, info2, nover);
-      CC(hipMemcpyAsync(seg_next, seg_cur, sizeof(int2) * ns, hipMemcpyDeviceToDevice, B.st));
-      k_seg_edges<<<Builder::grid(nb), BLK, 0, B.st>>>(m, seg_cur, pend, nb, info, pieces,
-                                                       npieces, PCAP, seg_next, done);
+      CC(hipMemsetAsync(nover, 0, 2 * sizeof(int), B.st));
+      k_seg_scan<<<nb, 64, 0, B.st>>>(m, seg, pend, nb, vtri, W2, kseg, info, info2, nover);
+      k_seg_edges<<<Builder::grid(nb), BLK, 0, B.st>>>(m, seg, pend, nb, info, pieces, npieces,
+                                                       PCAP, done);
       cep++;
-      k_seg_claim<<<Builder::grid(nb), BLK, 0, B.st>>>(m, nb, W2, kseg, info, cep);
-      k_seg_win<<<Builder::grid(nb), BLK, 0, B.st>>>(m, nb, W2, kseg, info, cep, swin);
-      k_seg_apply<<<EXACT_GRID, 64, 0, B.st>>>(m, seg_cur, pend, nb, W2, kseg, info, info2, swin,
-                                               arena, pieces, npieces, PCAP, seg_next, done);
+      k_seg_claim<<<nb, 64, 0, B.st>>>(m, nb, W2, kseg, info, cep);
+      k_seg_win<<<nb, 64, 0, B.st>>>(m, nb, W2, kseg, info, cep, swin);
+      k_seg_apply<true><<<nb, 64, 0, B.st>>>(m, seg, pend, nb, W2, kseg, info, info2, swin, arena,
+                                             pieces, npieces, PCAP, done, vtri, sslow, nover + 1);
+      k_seg_apply<false><<<std::min(nb, EXACT_GRID), 64, 0, B.st>>>(
+          m, seg, pend, nb, W2, kseg, info, info2, swin, arena, pieces, npieces, PCAP, done, vtri,
+          sslow, nover + 1);
       CC(hipGetLastError());
-      CC(hipMemcpyAsync(seg_cur, seg_next, sizeof(int2) * ns, hipMemcpyDeviceToDevice, B.st));
       k_seg_pending_flags<<<Builder::grid(ns), BLK, 0, B.st>>>(done, ns, flags);
       CC(hipGetLastError());
       npend = B.compact(flags, ns, nullptr, pend2, nullptr);
