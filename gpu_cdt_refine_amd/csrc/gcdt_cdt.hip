@@ -65,7 +65,9 @@ enum : unsigned {
   E_WALK = 2u,      // a walk exceeded its step cap
   E_CAVITY = 4u,    // a cavity or segment region exceeded its capacity
   E_TOPOLOGY = 8u,  // inconsistent neighbour links
-  E_DUPLICATE = 16u // two input points coincide
+  E_DUPLICATE = 16u, // two input points coincide
+  E_STALL = 32u,    // an insertion round without a candidate or a winner
+  E_SLOTS = 64u     // more triangles than 2 np - 2
 };
 
 constexpr int BLK = 256;
@@ -178,17 +180,16 @@ __device__ int locate(const MeshG &m, int t, double2 p, bool *on_vertex) {
       t = nb >> 2;
       continue;
     }
-    int jn = -1, zeros = 0;
-    for (int j = 0; j < 3; j++) {
-      const int a = comp4(v, (j + 1) % 3), b = comp4(v, (j + 2) % 3);
-      if (!vert_ok(m, a) || !vert_ok(m, b)) {
-        flag(m, E_INDEX);
-        return -1;
-      }
-      const int o = orient_v(m, a, b, p);
-      if (o < 0 && jn < 0) jn = j;
-      zeros += o == 0;
+    if (!vert_ok(m, v.x) || !vert_ok(m, v.y) || !vert_ok(m, v.z)) {
+      flag(m, E_INDEX);
+      return -1;
     }
+    const double2 A = m.P[v.x], B = m.P[v.y], C = m.P[v.z];
+    const int o0 = orient2d_sign(B.x, B.y, C.x, C.y, p.x, p.y, false, nullptr);
+    const int o1 = orient2d_sign(C.x, C.y, A.x, A.y, p.x, p.y, false, nullptr);
+    const int o2 = orient2d_sign(A.x, A.y, B.x, B.y, p.x, p.y, false, nullptr);
+    const int jn = o0 < 0 ? 0 : (o1 < 0 ? 1 : (o2 < 0 ? 2 : -1));
+    const int zeros = (o0 == 0) + (o1 == 0) + (o2 == 0);
     if (jn < 0) {
       if (zeros >= 2) *on_vertex = true;
       return t;
@@ -247,8 +248,15 @@ __device__ inline unsigned long long pick_key(const MeshG &m, unsigned long long
          (unsigned long long)(0xffffffffu - (unsigned)i);
 }
 
-__global__ void k_pick(MeshG m, const int *U, int nu, const int *ptri,
+// Device-resident state of the insertion rounds: the counts every kernel of a
+// round reads, so that rounds follow each other without a host round trip.
+// The uninserted points are counted in two words used in turn (a compaction
+// reads one and writes the other).
+enum { D_NU = 0, D_NC = 2, D_NW, D_TBASE, D_NSLOW, D_ROUNDS, D_N = 8 };
+
+__global__ void k_pick(MeshG m, const int *U, const int *cnt, int par, const int *ptri,
                        unsigned long long *pick, unsigned long long ep) {
+  const int nu = cnt[D_NU + par];
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nu; k += gridDim.x * blockDim.x) {
     const int i = U[k];
     const int t = ptri[i];
@@ -260,13 +268,134 @@ __global__ void k_pick(MeshG m, const int *U, int nu, const int *ptri,
   }
 }
 
-__global__ void k_cand_flags(MeshG m, const int *U, int nu, const int *ptri,
-                             const unsigned long long *pick, unsigned long long ep, int *flag_out) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nu; k += gridDim.x * blockDim.x) {
+// Candidates of a round: the points their triangle picked.
+struct PredCand {
+  MeshG m;
+  const int *U, *ptri;
+  const unsigned long long *pick;
+  unsigned long long ep;
+  __device__ bool operator()(int k) const {
     const int i = U[k];
     const int t = ptri[i];
-    flag_out[k] = tri_ok(m, t) && pick[t] == pick_key(m, ep, i, t);
+    return tri_ok(m, t) && pick[t] == pick_key(m, ep, i, t);
   }
+};
+struct PredIns {  // winners
+  const int *win;
+  __device__ bool operator()(int k) const { return win[k] != 0; }
+};
+struct PredOut {  // points not inserted yet
+  const int *U, *ptri;
+  __device__ bool operator()(int k) const { return ptri[U[k]] >= 0; }
+};
+// What a round's compaction does with its total.
+struct FinCand {
+  int *cnt;
+  unsigned *err;
+  int par, cmax;
+  __device__ void operator()(int total) const {
+    cnt[D_NC] = total < cmax ? total : cmax;
+    cnt[D_NSLOW] = 0;
+    if (cnt[D_NU + par] > 0) {
+      cnt[D_ROUNDS]++;
+      if (total == 0) atomicOr(err, E_STALL);
+    }
+  }
+};
+struct FinIns {
+  int *cnt;
+  unsigned *err;
+  int cap;
+  __device__ void operator()(int total) const {
+    cnt[D_NW] = total;
+    if (cnt[D_NC] > 0 && total == 0) atomicOr(err, E_STALL);
+    if ((long long)cnt[D_TBASE] + 2LL * total > cap) atomicOr(err, E_SLOTS);
+  }
+};
+struct FinOut {
+  int *cnt;
+  int par;
+  __device__ void operator()(int total) const {
+    cnt[D_NU + (par ^ 1)] = total;
+    cnt[D_TBASE] += 2 * cnt[D_NW];
+  }
+};
+
+// Ordered compaction of [0, *n) by pred: out[r] = src[k] (or k) and rank[k] =
+// r for the k it holds for, in ascending k.  Up to one tile: one block in one
+// launch; else tile counts, then a scatter whose blocks sum the counts before
+// their tile.  fin receives the total.
+constexpr int CMP_THREADS = 1024, CMP_ITEMS = 4, CMP_TILE = CMP_THREADS * CMP_ITEMS;
+template <class Pred>
+__device__ __forceinline__ int compact_tile(const Pred &pred, int n, int base, int run, int *out,
+                                            int *rank, const int *src) {
+  __shared__ int wcnt[CMP_ITEMS][CMP_THREADS / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned long long b[CMP_ITEMS];
+#pragma unroll
+  for (int q = 0; q < CMP_ITEMS; q++) {
+    const int k = base + q * CMP_THREADS + (int)threadIdx.x;
+    b[q] = __ballot(k < n && pred(k));
+    if (lane == 0) wcnt[q][wave] = __popcll(b[q]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < CMP_ITEMS; q++) {
+    int pre = 0, tot = 0;
+    for (int w = 0; w < CMP_THREADS / 64; w++) {
+      const int c = wcnt[q][w];
+      pre += w < wave ? c : 0;
+      tot += c;
+    }
+    if ((b[q] >> lane) & 1ull) {
+      const int k = base + q * CMP_THREADS + (int)threadIdx.x;
+      const int pos = run + pre + __popcll(b[q] & ((1ull << lane) - 1ull));
+      if (out) out[pos] = src ? src[k] : k;
+      if (rank) rank[k] = pos;
+    }
+    run += tot;
+  }
+  __syncthreads();
+  return run;
+}
+template <class Pred, class Fin>
+__global__ __launch_bounds__(CMP_THREADS) void k_compact_one(Pred pred, const int *n, int *out,
+                                                             int *rank, const int *src, Fin fin) {
+  const int total = compact_tile(pred, min(*n, CMP_TILE), 0, 0, out, rank, src);
+  if (threadIdx.x == 0) fin(total);
+}
+template <class Pred>
+__global__ __launch_bounds__(CMP_THREADS) void k_compact_count(Pred pred, const int *n, int *tiles) {
+  __shared__ int wsum[CMP_THREADS / 64];
+  const int base = blockIdx.x * CMP_TILE, nn = *n;
+  int c = 0;
+  for (int q = 0; q < CMP_ITEMS; q++) {
+    const int k = base + q * CMP_THREADS + (int)threadIdx.x;
+    c += __popcll(__ballot(k < nn && pred(k)));
+  }
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+    for (int w = 0; w < CMP_THREADS / 64; w++) t += wsum[w];
+    tiles[blockIdx.x] = t;
+  }
+}
+template <class Pred, class Fin>
+__global__ __launch_bounds__(CMP_THREADS) void k_compact_scatter(Pred pred, const int *n,
+                                                                 const int *tiles, int *out,
+                                                                 int *rank, const int *src,
+                                                                 Fin fin) {
+  __shared__ int wsum[CMP_THREADS / 64];
+  int c = 0;
+  for (int b = threadIdx.x; b < (int)blockIdx.x; b += CMP_THREADS) c += tiles[b];
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off, 64);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = c;
+  __syncthreads();
+  int run = 0;
+  for (int w = 0; w < CMP_THREADS / 64; w++) run += wsum[w];
+  run = compact_tile(pred, *n, blockIdx.x * CMP_TILE, run, out, rank, src);
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) fin(run);
 }
 
 enum { CS_NONE = 0, CS_VALID = 1, CS_DEFER = 2, CS_OVERFLOW = 3 };
@@ -275,8 +404,7 @@ enum { CS_NONE = 0, CS_VALID = 1, CS_DEFER = 2, CS_OVERFLOW = 3 };
 // reachable across edges (ghost triangles by the half-plane rule), sorted by
 // slot; the boundary in star order (starting at the edge with the smallest
 // origin vertex), written to the candidate's workspace as cavity | u | v |
-// outer.  FAST: undecided incircle signs defer the candidate.
-template <bool FAST>
+// outer.  One lane, exact signs: the candidates the grouped kernel defers.
 __device__ void cavity_one(const MeshG &m, int c, int seed, int *W, int *status, int *ncav,
                            double *ws) {
   const double2 p = m.P[c];
@@ -287,11 +415,7 @@ __device__ void cavity_one(const MeshG &m, int c, int seed, int *W, int *status,
     *status = CS_NONE;
     return;
   }
-  int c0 = conflict<FAST>(m, seed, p, ws);
-  if (c0 == PRED_UNSURE) {
-    *status = CS_DEFER;
-    return;
-  }
+  int c0 = conflict<false>(m, seed, p, ws);
   if (c0 != 1) {  // the stored triangle must contain (or see) the point
     flag(m, E_TOPOLOGY);
     *status = CS_NONE;
@@ -311,11 +435,7 @@ __device__ void cavity_one(const MeshG &m, int c, int seed, int *W, int *status,
         return;
       }
       if (in_list(L, n, u)) continue;
-      const int cf = conflict<FAST>(m, u, p, ws);
-      if (cf == PRED_UNSURE) {
-        *status = CS_DEFER;
-        return;
-      }
+      const int cf = conflict<false>(m, u, p, ws);
       if (cf == 1) {
         if (n == KCAV) {
           *status = CS_OVERFLOW;
@@ -386,30 +506,198 @@ __device__ void cavity_one(const MeshG &m, int c, int seed, int *W, int *status,
   *status = CS_VALID;
 }
 
-__global__ void k_ins_cavity_fast(MeshG m, const int *C, int nc, const int *ptri, int *W,
-                                  int *cstat, int *cn, int *slow, int *nslow) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += gridDim.x * blockDim.x) {
-    const int c = C[k];
-    int st = CS_NONE, n = 0;
-    cavity_one<true>(m, c, ptri[c], W + (size_t)k * WS_INS, &st, &n, nullptr);
-    cstat[k] = st;
-    cn[k] = n;
-    if (st == CS_DEFER) slow[atomicAdd(nslow, 1)] = k;
+// The same cavity by a group of INS_LANES lanes, four candidates a wave: the
+// cavity grows level by level with the edges of a level's triangles tested in
+// parallel (membership is an LDS hash set, so the set does not depend on the
+// order), slots are rank-sorted, boundary edges linked by a search per lane.
+// Undecided incircle signs and cavities of more than INS_K triangles defer
+// the candidate to the exact kernel.  The kernel is bound by its chain of
+// dependent gathers (slot, vertices, coordinates per level); one lane per
+// candidate made that chain one round trip per tested triangle.
+constexpr int INS_LANES = 16, INS_K = 32, INS_HASH = 128;
+constexpr int INS_GROUP_INTS = (INS_K + INS_LANES) + INS_K + INS_HASH + 5 * (INS_K + 2) + 4;
+enum { IS_N = 0, IS_NB, IS_DEFER, IS_BAD };
+
+__device__ __forceinline__ unsigned ins_hash(int x) {
+  const unsigned h = (unsigned)x * 0x9E3779B1u;
+  return (h ^ (h >> 15)) & (INS_HASH - 1);
+}
+// true if x was absent (and is now present); fewer than INS_HASH / 2 inserts
+__device__ __forceinline__ bool ins_add(int *h, int x) {
+  for (unsigned k = ins_hash(x);; k = (k + 1) & (INS_HASH - 1)) {
+    const int prev = atomicCAS(&h[k], -1, x);
+    if (prev == -1) return true;
+    if (prev == x) return false;
+  }
+}
+__device__ __forceinline__ bool ins_has(const int *h, int x) {
+  for (unsigned k = ins_hash(x);; k = (k + 1) & (INS_HASH - 1)) {
+    const int v = h[k];
+    if (v == x) return true;
+    if (v == -1) return false;
+  }
+}
+
+__global__ __launch_bounds__(64) void k_ins_cavity_fast(MeshG m, const int *C, int *cnt,
+                                                        const int *ptri, int *W, int *cstat,
+                                                        int *cn, int *slow) {
+  constexpr int NG = 64 / INS_LANES;
+  __shared__ int sm[NG * INS_GROUP_INTS];
+  const int grp = threadIdx.x / INS_LANES, gl = threadIdx.x % INS_LANES;
+  int *L = sm + grp * INS_GROUP_INTS;
+  int *S = L + INS_K + INS_LANES;  // the cavity in slot order
+  int *h = S + INS_K;
+  int *eu = h + INS_HASH, *ev = eu + INS_K + 2, *eo = ev + INS_K + 2, *es = eo + INS_K + 2,
+      *eord = es + INS_K + 2;
+  int *sc = eord + INS_K + 2;
+  const int nc = cnt[D_NC];
+  for (int base = blockIdx.x * NG; base < nc; base += gridDim.x * NG) {
+    const int k = base + grp;
+    const bool act = k < nc;
+    int st = CS_NONE, seed = -1;
+    double2 p = make_double2(0.0, 0.0);
+    if (act) {
+      const int c = C[k];
+      p = m.P[c];
+      seed = ptri[c];
+      if (!tri_ok(m, seed)) {
+        flag(m, E_INDEX);
+      } else {
+        const int c0 = conflict<true>(m, seed, p, nullptr);
+        if (c0 == PRED_UNSURE) st = CS_DEFER;
+        else if (c0 == 1) st = CS_VALID;
+        else flag(m, E_TOPOLOGY);  // the stored triangle must contain (or see) the point
+      }
+    }
+    for (int q = gl; q < INS_HASH; q += INS_LANES) h[q] = -1;
+    if (gl < 4) sc[gl] = 0;
+    __syncthreads();
+    const bool grow = st == CS_VALID;
+    if (grow && gl == 0) {
+      L[0] = seed;
+      ins_add(h, seed);
+      sc[IS_N] = 1;
+    }
+    __syncthreads();
+    int fb = 0;
+    for (;;) {
+      const int fe = sc[IS_N];
+      const bool more = grow && !(sc[IS_DEFER] | sc[IS_BAD]) && fb < fe;
+      __syncthreads();
+      if (__ballot(more) == 0ull) break;  // wave-uniform exit
+      if (more)
+        for (int it = gl; it < 3 * (fe - fb); it += INS_LANES) {
+          const int nb = reinterpret_cast<const int *>(&m.N[L[fb + it / 3]])[it % 3];
+          if (nb < 0) continue;
+          const int u = nb >> 2;
+          if (!tri_ok(m, u)) {
+            flag(m, E_INDEX);
+            sc[IS_BAD] = 1;
+            continue;
+          }
+          if (ins_has(h, u)) continue;
+          const int cf = conflict<true>(m, u, p, nullptr);
+          if (cf == PRED_UNSURE) {
+            sc[IS_DEFER] = 1;
+          } else if (cf == 1) {
+            // fewer than INS_K + INS_LANES inserts: a full cavity stops them
+            if (sc[IS_N] >= INS_K) {
+              if (!ins_has(h, u)) sc[IS_DEFER] = 1;
+            } else if (ins_add(h, u)) {
+              L[atomicAdd(&sc[IS_N], 1)] = u;
+            }
+          }
+        }
+      __syncthreads();
+      if (more) fb = fe;
+    }
+    const int n = sc[IS_N];
+    if (grow) {
+      if (sc[IS_BAD]) st = CS_NONE;
+      else if (sc[IS_DEFER] || n > INS_K) st = CS_DEFER;
+    }
+    const bool ok = grow && st == CS_VALID;
+    if (ok)
+      for (int e = gl; e < n; e += INS_LANES) {
+        const int v = L[e];
+        int rank = 0;
+        for (int x = 0; x < n; x++) rank += L[x] < v;
+        S[rank] = v;
+      }
+    __syncthreads();
+    if (ok)
+      for (int it = gl; it < 3 * n; it += INS_LANES) {
+        const int t = S[it / 3], j = it % 3;
+        const int nb = reinterpret_cast<const int *>(&m.N[t])[j];
+        if (nb >= 0 && ins_has(h, nb >> 2)) continue;
+        const int b = atomicAdd(&sc[IS_NB], 1);
+        if (b < INS_K + 2) {
+          const int4 v = m.V[t];
+          eu[b] = comp4(v, (j + 1) % 3);
+          ev[b] = comp4(v, (j + 2) % 3);
+          eo[b] = nb;
+        }
+      }
+    __syncthreads();
+    const int nb = n + 2;
+    const bool disk = ok && sc[IS_NB] == nb;  // a Delaunay cavity is a disk
+    if (disk)
+      for (int e = gl; e < nb; e += INS_LANES) {
+        const int v = ev[e];
+        int f = 0;
+        while (f < nb && eu[f] != v) f++;
+        if (f == nb) sc[IS_BAD] = 1;
+        es[e] = f < nb ? f : 0;
+      }
+    __syncthreads();
+    if (disk && gl == 0) {
+      int start = 0;
+      for (int e = 1; e < nb; e++)
+        if (eu[e] < eu[start]) start = e;
+      int e = start;
+      for (int q = 0; q < nb; q++) {
+        eord[q] = e;
+        e = es[e];
+      }
+      if (e != start) sc[IS_BAD] = 1;
+    }
+    __syncthreads();
+    if (ok && (!disk || sc[IS_BAD])) {
+      flag(m, E_TOPOLOGY);
+      st = CS_NONE;
+    }
+    if (ok && st == CS_VALID) {
+      int *Wk = W + (size_t)k * WS_INS;
+      int *Bu = Wk + KCAV, *Bv = Bu + (KCAV + 2), *Bo = Bv + (KCAV + 2);
+      for (int q = gl; q < n; q += INS_LANES) Wk[q] = S[q];
+      for (int q = gl; q < nb; q += INS_LANES) {
+        const int e = eord[q];
+        Bu[q] = eu[e];
+        Bv[q] = ev[e];
+        Bo[q] = eo[e];
+      }
+    }
+    if (act && gl == 0) {
+      cstat[k] = st;
+      cn[k] = st == CS_VALID ? n : 0;
+      if (st == CS_DEFER) slow[atomicAdd(&cnt[D_NSLOW], 1)] = k;
+    }
+    __syncthreads();  // LDS is reused by the next candidates
   }
 }
 
 // the deferred candidates with the exact stage (GCDT_INCIRCLE_WS doubles of
 // arena per lane of a grid of at most EXACT_GRID blocks of 64)
-__global__ void k_ins_cavity_slow(MeshG m, const int *C, const int *ptri, int *W, int *cstat,
-                                  int *cn, const int *slow, const int *nslow, double *arena) {
+__global__ void k_ins_cavity_slow(MeshG m, const int *C, const int *cnt, const int *ptri, int *W,
+                                  int *cstat, int *cn, const int *slow, double *arena) {
   const int lane = blockIdx.x * blockDim.x + threadIdx.x;
   double *ws = arena + (size_t)lane * GCDT_INCIRCLE_WS;
-  const int ns = *nslow;
+  const int ns = cnt[D_NSLOW];
   for (int q = lane; q < ns; q += gridDim.x * blockDim.x) {
     const int k = slow[q];
     const int c = C[k];
     int st = CS_NONE, n = 0;
-    cavity_one<false>(m, c, ptri[c], W + (size_t)k * WS_INS, &st, &n, ws);
+    cavity_one(m, c, ptri[c], W + (size_t)k * WS_INS, &st, &n, ws);
     cstat[k] = st;
     cn[k] = n;
   }
@@ -429,52 +717,79 @@ __device__ inline unsigned long long claim_key(unsigned long long ep, int k) {
 // index is best.  Several iterations per round: a winner stamps its region
 // with the round's sticky epoch; a loser whose region meets a stamp drops
 // out, the others claim again.
-__global__ void k_ins_claim(MeshG m, int nc, const int *W, const int *cstat, const int *cn,
-                            int *active, int iter, unsigned long long ep,
-                            unsigned long long sticky) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += gridDim.x * blockDim.x) {
+// An entry of a candidate's cavity or ring per lane of a group of INS_LANES,
+// so its loads and atomics are in flight together.
+__device__ __forceinline__ bool group_any(bool x) {
+  const int base = (threadIdx.x & 63) & ~(INS_LANES - 1);
+  return ((__ballot(x) >> base) & ((1ull << INS_LANES) - 1ull)) != 0ull;
+}
+__global__ __launch_bounds__(BLK) void k_ins_claim(MeshG m, const int *cnt, const int *W,
+                                                   const int *cstat, const int *cn, int *active,
+                                                   int iter, unsigned long long ep,
+                                                   unsigned long long sticky) {
+  const int gl = threadIdx.x % INS_LANES, per = blockDim.x / INS_LANES, nc = cnt[D_NC];
+  for (int k = blockIdx.x * per + threadIdx.x / INS_LANES; k < nc; k += gridDim.x * per) {
     const int *L = W + (size_t)k * WS_INS;
     const int *Bo = L + KCAV + 2 * (KCAV + 2);
     const int n = cn[k];
+    bool on;
     if (iter == 0) {
-      active[k] = cstat[k] == CS_VALID;
-    } else if (active[k]) {
-      bool hit = false;
-      for (int q = 0; q < n && !hit; q++)
-        hit = (m.claim[2 * (size_t)L[q]] >> 32) == sticky ||
-              (m.claim[2 * (size_t)L[q] + 1] >> 32) == sticky;
-      for (int q = 0; q < n + 2 && !hit; q++)
-        if (Bo[q] >= 0) hit = (m.claim[2 * (size_t)(Bo[q] >> 2)] >> 32) == sticky;
-      if (hit) active[k] = 0;
+      on = cstat[k] == CS_VALID;
+      if (gl == 0) active[k] = on;
+    } else {
+      on = active[k] != 0;
+      if (on) {
+        bool hit = false;
+        for (int q = gl; q < n; q += INS_LANES)
+          hit |= (m.claim[2 * (size_t)L[q]] >> 32) == sticky ||
+                 (m.claim[2 * (size_t)L[q] + 1] >> 32) == sticky;
+        for (int q = gl; q < n + 2; q += INS_LANES)
+          if (Bo[q] >= 0) hit |= (m.claim[2 * (size_t)(Bo[q] >> 2)] >> 32) == sticky;
+        if (group_any(hit)) {
+          on = false;
+          if (gl == 0) active[k] = 0;
+        }
+      }
     }
-    if (!active[k]) continue;
+    if (!on) continue;
     const unsigned long long key = claim_key(ep, k);
-    for (int q = 0; q < n; q++) atomicMax(&m.claim[2 * (size_t)L[q]], key);
-    for (int q = 0; q < n + 2; q++)
+    for (int q = gl; q < n; q += INS_LANES) atomicMax(&m.claim[2 * (size_t)L[q]], key);
+    for (int q = gl; q < n + 2; q += INS_LANES)
       if (Bo[q] >= 0) atomicMax(&m.claim[2 * (size_t)(Bo[q] >> 2) + 1], key);
   }
 }
 
-__global__ void k_ins_win(MeshG m, int nc, const int *W, const int *cn, int *active, int iter,
-                          unsigned long long ep, unsigned long long sticky, int *win) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += gridDim.x * blockDim.x) {
-    if (iter == 0) win[k] = 0;
-    if (!active[k]) continue;
+__global__ __launch_bounds__(BLK) void k_ins_win(MeshG m, const int *cnt, const int *W,
+                                                 const int *cn, int *active, int iter,
+                                                 unsigned long long ep, unsigned long long sticky,
+                                                 int *win) {
+  const int gl = threadIdx.x % INS_LANES, per = blockDim.x / INS_LANES, nc = cnt[D_NC];
+  for (int k = blockIdx.x * per + threadIdx.x / INS_LANES; k < nc; k += gridDim.x * per) {
+    const bool on = active[k] != 0;
+    if (!on) {
+      if (iter == 0 && gl == 0) win[k] = 0;
+      continue;
+    }
     const int *L = W + (size_t)k * WS_INS;
     const int *Bo = L + KCAV + 2 * (KCAV + 2);
     const int n = cn[k];
     const unsigned long long key = claim_key(ep, k);
-    bool w = true;
-    for (int q = 0; q < n && w; q++)
-      w = m.claim[2 * (size_t)L[q]] == key && m.claim[2 * (size_t)L[q] + 1] <= key;
-    for (int q = 0; q < n + 2 && w; q++)
-      if (Bo[q] >= 0) w = m.claim[2 * (size_t)(Bo[q] >> 2)] <= key;
-    if (!w) continue;
-    win[k] = 1;
-    active[k] = 0;
+    bool lose = false;
+    for (int q = gl; q < n; q += INS_LANES)
+      lose |= m.claim[2 * (size_t)L[q]] != key || m.claim[2 * (size_t)L[q] + 1] > key;
+    for (int q = gl; q < n + 2; q += INS_LANES)
+      if (Bo[q] >= 0) lose |= m.claim[2 * (size_t)(Bo[q] >> 2)] > key;
+    if (group_any(lose)) {
+      if (iter == 0 && gl == 0) win[k] = 0;
+      continue;
+    }
+    if (gl == 0) {
+      win[k] = 1;
+      active[k] = 0;
+    }
     const unsigned long long stamp = (sticky << 32) | 0xffffffffull;
-    for (int q = 0; q < n; q++) m.claim[2 * (size_t)L[q]] = stamp;
-    for (int q = 0; q < n + 2; q++)
+    for (int q = gl; q < n; q += INS_LANES) m.claim[2 * (size_t)L[q]] = stamp;
+    for (int q = gl; q < n + 2; q += INS_LANES)
       if (Bo[q] >= 0) m.claim[2 * (size_t)(Bo[q] >> 2) + 1] = stamp;
   }
 }
@@ -482,43 +797,44 @@ __global__ void k_ins_win(MeshG m, int nc, const int *W, const int *cn, int *act
 // Star insertion of a winner: star triangle q = (p, u_q, v_q) takes cavity
 // slot L[q] (q < n) or new slot tbase + 2 rank + (q - n); the outer
 // neighbours' links are repaired; the star's slots are stamped so that the
-// points they held are relocated.
-__global__ void k_ins_apply(MeshG m, const int *C, int nc, const int *W, const int *cn,
-                            const int *win, const int *rank, int tbase, int *ptri,
-                            unsigned long long *dirty, unsigned long long ep) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nc; k += gridDim.x * blockDim.x) {
+// points they held are relocated.  A star triangle per lane.
+constexpr int STAR_LANES = 8;
+__global__ __launch_bounds__(BLK) void k_ins_apply(MeshG m, const int *C, const int *cnt,
+                                                   const int *W, const int *cn, const int *win,
+                                                   const int *rank, int *ptri,
+                                                   unsigned long long *dirty,
+                                                   unsigned long long ep) {
+  const int gl = threadIdx.x % STAR_LANES, per = blockDim.x / STAR_LANES, nc = cnt[D_NC];
+  for (int k = blockIdx.x * per + threadIdx.x / STAR_LANES; k < nc; k += gridDim.x * per) {
     if (!win[k]) continue;
     const int c = C[k];
     const int *L = W + (size_t)k * WS_INS;
     const int *Bu = L + KCAV, *Bv = Bu + (KCAV + 2), *Bo = Bv + (KCAV + 2);
     const int n = cn[k], ns = n + 2;
-    const int tb = tbase + 2 * rank[k];
+    const int tb = cnt[D_TBASE] + 2 * rank[k];
     if (tb < 0 || tb + 1 >= m.cap) {
       flag(m, E_INDEX);
       continue;
     }
-    for (int q = 0; q < ns; q++) {
+    for (int q = gl; q < ns; q += STAR_LANES) {
       const int st = q < n ? L[q] : tb + (q - n);
       const int qn = q + 1 < ns ? q + 1 : 0, qp = q > 0 ? q - 1 : ns - 1;
       const int sn = qn < n ? L[qn] : tb + (qn - n), sp = qp < n ? L[qp] : tb + (qp - n);
-      m.V[st] = make_int4(c, Bu[q], Bv[q], 0);
-      m.N[st] = make_int4(Bo[q], (sn << 2) | 2, (sp << 2) | 1, 0);
-      dirty[st] = ep;
       const int o = Bo[q];
-      if (o >= 0) {
-        const int r = o >> 2, j = o & 3;
-        int *slot = reinterpret_cast<int *>(&m.N[r]) + j;
-        *slot = (st << 2) | 0;
-      }
+      m.V[st] = make_int4(c, Bu[q], Bv[q], 0);
+      m.N[st] = make_int4(o, (sn << 2) | 2, (sp << 2) | 1, 0);
+      dirty[st] = ep;
+      if (o >= 0) reinterpret_cast<int *>(&m.N[o >> 2])[o & 3] = (st << 2) | 0;
     }
-    ptri[c] = -1;
+    if (gl == 0) ptri[c] = -1;
   }
 }
 
 // Points whose triangle was rewritten this round walk from that slot (now a
 // triangle of the star that replaced it) to their new triangle.
-__global__ void k_relocate(MeshG m, const int *U, int nu, int *ptri,
+__global__ void k_relocate(MeshG m, const int *U, const int *cnt, int par, int *ptri,
                            const unsigned long long *dirty, unsigned long long ep) {
+  const int nu = cnt[D_NU + par];
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nu; k += gridDim.x * blockDim.x) {
     const int i = U[k];
     const int t = ptri[i];
@@ -537,11 +853,6 @@ __global__ void k_relocate(MeshG m, const int *U, int nu, int *ptri,
     }
     ptri[i] = t2 < 0 ? -2 : t2;
   }
-}
-
-__global__ void k_still_out(const int *U, int nu, const int *ptri, int *flag_out) {
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nu; k += gridDim.x * blockDim.x)
-    flag_out[k] = ptri[U[k]] >= 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1170,7 +1481,7 @@ struct Builder {
   }
   Builder() {
     CC(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-    CC(hipHostMalloc((void **)&h_total, 4 * sizeof(int), hipHostMallocDefault));
+    CC(hipHostMalloc((void **)&h_total, (D_N + 1) * sizeof(int), hipHostMallocDefault));
     d_err = alloc<unsigned>(1);
     scan_total = alloc<int>(1);
   }
@@ -1209,6 +1520,8 @@ struct Builder {
     if (e & E_CAVITY) msg += " region capacity exceeded;";
     if (e & E_TOPOLOGY) msg += " inconsistent triangulation;";
     if (e & E_DUPLICATE) msg += " duplicate input points;";
+    if (e & E_STALL) msg += " no progress (cavity capacity);";
+    if (e & E_SLOTS) msg += " triangle slots exhausted;";
     throw std::runtime_error(msg);
   }
 };
@@ -1399,6 +1712,7 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
   unsigned long long *dirty = B.alloc<unsigned long long>(cap);
   unsigned long long *pick = B.alloc<unsigned long long>(cap);
   int *flags = B.alloc<int>(std::max(np, cap));
+  int *cnt = B.alloc<int>(D_N);
   CC(hipMemcpyAsync(ptri, hptri.data(), sizeof(int) * np, hipMemcpyHostToDevice, B.st));
   if (nu) CC(hipMemcpyAsync(U, hU.data(), sizeof(int) * nu, hipMemcpyHostToDevice, B.st));
   CC(hipMemsetAsync(dirty, 0, sizeof(unsigned long long) * cap, B.st));
@@ -1408,71 +1722,80 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
     std::vector<unsigned long long> d0((size_t)t_init, ep);
     CC(hipMemcpyAsync(dirty, d0.data(), sizeof(unsigned long long) * t_init, hipMemcpyHostToDevice,
                       B.st));
-    k_relocate<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, nu, ptri, dirty, ep);
+    const int c0[D_N] = {nu, 0, 0, 0, t_init, 0, 0, 0};
+    CC(hipMemcpyAsync(cnt, c0, sizeof(c0), hipMemcpyHostToDevice, B.st));
+    k_relocate<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, cnt, 0, ptri, dirty, ep);
     CC(hipGetLastError());
     CC(hipStreamSynchronize(B.st));
   }
   B.check_err("initial location");
   // ---- phase 1: rounds of insertion ----
-  const int CMAX = 1 << 19;
-  int *C = B.alloc<int>(np);  // every flagged point is compacted into it
-  int *cstat = B.alloc<int>(std::min(np, CMAX) + 1);
-  int *cn = B.alloc<int>(std::min(np, CMAX) + 1);
-  int *slow = B.alloc<int>(std::min(np, CMAX) + 1);
-  int *nslow = B.alloc<int>(1);
-  int *win = B.alloc<int>(std::min(np, CMAX) + 1);
-  int *active = B.alloc<int>(std::min(np, CMAX) + 1);
-  const int ITERS = 4;
-  int *rank = B.alloc<int>(std::min(np, CMAX) + 1);
+  // A round is a chain of launches whose counts stay on the device; the host
+  // reads them back every ROUNDS_PER_SYNC rounds (rounds behind the last
+  // point do nothing).
+  constexpr int CMAX = 1 << 19, ITERS = 4, ROUNDS_PER_SYNC = 4;
+  const int ccap = std::min(np, CMAX);
+  int *C = B.alloc<int>(np);  // every picked point is compacted into it
+  int *cstat = B.alloc<int>((size_t)ccap);
+  int *cn = B.alloc<int>((size_t)ccap);
+  int *slow = B.alloc<int>((size_t)ccap);
+  int *win = B.alloc<int>((size_t)ccap);
+  int *active = B.alloc<int>((size_t)ccap);
+  int *rank = B.alloc<int>((size_t)ccap);
+  int *tiles = B.alloc<int>((size_t)(np / CMP_TILE + 1));
+  int *W = B.alloc<int>((size_t)ccap * WS_INS);
   double *arena = B.alloc<double>((size_t)EXACT_GRID * 64 * GCDT_INCIRCLE_WS);
-  int *W = nullptr;
-  long long w_cap = 0;
-  int tbase = t_init;
+  auto compact = [&](auto pred, int bound, const int *n, int *out, int *rk, const int *src,
+                     auto fin) {
+    if (bound <= CMP_TILE) {
+      k_compact_one<<<1, CMP_THREADS, 0, B.st>>>(pred, n, out, rk, src, fin);
+    } else {
+      const int nt = (bound + CMP_TILE - 1) / CMP_TILE;
+      k_compact_count<<<nt, CMP_THREADS, 0, B.st>>>(pred, n, tiles);
+      k_compact_scatter<<<nt, CMP_THREADS, 0, B.st>>>(pred, n, tiles, out, rk, src, fin);
+    }
+  };
   unsigned long long cep = 0;  // claim epoch
-  int rounds = 0;
+  int rounds = 0, par = 0, tbase = t_init;
   while (nu > 0) {
-    if (++rounds > 100000) throw std::runtime_error("CDT insertion did not finish");
-    ep++;
-    k_pick<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, nu, ptri, pick, ep);
-    k_cand_flags<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, nu, ptri, pick, ep, flags);
-    CC(hipGetLastError());
-    int nc = B.compact(flags, nu, U, C, nullptr);
-    nc = std::min(nc, CMAX);
-    if (nc == 0) {
-      B.check_err("candidate selection");
-      throw std::runtime_error("CDT insertion: no candidate");
+    const int cb = std::min(nu, CMAX);  // at most this many candidates
+    for (int r = 0; r < ROUNDS_PER_SYNC; r++, par ^= 1) {
+      ep++;
+      const int *dnu = cnt + D_NU + par;
+      k_pick<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, cnt, par, ptri, pick, ep);
+      compact(PredCand{m, U, ptri, pick, ep}, nu, dnu, C, nullptr, U,
+              FinCand{cnt, m.err, par, CMAX});
+      k_ins_cavity_fast<<<Builder::grid(cb, 64 / INS_LANES), 64, 0, B.st>>>(m, C, cnt, ptri, W,
+                                                                            cstat, cn, slow);
+      k_ins_cavity_slow<<<std::min(EXACT_GRID, Builder::grid(cb, 64)), 64, 0, B.st>>>(
+          m, C, cnt, ptri, W, cstat, cn, slow, arena);
+      // claim iterations; the round's sticky epoch is above all its claims
+      const unsigned long long sticky = cep + ITERS + 1;
+      const int gc = std::min(Builder::grid(cb, BLK / INS_LANES), 4096);
+      for (int it = 0; it < ITERS; it++) {
+        cep++;
+        k_ins_claim<<<gc, BLK, 0, B.st>>>(m, cnt, W, cstat, cn, active, it, cep, sticky);
+        k_ins_win<<<gc, BLK, 0, B.st>>>(m, cnt, W, cn, active, it, cep, sticky, win);
+      }
+      cep = sticky;
+      compact(PredIns{win}, cb, cnt + D_NC, nullptr, rank, nullptr, FinIns{cnt, m.err, cap});
+      k_ins_apply<<<Builder::grid(cb, BLK / STAR_LANES), BLK, 0, B.st>>>(m, C, cnt, W, cn, win,
+                                                                         rank, ptri, dirty, ep);
+      k_relocate<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, cnt, par, ptri, dirty, ep);
+      compact(PredOut{U, ptri}, nu, dnu, U2, nullptr, U, FinOut{cnt, par});
+      std::swap(U, U2);
     }
-    if ((long long)nc * WS_INS > w_cap) {
-      w_cap = std::max<long long>((long long)nc * WS_INS, 2 * w_cap);
-      W = B.alloc<int>((size_t)w_cap);
-    }
-    CC(hipMemsetAsync(nslow, 0, sizeof(int), B.st));
-    k_ins_cavity_fast<<<Builder::grid(nc, 64), 64, 0, B.st>>>(m, C, nc, ptri, W, cstat, cn, slow,
-                                                              nslow);
-    k_ins_cavity_slow<<<EXACT_GRID, 64, 0, B.st>>>(m, C, ptri, W, cstat, cn, slow, nslow, arena);
-    // claim iterations; the round's sticky epoch is above all its claims
-    const unsigned long long sticky = cep + ITERS + 1;
-    for (int it = 0; it < ITERS; it++) {
-      cep++;
-      k_ins_claim<<<Builder::grid(nc), BLK, 0, B.st>>>(m, nc, W, cstat, cn, active, it, cep,
-                                                        sticky);
-      k_ins_win<<<Builder::grid(nc), BLK, 0, B.st>>>(m, nc, W, cn, active, it, cep, sticky, win);
-    }
-    cep = sticky;
     CC(hipGetLastError());
-    const int nw = B.compact(win, nc, nullptr, nullptr, rank);
-    B.check_err("insertion cavities");
-    if (nw == 0) throw std::runtime_error("CDT insertion made no progress (cavity capacity)");
-    if (tbase + 2LL * nw > cap) throw std::runtime_error("CDT triangle slots exhausted");
-    k_ins_apply<<<Builder::grid(nc), BLK, 0, B.st>>>(m, C, nc, W, cn, win, rank, tbase, ptri,
-                                                      dirty, ep);
-    tbase += 2 * nw;
-    k_relocate<<<Builder::grid(nu), BLK, 0, B.st>>>(m, U, nu, ptri, dirty, ep);
-    k_still_out<<<Builder::grid(nu), BLK, 0, B.st>>>(U, nu, ptri, flags);
-    CC(hipGetLastError());
-    nu = B.compact(flags, nu, U, U2, nullptr);
-    std::swap(U, U2);
-    B.check_err("insertion");
+    int hc[D_N];
+    CC(hipMemcpyAsync(B.h_total, cnt, sizeof(hc), hipMemcpyDeviceToHost, B.st));
+    CC(hipMemcpyAsync(B.h_total + D_N, m.err, sizeof(unsigned), hipMemcpyDeviceToHost, B.st));
+    CC(hipStreamSynchronize(B.st));
+    memcpy(hc, B.h_total, sizeof(hc));
+    if (B.h_total[D_N]) B.check_err("insertion");
+    nu = hc[D_NU + par];
+    rounds = hc[D_ROUNDS];
+    tbase = hc[D_TBASE];
+    if (rounds > 100000) throw std::runtime_error("CDT insertion did not finish");
   }
   if (tbase != cap) throw std::runtime_error("CDT insertion left unused slots (duplicate points?)");
   // ---- phase 2: constraint recovery ----
