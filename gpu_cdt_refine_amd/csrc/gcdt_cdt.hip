@@ -76,12 +76,24 @@ constexpr int WS_INS = 4 * KCAV + 8;  // per-candidate ints: cavity | boundary u
 constexpr int EXACT_GRID = 512;   // blocks of 64 of the exact-stage kernels
 constexpr long long WALK_CAP = 1LL << 16;
 
+// One 128-byte line per triangle: a walk step and a conflict test need the
+// vertices, their coordinates and (for the next step) the neighbours together
+// and visit triangles at random, so a line replaces five gathers in a chain
+// of two (relocation of the uninserted points at 500,000 points: 14.4 ms a
+// build with separate arrays, bound by those gathers).
+struct __align__(128) CdtTri {
+  int4 V;        // vertices (w unused)
+  int4 N;        // neighbour otri (t << 2 | edge in the neighbour), -1 none
+  double2 X[3];  // the vertices' coordinates (the ghost vertex's are unused)
+  int4 pad[3];
+};
+static_assert(sizeof(CdtTri) == 128, "one L2 line per triangle");
+
 struct MeshG {
   const double2 *P;
-  int np;   // input points; the ghost vertex is np
-  int4 *V;  // triangle vertices (w unused)
-  int4 *N;  // neighbour otri (t << 2 | edge in the neighbour), -1 none
-  int cap;  // triangle slots (2 np - 2)
+  int np;     // input points; the ghost vertex is np
+  CdtTri *T;
+  int cap;    // triangle slots (2 np - 2)
   unsigned long long *claim;
   unsigned *err;
 };
@@ -98,15 +110,8 @@ __device__ inline void flag(const MeshG &m, unsigned e) { atomicOr(m.err, e); }
 __device__ inline bool tri_ok(const MeshG &m, int t) { return t >= 0 && t < m.cap; }
 __device__ inline bool vert_ok(const MeshG &m, int v) { return v >= 0 && v <= m.np; }
 
-// Orientation of (a, b, p) with a, b real vertices.
-__device__ inline int orient_v(const MeshG &m, int a, int b, double2 p) {
-  const double2 A = m.P[a], B = m.P[b];
-  return orient2d_sign(A.x, A.y, B.x, B.y, p.x, p.y, false, nullptr);
-}
-
-// p strictly inside segment (a, b), p collinear with it
-__device__ inline bool strictly_between(const MeshG &m, int a, int b, double2 p) {
-  const double2 A = m.P[a], B = m.P[b];
+// p strictly inside segment (A, B), p collinear with it
+__device__ inline bool strictly_between(double2 A, double2 B, double2 p) {
   // the dot products of (p - a, b - a) and (p - b, a - b) are both positive;
   // p is on the line, so their signs are exact when both are far from 0 and
   // exactly decidable by comparing coordinates otherwise
@@ -118,19 +123,18 @@ __device__ inline bool strictly_between(const MeshG &m, int a, int b, double2 p)
 // the filters (FAST) -- with ws given, always decided.
 template <bool FAST>
 __device__ int conflict(const MeshG &m, int t, double2 p, double *ws) {
-  const int4 v = m.V[t];
-  int g = -1;
-  if (v.x == m.np) g = 0;
-  else if (v.y == m.np) g = 1;
-  else if (v.z == m.np) g = 2;
-  if (g >= 0) {  // ghost triangle (a, b, G): the open half-plane right of b -> a ...
-    const int a = comp4(v, (g + 1) % 3), b = comp4(v, (g + 2) % 3);
-    const int o = orient_v(m, a, b, p);
+  const CdtTri &r = m.T[t];
+  const int4 v = r.V;
+  const double2 A = r.X[0], B = r.X[1], C = r.X[2];
+  if (v.x == m.np || v.y == m.np || v.z == m.np) {
+    // ghost triangle (a, b, G): the open half-plane right of b -> a ...
+    const double2 E = v.x == m.np ? B : (v.y == m.np ? C : A);
+    const double2 F = v.x == m.np ? C : (v.y == m.np ? A : B);
+    const int o = orient2d_sign(E.x, E.y, F.x, F.y, p.x, p.y, false, nullptr);
     if (o > 0) return 1;  // p strictly outside the hull edge (b, a)
     if (o < 0) return 0;
-    return strictly_between(m, a, b, p) ? 1 : 0;
+    return strictly_between(E, F, p) ? 1 : 0;
   }
-  const double2 A = m.P[v.x], B = m.P[v.y], C = m.P[v.z];
   int s = incircle_filtered(A.x, A.y, B.x, B.y, C.x, C.y, p.x, p.y, false, nullptr);
   if (s == PRED_UNSURE) {
     s = incircle_dd_sign(A.x, A.y, B.x, B.y, C.x, C.y, p.x, p.y);
@@ -153,22 +157,19 @@ __device__ int locate(const MeshG &m, int t, double2 p, bool *on_vertex) {
       flag(m, E_INDEX);
       return -1;
     }
-    const int4 v = m.V[t];
-    const int4 n = m.N[t];
-    int g = -1;
-    if (v.x == m.np) g = 0;
-    else if (v.y == m.np) g = 1;
-    else if (v.z == m.np) g = 2;
+    const CdtTri &r = m.T[t];
+    const int4 v = r.V, n = r.N;
+    const double2 A = r.X[0], B = r.X[1], C = r.X[2];
+    if (!vert_ok(m, v.x) || !vert_ok(m, v.y) || !vert_ok(m, v.z)) {
+      flag(m, E_INDEX);
+      return -1;
+    }
+    const int g = v.x == m.np ? 0 : (v.y == m.np ? 1 : (v.z == m.np ? 2 : -1));
     if (g >= 0) {
-      const int a = comp4(v, (g + 1) % 3), b = comp4(v, (g + 2) % 3);
-      if (!vert_ok(m, a) || !vert_ok(m, b) || a == m.np || b == m.np) {
-        flag(m, E_INDEX);
-        return -1;
-      }
-      const int o = orient_v(m, a, b, p);
-      if (o > 0 || (o == 0 && strictly_between(m, a, b, p))) return t;
-      const double2 A = m.P[a], B = m.P[b];
-      if ((A.x == p.x && A.y == p.y) || (B.x == p.x && B.y == p.y)) {
+      const double2 E = g == 0 ? B : (g == 1 ? C : A), F = g == 0 ? C : (g == 1 ? A : B);
+      const int o = orient2d_sign(E.x, E.y, F.x, F.y, p.x, p.y, false, nullptr);
+      if (o > 0 || (o == 0 && strictly_between(E, F, p))) return t;
+      if ((E.x == p.x && E.y == p.y) || (F.x == p.x && F.y == p.y)) {
         *on_vertex = true;
         return t;
       }
@@ -180,11 +181,6 @@ __device__ int locate(const MeshG &m, int t, double2 p, bool *on_vertex) {
       t = nb >> 2;
       continue;
     }
-    if (!vert_ok(m, v.x) || !vert_ok(m, v.y) || !vert_ok(m, v.z)) {
-      flag(m, E_INDEX);
-      return -1;
-    }
-    const double2 A = m.P[v.x], B = m.P[v.y], C = m.P[v.z];
     const int o0 = orient2d_sign(B.x, B.y, C.x, C.y, p.x, p.y, false, nullptr);
     const int o1 = orient2d_sign(C.x, C.y, A.x, A.y, p.x, p.y, false, nullptr);
     const int o2 = orient2d_sign(A.x, A.y, B.x, B.y, p.x, p.y, false, nullptr);
@@ -228,15 +224,16 @@ __device__ inline unsigned hash16(unsigned i) {
 // Key (largest wins): round epoch | inverted float bits of the squared
 // distance | inverted index.
 __device__ inline unsigned long long pick_key(const MeshG &m, unsigned long long ep, int i, int t) {
-  const int4 v = m.V[t];
+  const CdtTri &r = m.T[t];
+  const int4 v = r.V;
   const double2 p = m.P[i];
   double cx = 0.0, cy = 0.0;
   int k = 0;
   for (int j = 0; j < 3; j++) {
     const int x = comp4(v, j);
     if (x >= 0 && x < m.np) {
-      cx += m.P[x].x;
-      cy += m.P[x].y;
+      cx += r.X[j].x;
+      cy += r.X[j].y;
       k++;
     }
   }
@@ -424,7 +421,7 @@ __device__ void cavity_one(const MeshG &m, int c, int seed, int *W, int *status,
   int n = 0;
   L[n++] = seed;
   for (int idx = 0; idx < n; idx++) {
-    const int4 nb4 = m.N[L[idx]];
+    const int4 nb4 = m.T[L[idx]].N;
     for (int j = 0; j < 3; j++) {
       const int nb = comp4(nb4, j);
       if (nb < 0) continue;
@@ -460,7 +457,7 @@ __device__ void cavity_one(const MeshG &m, int c, int seed, int *W, int *status,
   int tu[KCAV + 2], tv[KCAV + 2], to[KCAV + 2];
   for (int idx = 0; idx < n; idx++) {
     const int t = L[idx];
-    const int4 v = m.V[t], nn = m.N[t];
+    const int4 v = m.T[t].V, nn = m.T[t].N;
     for (int j = 0; j < 3; j++) {
       const int nb = comp4(nn, j);
       if (nb >= 0 && in_list(L, n, nb >> 2)) continue;
@@ -587,7 +584,7 @@ __global__ __launch_bounds__(64) void k_ins_cavity_fast(MeshG m, const int *C, i
       if (__ballot(more) == 0ull) break;  // wave-uniform exit
       if (more)
         for (int it = gl; it < 3 * (fe - fb); it += INS_LANES) {
-          const int nb = reinterpret_cast<const int *>(&m.N[L[fb + it / 3]])[it % 3];
+          const int nb = reinterpret_cast<const int *>(&m.T[L[fb + it / 3]].N)[it % 3];
           if (nb < 0) continue;
           const int u = nb >> 2;
           if (!tri_ok(m, u)) {
@@ -628,11 +625,11 @@ __global__ __launch_bounds__(64) void k_ins_cavity_fast(MeshG m, const int *C, i
     if (ok)
       for (int it = gl; it < 3 * n; it += INS_LANES) {
         const int t = S[it / 3], j = it % 3;
-        const int nb = reinterpret_cast<const int *>(&m.N[t])[j];
+        const int nb = reinterpret_cast<const int *>(&m.T[t].N)[j];
         if (nb >= 0 && ins_has(h, nb >> 2)) continue;
         const int b = atomicAdd(&sc[IS_NB], 1);
         if (b < INS_K + 2) {
-          const int4 v = m.V[t];
+          const int4 v = m.T[t].V;
           eu[b] = comp4(v, (j + 1) % 3);
           ev[b] = comp4(v, (j + 2) % 3);
           eo[b] = nb;
@@ -816,15 +813,23 @@ __global__ __launch_bounds__(BLK) void k_ins_apply(MeshG m, const int *C, const 
       flag(m, E_INDEX);
       continue;
     }
+    const double2 pc = m.P[c];
     for (int q = gl; q < ns; q += STAR_LANES) {
       const int st = q < n ? L[q] : tb + (q - n);
       const int qn = q + 1 < ns ? q + 1 : 0, qp = q > 0 ? q - 1 : ns - 1;
       const int sn = qn < n ? L[qn] : tb + (qn - n), sp = qp < n ? L[qp] : tb + (qp - n);
       const int o = Bo[q];
-      m.V[st] = make_int4(c, Bu[q], Bv[q], 0);
-      m.N[st] = make_int4(o, (sn << 2) | 2, (sp << 2) | 1, 0);
+      const int u = Bu[q], v = Bv[q];
+      CdtTri r;
+      r.V = make_int4(c, u, v, 0);
+      r.N = make_int4(o, (sn << 2) | 2, (sp << 2) | 1, 0);
+      r.X[0] = pc;
+      r.X[1] = u < m.np ? m.P[u] : make_double2(0.0, 0.0);
+      r.X[2] = v < m.np ? m.P[v] : make_double2(0.0, 0.0);
+      r.pad[0] = r.pad[1] = r.pad[2] = make_int4(0, 0, 0, 0);
+      m.T[st] = r;
       dirty[st] = ep;
-      if (o >= 0) reinterpret_cast<int *>(&m.N[o >> 2])[o & 3] = (st << 2) | 0;
+      if (o >= 0) reinterpret_cast<int *>(&m.T[o >> 2].N)[o & 3] = (st << 2) | 0;
     }
     if (gl == 0) ptri[c] = -1;
   }
@@ -930,7 +935,7 @@ constexpr int SLIT = -3;  // boundary entry whose far side is in the region
 // up to date where regions are retriangulated).
 __global__ void k_vtri(MeshG m, int nt, int *vtri) {
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += gridDim.x * blockDim.x) {
-    const int4 v = m.V[t];
+    const int4 v = m.T[t].V;
     for (int j = 0; j < 3; j++) {
       const int x = comp4(v, j);
       if (x >= 0 && x < m.np) atomicMin(&vtri[x], t);
@@ -983,7 +988,8 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
   int x = -1, y = -1, t0 = -1;
   int4 v0, n0;
   for (int guard = 0; guard < 65536; guard++) {
-    const int4 v = m.V[t], nn = m.N[t];
+    const CdtTri &r = m.T[t];
+    const int4 v = r.V, nn = r.N;
     const int ia = index_of(v, a);
     if (ia < 0) {
       flag(m, E_TOPOLOGY);
@@ -1002,7 +1008,7 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
         flag(m, E_INDEX);
         return o;
       }
-      const double2 X = m.P[xv], Y = m.P[yv];
+      const double2 X = r.X[(ia + 1) % 3], Y = r.X[(ia + 2) % 3];
       const int o1 = orient2d_sign(pa.x, pa.y, X.x, X.y, pb.x, pb.y, false, nullptr);
       const int o2 = orient2d_sign(pa.x, pa.y, Y.x, Y.y, pb.x, pb.y, false, nullptr);
       // a vertex on the ray a -> b: the segment is split there (it lies
@@ -1086,7 +1092,8 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
       return o;
     }
     const int u = nb >> 2, ju = nb & 3;  // in u, the crossed edge is opposite ju
-    const int4 vu = m.V[u], nu = m.N[u];
+    const CdtTri &ru = m.T[u];
+    const int4 vu = ru.V, nu = ru.N;
     const int z = comp4(vu, ju);
     if (z == m.np || !vert_ok(m, z)) {  // the segment cannot leave the hull
       flag(m, E_TOPOLOGY);
@@ -1107,7 +1114,7 @@ __device__ SegOut seg_scan(const MeshG &m, int a, int b, const int *vtri, int *W
       o.z = b;
       break;
     }
-    const double2 Z = m.P[z];
+    const double2 Z = ru.X[ju];
     const int oz = orient2d_sign(pa.x, pa.y, pb.x, pb.y, Z.x, Z.y, false, nullptr);
     if (oz == 0) {  // the segment passes through z: the region ends here
       if (!add_bnd(vu, nu, iL) || !add_bnd(vu, nu, iR)) return over;
@@ -1291,7 +1298,9 @@ __global__ __launch_bounds__(64) void k_seg_apply(MeshG m, int2 *seg, const int 
           const double2 Cb = xy(best);
           const int i = pos + lane;
           bool in_c = false, und = false;
-          if (i <= hi) {
+          // a chain names a vertex twice where its region has a slit: the
+          // sign is 0 (and no filter could tell)
+          if (i <= hi && id(i) != id(best) && id(i) != id(lo - 1) && id(i) != id(hi + 1)) {
             const double2 D = xy(i);
             int sg = incircle_filtered(X.x, X.y, Y.x, Y.y, Cb.x, Cb.y, D.x, D.y, false, nullptr);
             if (sg == PRED_UNSURE) {
@@ -1377,16 +1386,18 @@ __global__ __launch_bounds__(64) void k_seg_apply(MeshG m, int2 *seg, const int 
           if (Bu[e] == u && Bv[e] == v && Bo[e] != SLIT) {
             link = Bo[e];
             // the outer triangle's back-link
-            if (link >= 0) reinterpret_cast<int *>(&m.N[link >> 2])[link & 3] = (st << 2) | j;
+            if (link >= 0) reinterpret_cast<int *>(&m.T[link >> 2].N)[link & 3] = (st << 2) | j;
             break;
           }
       if (link == -2) {
         ok = false;
         continue;
       }
-      reinterpret_cast<int *>(&m.N[st])[j] = link;
-      reinterpret_cast<int *>(&m.V[st])[j] = NT[it3];
-      vtri[NT[it3]] = st;  // any triangle at the vertex serves the next pass's scans
+      const int w = NT[it3];
+      reinterpret_cast<int *>(&m.T[st].N)[j] = link;
+      reinterpret_cast<int *>(&m.T[st].V)[j] = w;
+      m.T[st].X[j] = m.P[w];
+      vtri[w] = st;  // any triangle at the vertex serves the next pass's scans
     }
     if (__ballot(!ok) != 0ull) {
       flag(m, E_TOPOLOGY);
@@ -1435,7 +1446,7 @@ __global__ void k_seg_pending_flags(const int *done, int ns, int *flag_out) {
 // ---------------------------------------------------------------------------
 __global__ void k_real_flags(MeshG m, int nt, int *flag_out) {
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += gridDim.x * blockDim.x) {
-    const int4 v = m.V[t];
+    const int4 v = m.T[t].V;
     flag_out[t] = v.x != m.np && v.y != m.np && v.z != m.np;
   }
 }
@@ -1444,7 +1455,7 @@ __global__ void k_export_cdt(MeshG m, int nt, const int *flag_in, const int *new
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nt; t += gridDim.x * blockDim.x) {
     if (!flag_in[t]) continue;
     const int o = newid[t];
-    const int4 v = m.V[t], n = m.N[t];
+    const int4 v = m.T[t].V, n = m.T[t].N;
     T[3 * o] = v.x;
     T[3 * o + 1] = v.y;
     T[3 * o + 2] = v.z;
@@ -1623,8 +1634,7 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
   m.P = dP;
   m.np = np;
   m.cap = cap;
-  m.V = B.alloc<int4>(cap);
-  m.N = B.alloc<int4>(cap);
+  m.T = B.alloc<CdtTri>(cap);
   m.claim = B.alloc<unsigned long long>(2 * (size_t)cap);
   m.err = B.d_err;
   CC(hipMemsetAsync(m.claim, 0, sizeof(unsigned long long) * 2 * cap, B.st));
@@ -1689,13 +1699,18 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
         if (it == edges.end() || it->first != rk) throw std::runtime_error("initial triangulation links");
         tn[3 * t + j] = it->second;
       }
-    std::vector<int4> hv(t_init), hn(t_init);
+    std::vector<CdtTri> ht(t_init);
     for (int t = 0; t < t_init; t++) {
-      hv[t] = make_int4(tv[3 * t], tv[3 * t + 1], tv[3 * t + 2], 0);
-      hn[t] = make_int4(tn[3 * t], tn[3 * t + 1], tn[3 * t + 2], 0);
+      CdtTri r{};
+      r.V = make_int4(tv[3 * t], tv[3 * t + 1], tv[3 * t + 2], 0);
+      r.N = make_int4(tn[3 * t], tn[3 * t + 1], tn[3 * t + 2], 0);
+      for (int j = 0; j < 3; j++) {
+        const int v = tv[3 * t + j];
+        if (v < np) r.X[j] = make_double2(points[2 * (size_t)v], points[2 * (size_t)v + 1]);
+      }
+      ht[t] = r;
     }
-    CC(hipMemcpyAsync(m.V, hv.data(), sizeof(int4) * t_init, hipMemcpyHostToDevice, B.st));
-    CC(hipMemcpyAsync(m.N, hn.data(), sizeof(int4) * t_init, hipMemcpyHostToDevice, B.st));
+    CC(hipMemcpyAsync(m.T, ht.data(), sizeof(CdtTri) * t_init, hipMemcpyHostToDevice, B.st));
     CC(hipStreamSynchronize(B.st));
   }
   // uninserted points, all located from triangle 0 first
