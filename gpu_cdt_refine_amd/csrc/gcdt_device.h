@@ -200,6 +200,39 @@ struct PassD {
   int lshift;
 };
 
+// State of the host loop that k_small_rounds carries from pass to pass, and
+// hands back.
+enum : int {
+  SR_BOUNDARY = 0,  // stopped at a pass boundary, before the segment check
+  SR_DONE,          // refinement ended, status set
+  SR_ROUNDS,        // max_rounds reached
+  SR_SLOW           // a pass waits for the exact cavity kernel
+};
+struct SmallState {
+  int np, nt, ns;
+  int epoch, pass_index, prev_win, round, np_round;
+  int ne;  // encroached subsegments listed (-1: list lost)
+  int nb;  // in: bad triangles listed (-1: unknown)
+  int status, grow;  // grow: a cavity overflowed, the capacity K doubles
+  int seg_passes, bad_passes, cand_evals, passes;
+  int code, stage, nc, nseg;  // SR_SLOW: stage 1 subsegment, 2 all filtered cavities done
+};
+struct SmallOut {
+  SmallState st;
+  unsigned long long acc[CNT_N];  // counters of the completed passes
+};
+struct SmallArgs {
+  SmallState st;
+  const int *enc, *bad;  // encroached subsegments, bad triangles (ascending)
+  int *enc_out, *ids_out, *dirty;
+  float *feat, *score;
+  const float *mlp;  // priority network (nullptr: none)
+  int lshift, mix_below, cap, cand_factor, cand_min, kmax, seg_iters, bad_iters, max_rounds;
+  int del_on;
+  long long capP, capT, capS;
+  SmallOut *out;  // mapped host memory
+};
+
 // Learned claim priority of a bad-triangle candidate: its shortest-edge
 // bucket coarsened by 2^shift half-octaves, then higher predicted conflict
 // first (the score quantised to 8 bits).

@@ -57,6 +57,7 @@ enum KernelId {
   K_MLP,
   K_DEL_SCAN,
   K_DEL_APPLY,
+  K_SMALL,
   K_NKERN
 };
 
@@ -139,7 +140,16 @@ class Refiner {
   void ensure_cb(int nb);
   void flush_counters();
   int run_pass(const int *ids, int nc, int nseg, long long *progress, bool *overflowed,
-               int *nwin_seg, bool list_enc = false);
+               int *nwin_seg, bool list_enc = false, int resume = 0);
+  void wrap_epoch(int iters);
+  void ensure_feat(int nc);
+  bool small_pass(int nc, int nseg) const;
+  bool run_small(const int *enc, int ne, const int *bad, int nb, int *round, int *prev_win,
+                 bool *done);
+  void after_seg_pass(bool of);
+  bool after_bad_pass(int ne, int nbc, int nwin, int nws, long long prog, bool of, int *prev_win,
+                      int *round);
+  void add_pass_stats(const unsigned long long *c);
   DelD del_base() const;
   void enqueue_deletion(const DelD &dd);
   void compact_points();
@@ -152,12 +162,12 @@ class Refiner {
   void loop_graph();
   void loop_host();
   void loop_mixed();
-  bool bad_pass(int ne, int *prev_win);
+  bool bad_pass(int ne, int *prev_win, int *round);
   void ensure_mix(long long n);
   void size_pass_buffers();
   unsigned long long *ctl_cnt_ptr() const;
   int cavity_lanes(int Kc) const;
-  void launch_cavity(bool is_seg, int grid, const PassD &ps);
+  void launch_cavity(bool is_seg, int grid, const PassD &ps, bool resumed = false);
   int select_by_priority(int *ids, int nb, int cap, int **out_ids);
   void ensure_capacity(long long needP, long long needT, long long needS);
   bool vm_setup();
@@ -209,6 +219,9 @@ class Refiner {
   int *sel_prio = nullptr, *sel_tmp = nullptr, *sel_list = nullptr;
   int sel_cap = 0;
   unsigned *d_hist = nullptr;
+  // runs of small passes: rewritten triangles, the kernel's answer (mapped)
+  int *sr_dirty = nullptr;
+  SmallOut *sr_out = nullptr, *d_sr_out = nullptr;
   float *c_feat = nullptr, *c_score = nullptr;
   int *c_deg = nullptr, *t_cnt = nullptr;
   long long t_cnt_cap = 0;

@@ -25,42 +25,9 @@
 #include <vector>
 
 #include "gpu_cdt_refine.h"
+#include "mlp_infer.h"
 
 namespace gcdt {
-
-constexpr int MLP_IN = 16, MLP_H = 64;
-constexpr int OFF_W1 = 0, OFF_B1 = OFF_W1 + MLP_IN * MLP_H, OFF_W2 = OFF_B1 + MLP_H,
-              OFF_B2 = OFF_W2 + MLP_H * MLP_H, OFF_W3 = OFF_B2 + MLP_H,
-              OFF_B3 = OFF_W3 + MLP_H, MLP_NPARAM = OFF_B3 + 1;
-
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ short f2bf(float f) {  // round to nearest even
-  unsigned u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (short)(u >> 16);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (short)(u >> 16);
-}
-__device__ __forceinline__ float bf2f(short h) {
-  return __uint_as_float(((unsigned)(unsigned short)h) << 16);
-}
-
-__device__ __forceinline__ floatx4 mfma(bf16x4 a, bf16x4 b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
-
-// gfx950's double-K BF16 MFMA (v_mfma_f32_16x16x32_bf16), used by the
-// inference kernel's 64-wide hidden layer: two instructions per 16x16 output
-// block instead of four.  Operand layout (checked by k_mfma_probe32 against a
-// host product): A[16][32]: lane l holds row l%16, k = 8*(l/16) + 0..7;
-// B[32][16]: lane l holds col l%16, k = 8*(l/16) + 0..7; D as for 16x16x16.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef short shortx8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ floatx4 mfma32(shortx8 a, shortx8 b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 
 // One wave computes the forward pass of 16 samples starting at row0.
 // Outputs D-layout activations (pre-ReLU kept implicitly by value > 0).
@@ -146,97 +113,23 @@ __global__ __launch_bounds__(64) void k_mlp_forward(const float *X, int n,
 // forward (inputs, weights and hidden activations in BF16, FP32 accumulate);
 // only layer 2's accumulation order differs.
 constexpr int INF_WAVES = 4;
-// LDS written by some lanes of a wave and read by others: release, the
-// wave's convergence point, acquire (wavefront scope).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-constexpr int W2T_STRIDE = MLP_H + 8;  // transposed W2 rows, padded against bank conflicts
-constexpr int H1_STRIDE = MLP_H + 8;
 __global__ __launch_bounds__(64 * INF_WAVES) void k_mlp_infer(const float *X, int n,
                                                               const float *P, float *y,
                                                               const int *dn, const int *dgo) {
-  __shared__ short w1[MLP_IN * MLP_H];                 // [k][c]
-  __shared__ __align__(16) short w2t[MLP_H * W2T_STRIDE];  // [c][k]
-  __shared__ float b1[MLP_H], b2[MLP_H], w3[MLP_H];
+  __shared__ MlpWeights w;
   __shared__ __align__(16) short h1[INF_WAVES][16 * H1_STRIDE];  // per wave: [row][k]
   if (dn) n = *dgo ? *dn : 0;
   if (n <= 0 || (int)blockIdx.x * INF_WAVES * 16 >= n) return;
-  // Small passes are bound by this staging, so every load of it is in flight
-  // at once: 16.2 -> 5.5 us a launch in a 41,003-point refinement, together
-  // with more blocks (infer_blocks).
-  constexpr int NT = 64 * INF_WAVES, N1 = MLP_IN * MLP_H / NT, N2 = MLP_H * MLP_H / NT;
-  {
-    float v1[N1], v2[N2], vb1 = 0.f, vb2 = 0.f, vw3 = 0.f;
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < N1; q++) v1[q] = P[OFF_W1 + q * NT + t];
-#pragma unroll
-    for (int q = 0; q < N2; q++) v2[q] = P[OFF_W2 + q * NT + t];
-    if (t < MLP_H) {
-      vb1 = P[OFF_B1 + t];
-      vb2 = P[OFF_B2 + t];
-      vw3 = P[OFF_W3 + t];
-    }
-#pragma unroll
-    for (int q = 0; q < N1; q++) w1[q * NT + t] = f2bf(v1[q]);
-#pragma unroll
-    for (int q = 0; q < N2; q++) {
-      const int k = (q * NT + t) / MLP_H, c = t % MLP_H;
-      w2t[c * W2T_STRIDE + k] = f2bf(v2[q]);
-    }
-    if (t < MLP_H) {
-      b1[t] = vb1;
-      b2[t] = vb2;
-      w3[t] = bf2f(f2bf(vw3));
-    }
-  }
+  // Small passes are bound by this staging: 16.2 -> 5.5 us a launch in a
+  // 41,003-point refinement with all of its loads in flight, together with
+  // more blocks (infer_blocks).
+  mlp_stage<64 * INF_WAVES>(P, w, (int)threadIdx.x);
   __syncthreads();
-  const float b3 = P[OFF_B3];
-  const int wv = threadIdx.x / 64, l = threadIdx.x & 63, r = l % 16, kb = l / 16;
-  short *H = h1[wv];
+  const int wv = threadIdx.x / 64;
   for (int row0 = (blockIdx.x * INF_WAVES + wv) * 16; row0 < n;
        row0 += gridDim.x * INF_WAVES * 16) {
-    // layer 1 (K = 16): A = X[row0 + r][4kb..4kb+3]
-    bf16x4 a;
-    const int row = row0 + r;
-    for (int j = 0; j < 4; j++)
-      a[j] = row < n ? f2bf(X[(size_t)row * MLP_IN + 4 * kb + j]) : (short)0;
-    for (int cb = 0; cb < 4; cb++) {
-      bf16x4 b;
-      for (int j = 0; j < 4; j++) b[j] = w1[(4 * kb + j) * MLP_H + cb * 16 + r];
-      floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      z = mfma(a, b, z);
-      const float bias = b1[cb * 16 + r];
-      // D layout: column cb*16 + r, rows 4kb + j
-      for (int j = 0; j < 4; j++) H[(4 * kb + j) * H1_STRIDE + cb * 16 + r] = f2bf(fmaxf(z[j] + bias, 0.f));
-    }
-    wave_sync();  // H written by the wave's lanes, read by others
-    // layer 2 (K = 64 = 2 x 32): A row r, k = kk*32 + 8kb + 0..7 (contiguous in H)
-    floatx4 h2[4];
-    for (int cb = 0; cb < 4; cb++) {
-      floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      for (int kk = 0; kk < 2; kk++) {
-        const shortx8 a2 = *reinterpret_cast<const shortx8 *>(&H[r * H1_STRIDE + kk * 32 + 8 * kb]);
-        const shortx8 b2v =
-            *reinterpret_cast<const shortx8 *>(&w2t[(cb * 16 + r) * W2T_STRIDE + kk * 32 + 8 * kb]);
-        z = mfma32(a2, b2v, z);
-      }
-      const float bias = b2[cb * 16 + r];
-      for (int j = 0; j < 4; j++) z[j] = fmaxf(z[j] + bias, 0.f);
-      h2[cb] = z;
-    }
-    // layer 3: y[row] = sum_c H2[row][c] W3[c] + b3 over the 16 lanes of a group
-    for (int j = 0; j < 4; j++) {
-      float s = 0.f;
-      for (int cb = 0; cb < 4; cb++) s += h2[cb][j] * w3[cb * 16 + r];
-      for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
-      const int ro = row0 + 4 * kb + j;
-      if (r == 0 && ro < n) y[ro] = s + b3;
-    }
-    wave_sync();  // H is rewritten by the next rows
+    mlp_rows16(X, n, row0, w, h1[wv], y);
+    wave_sync();  // the activations are rewritten by the next rows
   }
 }
 

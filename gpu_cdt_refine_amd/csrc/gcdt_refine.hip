@@ -30,6 +30,7 @@
 
 #include "gcdt_device.h"
 #include "gcdt_internal.h"
+#include "mlp_infer.h"
 
 namespace gcdt {
 
@@ -460,6 +461,16 @@ __device__ __forceinline__ bool mark_enc_local(const MeshD &m, int s) {
   return atomicCAS(&m.senc[s], 0, 1) == 0;
 }
 
+// What a pass's steps report as they change the mesh: the separate kernels
+// keep no lists (a scan finds the changes later); k_small_rounds does.
+struct NoTrace {
+  __device__ void encroached(int) const {}           // senc[s] went 0 -> 1
+  __device__ void rewritten(const MeshD &, int) const {}  // slot about to be rewritten
+  __device__ void seg_winners(const PassD &ps, unsigned n) const {
+    atomicAdd(&ps.cnt[CNT_SEGWIN], (unsigned long long)n);
+  }
+};
+
 __device__ __forceinline__ unsigned long long wave_sum(unsigned long long x) {
   for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
   return x;
@@ -472,7 +483,8 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long x) {
 // every wave (segment cavities of a 10^6-point refinement 59.6 us a launch
 // with the shuffles, 49.1 without).
 enum { CC_MARKS = 0, CC_GIVEUPS, CC_OVERFLOW, CC_REJ_ENC, CC_REJ_BLOCKED, CC_VALID,
-       CC_FP32, CC_FP64, CC_DD, CC_EXACT, CC_EXAM, CC_N };
+       CC_FP32, CC_FP64, CC_DD, CC_EXACT, CC_EXAM, CC_N,
+       CC_SLOW = CC_N, CC_ALL };  // CC_SLOW: deferred (counted by ps.cnt itself)
 __device__ __forceinline__ int cc_counter(int k, bool is_seg) {
   switch (k) {
     case CC_MARKS: return CNT_MARKS;
@@ -489,7 +501,7 @@ __device__ __forceinline__ int cc_counter(int k, bool is_seg) {
   }
 }
 struct CavCounts {
-  unsigned c[CC_N];
+  unsigned c[CC_ALL];
   // sums: CC_N ints of the wave's LDS, free by now
   __device__ void flush(unsigned long long *cnt, bool is_seg, unsigned *sums) {
     const int lane = threadIdx.x & 63;
@@ -589,17 +601,18 @@ constexpr int ST_SLOW = 6;   // deferred: an undecided sign, or a cavity beyond
 // the full cascade (double-double, then exact expansions in the per-lane
 // arena) and LDS for K triangles.  Neither the rare stages' registers nor the
 // largest cavities' LDS thus limit the occupancy of the hot kernel.
-template <bool IS_SEG, int LG, bool FAST>
-__device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
-                                            const PassD &ps, int Kmax) {
+// One wave of the evaluation, number wv of nwv, with sm its LDS.
+template <bool IS_SEG, int LG, bool FAST, class Trace>
+__device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, const PassD &ps,
+                                            int Kmax, int wv, int nwv, int *sm, CavCounts &cc,
+                                            const Trace &trace) {
   static_assert(LG >= 8 && 64 % LG == 0, "lane groups of 8..64 lanes");
   constexpr int NG = 64 / LG;
-  extern __shared__ int sm[];
   // K: the cavity capacity this kernel handles (LDS layout); ps.K: the
   // pass's capacity (workspace layout, overflow rule)
   const int K = FAST ? min(ps.K, ps.Kf) : ps.K;
   const int HC = cav_hash_cap(K, LG), HR = ring_hash_cap(K);
-  const int lane = threadIdx.x, grp = lane / LG, gl = lane % LG;
+  const int lane = threadIdx.x & 63, grp = lane / LG, gl = lane % LG;
   int *L = sm + grp * group_lds_ints(K, LG);
   int *hc = L + (2 * K + 2);
   int *hr = hc + HC;
@@ -607,11 +620,9 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
   int *eu = sc + 8, *ev = eu + (K + 2), *eo = ev + (K + 2), *es = eo + (K + 2);
   int *esucc = es + (K + 2), *eord = esucc + (K + 2);
   const bool fp32 = pr.use_fp32 != 0;
-  CavCounts cc;
-  for (int k = 0; k < CC_N; k++) cc.c[k] = 0u;
   // the exact stages' arena: only the exact kernel (whose grid the arena
   // covers) uses it
-  double *pws = FAST ? nullptr : ps.pws + ((size_t)blockIdx.x * 64 + lane) * GCDT_INCIRCLE_WS;
+  double *pws = FAST ? nullptr : ps.pws + ((size_t)wv * 64 + lane) * GCDT_INCIRCLE_WS;
   const int nc = pass_nc(ps);
   const int nseg = pass_nseg(ps);
   const int *ids = pass_ids(ps);
@@ -619,7 +630,6 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
   // [0, nseg), bad triangles [nseg, nc)), or the deferred ones of any kind
   const int lo = IS_SEG ? 0 : nseg;
   const int nwork = FAST ? (IS_SEG ? nseg : nc - nseg) : (nc > 0 ? (int)ps.cnt[CNT_SLOW] : 0);
-  if ((int)blockIdx.x * NG >= nwork) return;  // most passes defer nothing
   bool unsure = false;
   auto in_circle = [&](double2 a, double2 b, double2 c, double x, double y, PredStats *q) {
     if (!FAST) return incircle_sign(a.x, a.y, b.x, b.y, c.x, c.y, x, y, pws, fp32, q);
@@ -633,7 +643,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
     if (sg == PRED_UNSURE) { unsure = true; sg = 0; }
     return sg;
   };
-  for (int base = blockIdx.x * NG; base < nwork; base += gridDim.x * NG) {
+  for (int base = wv * NG; base < nwork; base += nwv * NG) {
     bool act = base + grp < nwork;
     int i = nc;
     if (act) {
@@ -703,7 +713,10 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
               status = ST_GIVEUP;
             } else {
               status = ST_REJ_BLOCKED;
-              if (gl == 0 && mark_enc_local(m, sg)) cc.c[CC_MARKS]++;
+              if (gl == 0 && mark_enc_local(m, sg)) {
+                cc.c[CC_MARKS]++;
+                trace.encroached(sg);
+              }
             }
           } else if (w == 2 || w == 4) {
             status = ST_GIVEUP;
@@ -715,7 +728,10 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
                 status = ST_GIVEUP;
               } else if (s >= 0) {
                 status = ST_REJ_BLOCKED;
-                if (gl == 0 && mark_enc_local(m, s)) cc.c[CC_MARKS]++;
+                if (gl == 0 && mark_enc_local(m, s)) {
+                  cc.c[CC_MARKS]++;
+                  trace.encroached(s);
+                }
               } else {
                 int nb = comp(m.T[tl].N, jl);
                 if (nb < 0) status = ST_GIVEUP;
@@ -732,7 +748,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
     for (int k = gl; k < HR; k += LG) hr[k] = -1;
     if (gl < 8) sc[gl] = 0;
     if (gl == 0) sc[SC_DSEG] = 0x7f7fffff;  // +FLT_MAX bits: no subsegment yet
-    __syncthreads();
+    wave_sync();
     if (grow && gl == 0) {
       L[0] = seed0;
       hset_insert(hc, HC, seed0);
@@ -744,13 +760,13 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
       }
       sc[SC_N] = c0;
     }
-    __syncthreads();
+    wave_sync();
     int fb = 0;
     for (;;) {
       int fe = sc[SC_N];
       int ovf = sc[SC_OVF] | sc[SC_SLOW];
       bool more = grow && !ovf && fb < fe;
-      __syncthreads();
+      wave_sync();
       if (__ballot(more) == 0ull) break;  // wave-uniform exit
       if (more) {
         int items = (fe - fb) * 3;
@@ -785,7 +801,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
           }
         }
       }
-      __syncthreads();
+      wave_sync();
       if (more) fb = fe;
     }
     int n = 0, r = 0;
@@ -805,10 +821,10 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
         for (int x = 0; x < n; x++) rank += L[x] < v;
         tmp[rank] = v;
       }
-    __syncthreads();
+    wave_sync();
     if (cav_ok)
       for (int e = gl; e < n; e += LG) L[e] = tmp[e];
-    __syncthreads();
+    wave_sync();
     // ---- disk and star checks over every cavity edge ----
     if (cav_ok)
       for (int it = gl; it < 3 * n; it += LG) {
@@ -875,7 +891,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
           }
         }
       }
-    __syncthreads();
+    wave_sync();
     if (cav_ok) {
       r = sc[SC_R];
       if (FAST && sc[SC_SLOW]) {
@@ -902,7 +918,10 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
           }
           if (enc) {
             live |= m.senc[s] != 2;
-            if (mark_enc_local(m, s)) cc.c[CC_MARKS]++;
+            if (mark_enc_local(m, s)) {
+              cc.c[CC_MARKS]++;
+              trace.encroached(s);
+            }
           }
         }
         // every lane of this group is here (the branch is group-uniform)
@@ -923,7 +942,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
         while (f < nbe && eu[f] != v) f++;
         esucc[e] = f < nbe ? f : 0;
       }
-    __syncthreads();
+    wave_sync();
     int nstar = 0;
     if (star) {
       int start = 0;
@@ -945,7 +964,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
         }
       }
     }
-    __syncthreads();
+    wave_sync();
     if (star) {
       int *G = ps.ws + (size_t)i * ps.R + (2 * ps.K + 2);
       for (int q = gl; q < nstar; q += LG) {
@@ -962,7 +981,10 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
       for (int q = gl; q < n + r; q += LG) G[q] = L[q];
     }
     if (status == ST_SLOW) {  // defer: no output, no side effect, no counts
-      if (gl == 0) ps.slow[atomicAdd(&ps.cnt[CNT_SLOW], 1ull)] = i;
+      if (gl == 0) {
+        ps.slow[atomicAdd(&ps.cnt[CNT_SLOW], 1ull)] = i;
+        cc.c[CC_SLOW]++;
+      }
     } else {
       cc.c[CC_FP32] += (unsigned)cst.fp32_hits;
       cc.c[CC_FP64] += (unsigned)cst.fp64_hits;
@@ -1016,8 +1038,22 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr,
         else m.tflag[t0] |= TF_GIVEUP;
       }
     }
-    __syncthreads();  // LDS is reused by the next candidates
+    wave_sync();  // LDS is reused by the next candidates
   }
+}
+
+// A kernel of one wave per block.
+template <bool IS_SEG, int LG, bool FAST>
+__device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr, const PassD &ps,
+                                            int Kmax) {
+  extern __shared__ int sm[];
+  if (!FAST) {  // most passes defer nothing
+    if (pass_nc(ps) <= 0 || ps.cnt[CNT_SLOW] == 0ull) return;
+  }
+  CavCounts cc;
+  for (int k = 0; k < CC_ALL; k++) cc.c[k] = 0u;
+  cavity_wave<IS_SEG, LG, FAST>(m, pr, ps, Kmax, (int)blockIdx.x, (int)gridDim.x, sm, cc,
+                                NoTrace{});
   cc.flush(ps.cnt, IS_SEG, (unsigned *)sm);
 }
 
@@ -1067,15 +1103,16 @@ __device__ __forceinline__ unsigned long long group_bits(unsigned long long b) {
 // region touches a winner's stamped region drops out (it is blocked, the
 // oracle's rule); the others claim again among themselves.  Stamps carry an
 // epoch above every claim of the pass, so concurrent claims never hide them.
+// Thread tid of nthr; ws_seg / ws_bad: workspace ints the cavities wrote.
 template <int G>
-__global__ __launch_bounds__(LIST_BLOCK) void k_claim(MeshD m, PassD ps, int *cact) {
+__device__ __forceinline__ void claim_body(const MeshD &m, const PassD &ps, int *cact, int tid,
+                                           int nthr, unsigned &ws_seg, unsigned &ws_bad) {
   const int nc = pass_nc(ps);
   const unsigned long long ep = pass_epoch(ps);
   const unsigned long long sticky = pass_sticky(ps);
-  const int gl = threadIdx.x % G, per = blockDim.x / G;
+  const int gl = tid % G, per = nthr / G;
   const int nseg = pass_nseg(ps);
-  unsigned ws_seg = 0, ws_bad = 0;  // workspace ints the cavity kernels wrote
-  for (int i = blockIdx.x * per + threadIdx.x / G; i < nc; i += gridDim.x * per) {
+  for (int i = tid / G; i < nc; i += per) {
     const int *L = ps.ws + (size_t)i * ps.R;
     int prio;
     if (ps.iter == 0) {
@@ -1120,6 +1157,13 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_claim(MeshD m, PassD ps, int *ca
     for (int q = gl; q < k; q += G)
       atomicMax(&m.claim[2 * (size_t)L[q] + ((ps.shared_ring && q >= n) ? 1 : 0)], key);
   }
+}
+
+template <int G>
+__global__ __launch_bounds__(LIST_BLOCK) void k_claim(MeshD m, PassD ps, int *cact) {
+  unsigned ws_seg = 0, ws_bad = 0;
+  claim_body<G>(m, ps, cact, (int)(blockIdx.x * blockDim.x + threadIdx.x),
+                (int)(gridDim.x * blockDim.x), ws_seg, ws_bad);
   if (ps.iter == 0) {
     const unsigned long long a = wave_sum(ws_seg), b = wave_sum(ws_bad);
     if ((threadIdx.x & 63) == 0) {
@@ -1133,12 +1177,13 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_claim(MeshD m, PassD ps, int *ca
 // a winner then stamps its region.  A stamp only replaces the winner's own
 // key, which no other candidate's test could match either.
 template <int G>
-__global__ __launch_bounds__(LIST_BLOCK) void k_win(MeshD m, PassD ps, const int *cact) {
+__device__ __forceinline__ void win_body(const MeshD &m, const PassD &ps, const int *cact, int tid,
+                                         int nthr) {
   const int nc = pass_nc(ps);
   const unsigned long long ep = pass_epoch(ps);
   const unsigned long long sticky = pass_sticky(ps);
-  const int gl = threadIdx.x % G, per = blockDim.x / G;
-  for (int i = blockIdx.x * per + threadIdx.x / G; i < nc; i += gridDim.x * per) {
+  const int gl = tid % G, per = nthr / G;
+  for (int i = tid / G; i < nc; i += per) {
     if (!cact[i]) continue;
     const unsigned long long key = claim_key(ep, ps.cprio[i], i);
     const int *L = ps.ws + (size_t)i * ps.R;
@@ -1165,6 +1210,12 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_win(MeshD m, PassD ps, const int
   }
 }
 
+template <int G>
+__global__ __launch_bounds__(LIST_BLOCK) void k_win(MeshD m, PassD ps, const int *cact) {
+  win_body<G>(m, ps, cact, (int)(blockIdx.x * blockDim.x + threadIdx.x),
+              (int)(gridDim.x * blockDim.x));
+}
+
 // Retriangulate a winner's cavity as the star of its new vertex; same star
 // order and slot rule as the oracle.  Also writes the new point, and for a
 // segment split the two subsegment halves.  Lane q of the group writes star
@@ -1172,10 +1223,11 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_win(MeshD m, PassD ps, const int
 // boundary edge.  The group's records are read (uniform loads) before any of
 // its lanes writes, and no lane reads a record another lane writes: the new
 // point's coordinates come from the candidate, not from P.
-template <int G>
+template <int G, class Trace>
 __device__ __forceinline__ void apply_one(const MeshD &m, const ParamsD &pr, const PassD &ps,
                                           int i, int gl, int nseg, const int *ids, int pbase,
-                                          int tbase, int sbase, unsigned long long &nflip) {
+                                          int tbase, int sbase, unsigned long long &nflip,
+                                          const Trace &trace) {
   {
     if (!ps.cwin[i]) return;
     // winners split subsegments first (candidates [0, nseg)), so a segment
@@ -1184,7 +1236,7 @@ __device__ __forceinline__ void apply_one(const MeshD &m, const ParamsD &pr, con
     {
       const unsigned long long wb = __ballot(gl == 0 && is_seg);
       if (wb != 0ull && (int)(threadIdx.x & 63) == __builtin_ctzll(wb))
-        atomicAdd(&ps.cnt[CNT_SEGWIN], (unsigned long long)__popcll(wb));
+        trace.seg_winners(ps, (unsigned)__popcll(wb));
     }
     const int rank = ps.crank[i];
     const int p = pbase + rank;
@@ -1243,6 +1295,7 @@ __device__ __forceinline__ void apply_one(const MeshD &m, const ParamsD &pr, con
       r.X[2] = Pv;
       r.pad[0] = r.pad[1] = make_int4(0, 0, 0, 0);
       m.T[st] = r;
+      trace.rewritten(m, st);
       m.tflag[st] = TF_ALIVE | TF_CHECK;
       if (o >= 0) *nbr_slot(m.T, o >> 2, o & 3) = (st << 2) | 0;
       if (s >= 0) {
@@ -1256,7 +1309,10 @@ __device__ __forceinline__ void apply_one(const MeshD &m, const ParamsD &pr, con
             const int2 sv = m.SV[s];
             enc = encroaches(m, lp, sv.x, sv.y, c.x, c.y);
           }
-          if (enc) m.senc[s] = 1;
+          if (enc) {
+            m.senc[s] = 1;
+            trace.encroached(s);
+          }
         }
       }
       if (is_seg) {
@@ -1294,6 +1350,7 @@ __device__ __forceinline__ void apply_one(const MeshD &m, const ParamsD &pr, con
         m.ST[sB] = kB == LLONG_MAX ? -1 : (int)(kB & 0xffffffffll);
         m.senc[sA] = eA ? 1 : 0;
         m.senc[sB] = eB ? 1 : 0;
+        if (eB) trace.encroached(sB);  // sA was a candidate: listed already
       }
     }
     if (gl == 0) {
@@ -1329,7 +1386,7 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_apply(MeshD m, ParamsD pr, PassD
   const int gl = threadIdx.x % G, per = blockDim.x / G;
   unsigned long long nflip = 0;
   for (int i = blockIdx.x * per + threadIdx.x / G; i < nc; i += gridDim.x * per)
-    apply_one<G>(m, pr, ps, i, gl, nseg, ids, pbase, tbase, sbase, nflip);
+    apply_one<G>(m, pr, ps, i, gl, nseg, ids, pbase, tbase, sbase, nflip, NoTrace{});
   nflip = wave_sum(nflip);
   if ((threadIdx.x & 63) == 0 && nflip) atomicAdd(&ps.cnt[CNT_FLIPS], nflip);
 }
@@ -1349,9 +1406,339 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_rank_apply(MeshD m, ParamsD pr, 
   const int gl = threadIdx.x % G, per = blockDim.x / G;
   unsigned long long nflip = 0;
   for (int i = threadIdx.x / G; i < nc; i += per)
-    apply_one<G>(m, pr, ps, i, gl, ps.nseg, ps.ids, pbase, tbase, sbase, nflip);
+    apply_one<G>(m, pr, ps, i, gl, ps.nseg, ps.ids, pbase, tbase, sbase, nflip, NoTrace{});
   nflip = wave_sum(nflip);
   if ((threadIdx.x & 63) == 0 && nflip) atomicAdd(&ps.cnt[CNT_FLIPS], nflip);
+}
+
+// ---------------------------------------------------------------------------
+// Small passes: whole rounds in one launch of one block.
+//
+// A pass over few candidates is a chain of 8 to 16 dependent launches (about
+// 4 us each for almost no work) and a host round trip.  Here one block of 16
+// waves runs the same steps with block barriers between them, pass after
+// pass, while every pass has at most SR_CAP candidates.  Steps and order are
+// the separate kernels' (the same device functions), so the mesh is the same
+// bit for bit.  Per-candidate arrays and the lists live in LDS; the
+// encroached subsegments and the triangles to test are listed as they change,
+// so no step scans the mesh.  The block returns to the host, at a pass
+// boundary, when a pass is larger, needs more mesh capacity, a list overflows
+// or the refinement ends; and inside a pass, after the cavities, when a
+// candidate needs the exact-predicate kernel, which the host then launches
+// (Refiner::run_pass with that pass to resume).
+// Bound by the cavities' dependent gathers and LDS chains (about 60% of a
+// pass); 16 waves of one CU.  A pass of 300 points' refinement takes 56 us
+// where the launches took 85 to 110 with the round trip; 8 waves (twice the
+// registers) took 59.  SR_CAP: a second and third batch of 64 cavities on the
+// one CU still costs less than the launches saved; at four batches the two
+// sides meet.
+// ---------------------------------------------------------------------------
+constexpr int SR_WAVES = 16, SR_THREADS = 64 * SR_WAVES;
+constexpr int SR_LG = 16;        // lanes per cavity
+constexpr int SR_K = 32;         // largest cavity held in LDS
+constexpr int SR_CAP = 256;      // candidates of a pass
+constexpr int SR_ENC = 1024;     // encroached subsegments listed
+constexpr int SR_DIRTY = 8192;   // rewritten triangles listed between two bad passes
+constexpr int SR_PASSES = 128;   // passes of one launch
+static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
+
+// The lists k_small_rounds keeps as passes change the mesh.
+struct ListTrace {
+  int *enc, *n_enc;      // LDS
+  int *dirty, *n_dirty;  // global list, LDS count
+  unsigned *cnt;         // LDS counters of the pass
+  int nt;                // slots from here on are new
+  bool track;            // the bad list is known: list what changes
+  __device__ void encroached(int s) const {
+    const int p = atomicAdd(n_enc, 1);
+    if (p < SR_ENC) enc[p] = s;
+  }
+  // once per slot between two marking passes: the first rewrite finds the
+  // check flag clear (a new slot's flags are not initialised)
+  __device__ void rewritten(const MeshD &m, int t) const {
+    if (track && (t >= nt || !(m.tflag[t] & TF_CHECK))) {
+      const int p = atomicAdd(n_dirty, 1);
+      if (p < SR_DIRTY) dirty[p] = t;
+    }
+  }
+  __device__ void seg_winners(const PassD &, unsigned n) const { atomicAdd(&cnt[CNT_SEGWIN], n); }
+};
+
+// One pass's counts of this thread into the block's LDS counters; deferred
+// candidates to a counter of their kind (read by all between two barriers).
+__device__ __forceinline__ void add_counts(CavCounts &cc, bool is_seg, unsigned *cnt,
+                                           unsigned *slow) {
+#pragma unroll
+  for (int k = 0; k < CC_N; k++)
+    if (cc.c[k]) atomicAdd(&cnt[cc_counter(k, is_seg)], cc.c[k]);
+  if (cc.c[CC_SLOW]) atomicAdd(&slow[is_seg ? 0 : 1], cc.c[CC_SLOW]);
+  for (int k = 0; k < CC_ALL; k++) cc.c[k] = 0u;
+}
+
+// Ascending order of the n distinct values in src (LDS, n <= SR_THREADS), to
+// dst: each thread counts the smaller values.  The caller synchronises.
+__device__ __forceinline__ void rank_sort(const int *src, int n, int *dst) {
+  if ((int)threadIdx.x < n) {
+    const int v = src[threadIdx.x];
+    int r = 0;
+    for (int x = 0; x < n; x++) r += src[x] < v;
+    dst[r] = v;
+  }
+}
+
+__global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr, PassD base,
+                                                             SmallArgs a) {
+  // the cavities' LDS; between them the network's and the sorts'
+  extern __shared__ __align__(16) int sm[];
+  __shared__ int s_enc[SR_ENC], s_bad[SR_CAP], s_ids[SR_CAP];
+  __shared__ double2 s_pt[SR_CAP];
+  __shared__ int s_status[SR_CAP], s_n[SR_CAP], s_r[SR_CAP], s_prio[SR_CAP], s_win[SR_CAP],
+      s_rank[SR_CAP], s_act[SR_CAP];
+  __shared__ unsigned s_cnt[CNT_N], s_slow[2];
+  __shared__ unsigned long long s_acc[CNT_N];
+  __shared__ int s_wave[SR_WAVES];
+  __shared__ int s_ne, s_nd, s_k;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  // uniform state
+  SmallState st = a.st;
+  bool known = st.nb >= 0;
+  int nb = known ? st.nb : 0;
+  int code = SR_BOUNDARY, stage = 0, nc = 0, nseg = 0, passes = 0;
+  if (tid < st.ne) s_enc[tid] = a.enc[tid];
+  if (tid < nb) s_bad[tid] = a.bad[tid];
+  if (tid < CNT_N) {
+    s_cnt[tid] = 0u;
+    s_acc[tid] = 0ull;
+  }
+  if (tid == 0) {
+    s_ne = st.ne;
+    s_nd = 0;
+    s_slow[0] = s_slow[1] = 0u;
+  }
+  __syncthreads();
+  CavCounts cc;
+  for (int k = 0; k < CC_ALL; k++) cc.c[k] = 0u;
+  for (; passes < SR_PASSES; passes++) {
+    nseg = st.ne;
+    int nbc = 0;
+    const bool seg_pass = st.ne > a.mix_below;
+    if (!seg_pass) {
+      // ---- bad triangles: the old list's survivors and the rewritten ones ----
+      const int nd = s_nd;
+      if (!known || nd > SR_DIRTY) break;
+      const int t0 = tid < nb ? s_bad[tid] : -1;
+      const uint8_t f0 = t0 >= 0 ? m.tflag[t0] : 0;
+      if (tid == 0) s_k = 0;
+      __syncthreads();
+      if ((f0 & (TF_ALIVE | TF_BAD | TF_GIVEUP | TF_CHECK)) == (TF_ALIVE | TF_BAD))
+        sm[atomicAdd(&s_k, 1)] = t0;
+      for (int q = tid; q < nd; q += SR_THREADS) {
+        const int t = a.dirty[q];
+        const uint8_t f = mark_bad_one(m, pr, t, m.tflag[t]);
+        if ((f & (TF_ALIVE | TF_BAD | TF_GIVEUP)) == (TF_ALIVE | TF_BAD)) {
+          const int p = atomicAdd(&s_k, 1);
+          if (p < 2 * SR_CAP) sm[p] = t;
+        }
+      }
+      __syncthreads();
+      nb = s_k;
+      if (nb > SR_CAP) {
+        known = false;
+        break;
+      }
+      rank_sort(sm, nb, s_bad);
+      if (tid == 0) s_nd = 0;
+      __syncthreads();
+      if (st.ne == 0 && nb == 0) {
+        code = SR_DONE;
+        st.status = 0;
+        break;
+      }
+      long long capb = (long long)a.cap - st.ne;
+      if (a.cand_factor > 0 && st.prev_win >= 0)
+        capb = min(capb, max((long long)a.cand_min, (long long)a.cand_factor * st.prev_win));
+      if (nb > capb) break;  // needs the selection by priority
+      nbc = nb;
+    }
+    nc = nseg + nbc;
+    const int iters = nbc == 0 ? a.seg_iters : a.bad_iters;
+    if (nc > SR_CAP || nc > a.cap || (a.del_on && nseg > 0) ||
+        st.epoch + iters + 3 >= (1 << 11) || st.np + (long long)nc > a.capP ||
+        st.nt + 2ll * nc > a.capT || st.ns + (long long)nseg > a.capS)
+      break;
+    if (tid < nseg) s_ids[tid] = s_enc[tid];
+    if (tid < nbc) s_ids[nseg + tid] = s_bad[tid];
+    PassD ps = base;
+    ps.ids = s_ids;
+    ps.nc = nc;
+    ps.nseg = nseg;
+    ps.iters = iters;
+    ps.epoch0 = ps.epoch = (unsigned long long)st.epoch + 1ull;
+    ps.iter = 0;
+    ps.cpt = s_pt;
+    ps.cstatus = s_status;
+    ps.cn = s_n;
+    ps.cr = s_r;
+    ps.cprio = s_prio;
+    ps.cwin = s_win;
+    ps.crank = s_rank;
+    ps.feat = nbc > 0 ? a.feat : nullptr;
+    ps.pass_index = st.pass_index;
+    const ListTrace trace{s_enc, &s_ne, a.dirty, &s_nd, s_cnt, st.nt, known};
+    __syncthreads();
+    // ---- cavities ----
+    int *cav = sm + wave * (64 / SR_LG) * group_lds_ints(min(ps.K, ps.Kf), SR_LG);
+    if (nseg > 0) {
+      cavity_wave<true, SR_LG, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
+      add_counts(cc, true, s_cnt, s_slow);
+      __syncthreads();
+      if (s_slow[0] != 0u) {
+        code = SR_SLOW;
+        stage = 1;
+        break;
+      }
+    }
+    if (nbc > 0) {
+      cavity_wave<false, SR_LG, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
+      add_counts(cc, false, s_cnt, s_slow);
+      __syncthreads();
+      if (s_slow[1] != 0u) {
+        code = SR_SLOW;
+        stage = 2;
+        break;
+      }
+      if (a.mlp) {
+        MlpWeights &w = *reinterpret_cast<MlpWeights *>(sm);
+        short *H = reinterpret_cast<short *>(sm) + sizeof(MlpWeights) / sizeof(short) +
+                   wave * 16 * H1_STRIDE;
+        mlp_stage<SR_THREADS>(a.mlp, w, tid);
+        __syncthreads();
+        for (int row0 = wave * 16; row0 < nbc; row0 += SR_WAVES * 16) {
+          mlp_rows16(a.feat + (size_t)nseg * FEAT, nbc, row0, w, H, a.score + nseg);
+          wave_sync();
+        }
+        ps.score = a.score;
+        ps.lshift = a.lshift;
+        __syncthreads();
+      }
+    }
+    // ---- claims ----
+    unsigned ws_seg = 0, ws_bad = 0;
+    for (int it = 0; it < iters; it++) {
+      ps.epoch = (unsigned long long)++st.epoch;
+      ps.iter = it;
+      claim_body<CLAIM_LANES>(m, ps, s_act, tid, SR_THREADS, ws_seg, ws_bad);
+      __syncthreads();
+      win_body<CLAIM_LANES>(m, ps, s_act, tid, SR_THREADS);
+      __syncthreads();
+    }
+    ++st.epoch;  // the winners' stamp epoch
+    if (ws_seg) atomicAdd(&s_cnt[CNT_WS_SEG], ws_seg);
+    if (ws_bad) atomicAdd(&s_cnt[CNT_WS_BAD], ws_bad);
+    // ---- ranks and apply ----
+    const bool win = tid < nc && s_win[tid] != 0;
+    const unsigned long long wb = __ballot(win);
+    if (lane == 0) s_wave[wave] = __popcll(wb);
+    __syncthreads();
+    int before = 0, nwin = 0;
+    for (int w = 0; w < SR_WAVES; w++) {
+      const int c = s_wave[w];
+      if (w < wave) before += c;
+      nwin += c;
+    }
+    if (win) s_rank[tid] = before + __popcll(wb & ((1ull << lane) - 1ull));
+    __syncthreads();
+    unsigned long long nflip = 0;
+    for (int i = tid / APPLY_LANES; i < nc; i += SR_THREADS / APPLY_LANES)
+      apply_one<APPLY_LANES>(m, pr, ps, i, tid % APPLY_LANES, nseg, s_ids, st.np, st.nt, st.ns,
+                             nflip, trace);
+    if (nflip) atomicAdd(&s_cnt[CNT_FLIPS], (unsigned)nflip);
+    if (tid == 0) s_cnt[CNT_NWIN] = (unsigned)nwin;
+    __syncthreads();
+    // ---- what the pass did ----
+    const int nws = (int)s_cnt[CNT_SEGWIN], listed = s_ne;
+    const bool ovf = s_cnt[CNT_OVERFLOW] > 0;
+    long long prog = (long long)nwin + s_cnt[CNT_MARKS] + s_cnt[CNT_GIVEUPS];
+    st.np += nwin;
+    st.nt += 2 * nwin;
+    st.ns += nws;
+    const int es = tid < min(listed, SR_ENC) ? s_enc[tid] : -1;
+    const bool still = es >= 0 && __hip_atomic_load(&m.senc[es], __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT) == 1;
+    if (tid == 0) s_k = 0;
+    __syncthreads();
+    if (still) sm[atomicAdd(&s_k, 1)] = es;
+    if (tid < CNT_N) {
+      s_acc[tid] += s_cnt[tid];
+      s_cnt[tid] = 0u;
+    }
+    __syncthreads();
+    st.ne = s_k;
+    rank_sort(sm, st.ne, s_enc);
+    if (tid == 0) s_ne = st.ne;
+    __syncthreads();
+    if (listed > SR_ENC) st.ne = -1;
+    const bool grow = ovf && base.K < a.kmax;
+    if (seg_pass) {
+      st.seg_passes++;
+    } else {
+      if (nseg > 0) st.seg_passes++;
+      if (nbc > 0) {
+        st.pass_index++;
+        st.bad_passes++;
+        st.cand_evals += nbc;
+        st.prev_win = nwin - nws;
+      }
+      if (grow) prog++;
+      if (prog == 0) {
+        code = SR_DONE;
+        st.status = 2;
+        passes++;
+        break;
+      }
+      st.round++;
+      if (st.round >= a.max_rounds) {
+        code = SR_ROUNDS;
+        passes++;
+        break;
+      }
+      st.np_round = st.np;
+    }
+    st.grow = grow ? 1 : 0;
+    if (grow || st.ne < 0) {
+      passes++;
+      break;
+    }
+  }
+  // ---- back to the host ----
+  __syncthreads();
+  if (code == SR_SLOW) {  // this pass's candidates and counts, for the separate kernels
+    if (tid < nc) {
+      a.ids_out[tid] = s_ids[tid];
+      base.cpt[tid] = s_pt[tid];
+      base.cstatus[tid] = s_status[tid];
+      base.cn[tid] = s_n[tid];
+      base.cr[tid] = s_r[tid];
+      base.cprio[tid] = s_prio[tid];
+    }
+    if (tid < CNT_N && tid != CNT_SLOW) base.cnt[tid] = s_cnt[tid];
+  } else if (tid < st.ne) {
+    a.enc_out[tid] = s_enc[tid];
+  }
+  if (tid < CNT_N)
+    __hip_atomic_store(&a.out->acc[tid], s_acc[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (tid == 0) {
+    st.code = code;
+    st.stage = stage;
+    st.nc = nc;
+    st.nseg = nseg;
+    st.passes = passes;
+    const int *src = reinterpret_cast<const int *>(&st);
+    int *dst = reinterpret_cast<int *>(&a.out->st);
+    for (int k = 0; k < (int)(sizeof(SmallState) / sizeof(int)); k++)
+      __hip_atomic_store(dst + k, src[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  __threadfence_system();
 }
 
 // ---------------------------------------------------------------------------
@@ -2249,6 +2636,8 @@ Refiner::~Refiner() {
   if (h_scalar) (void)hipHostFree(h_scalar);
   if (h_total) (void)hipHostFree(h_total);
   if (h_cnt) (void)hipHostFree(h_cnt);
+  if (sr_out) (void)hipHostFree(sr_out);
+  dfree(sr_dirty);
   dfree(d_val);
   if (h_val4) (void)hipHostFree(h_val4);
   delete copier;
@@ -2557,7 +2946,8 @@ const char *Refiner::kname(int id) {
   static const char *names[] = {"init",       "mark_bad", "compact",
                                 "seg_cavity", "bad_cavity", "claim",
                                 "win",        "apply",      "export",
-                                "mlp",        "del_scan",   "del_apply"};
+                                "mlp",        "del_scan",   "del_apply",
+                                "small_rounds"};
   return names[id];
 }
 
@@ -2838,8 +3228,11 @@ void Refiner::enqueue_claims(PassD ps, int gc, int iters) {
 // list_enc: also list the subsegments encroached after the pass in tmp_list
 // (listed_enc), queued behind the apply kernel so that one synchronisation
 // serves both; the next segment phase then starts from that list.
+//
+// resume: the pass k_small_rounds left (SR_SLOW), whose filtered cavities are
+// done up to its stage (1 the subsegments', 2 all).
 int Refiner::run_pass(const int *ids, int nc, int nseg, long long *progress, bool *overflowed,
-                      int *nwin_seg, bool list_enc) {
+                      int *nwin_seg, bool list_enc, int resume) {
   const int nbad = nc - nseg;
   // room for every candidate winning: the winners' count is only read back
   // with the pass counters, after the apply kernel
@@ -2851,24 +3244,16 @@ int Refiner::run_pass(const int *ids, int nc, int nseg, long long *progress, boo
   ps.nseg = nseg;
   const int iters = iters_for(nseg == nc);
   ps.iters = iters;
-  if (epoch + iters + 3 >= (1ull << 11)) {  // epoch wrap: clear claims
-    HC(hipMemsetAsync(m.claim, 0, sizeof(unsigned long long) * 2 * capT, stream));
-    epoch = 0;
-  }
+  wrap_epoch(iters);
   ps.iter = 0;
   bool want_feat = nbad > 0 && (opt.priority == 2 || opt.log_training);
-  if (want_feat && nc > feat_cap) {
-    dfree(c_feat); dfree(c_score); dfree(c_deg);
-    feat_cap = std::max(nc, 2 * feat_cap);
-    dalloc(&c_feat, (size_t)feat_cap * FEAT);
-    dalloc(&c_score, (size_t)feat_cap);
-    dalloc(&c_deg, (size_t)feat_cap);
-  }
+  if (want_feat) ensure_feat(nc);
   ps.feat = want_feat ? c_feat : nullptr;
   ps.pass_index = pass_index;
-  if (!cnt_zero) HC(hipMemsetAsync(d_cnt, 0, CNT_N * sizeof(unsigned long long), stream));
+  if (!resume && !cnt_zero)
+    HC(hipMemsetAsync(d_cnt, 0, CNT_N * sizeof(unsigned long long), stream));
   cnt_zero = false;
-  if (del_on && nseg > 0) {  // vertex deletion first, with its own claim epoch
+  if (!resume && del_on && nseg > 0) {  // vertex deletion first, with its own claim epoch
     DelD dd = del_base();
     dd.ids = ids;
     dd.nseg = nseg;
@@ -2885,12 +3270,12 @@ int Refiner::run_pass(const int *ids, int nc, int nseg, long long *progress, boo
   };
   if (nseg > 0) {
     tbegin(K_SEGCAV);
-    launch_cavity(true, cav_grid(nseg), ps);
+    if (resume != 2) launch_cavity(true, cav_grid(nseg), ps, resume == 1);
     tend(K_SEGCAV, nseg);
   }
   if (nbad > 0) {
     tbegin(K_BADCAV);
-    launch_cavity(false, cav_grid(nbad), ps);
+    launch_cavity(false, cav_grid(nbad), ps, resume == 2);
     tend(K_BADCAV, nbad);
   }
   HC(hipGetLastError());
@@ -2950,32 +3335,195 @@ int Refiner::run_pass(const int *ids, int nc, int nseg, long long *progress, boo
   const int nwin = (int)h_cnt[CNT_NWIN];
   const int nws = (int)h_cnt[CNT_SEGWIN];
   const long long ndel = (long long)h_cnt[CNT_DEL];
-  st.deleted += ndel;
-  st.flips += (long long)h_cnt[CNT_FLIPS];
-  if (opt.profile && !capturing) ktimes[K_APPLY].items += nwin;  // winners applied
+  add_pass_stats(h_cnt);
   np += nwin;
   nt += 2 * nwin;
   ns += nws;
-  st.rej_overflow += h_cnt[CNT_OVERFLOW];
-  st.rej_encroach += h_cnt[CNT_REJ_ENC];
-  st.rej_blocked += h_cnt[CNT_REJ_BLOCKED];
-  st.giveups += h_cnt[CNT_GIVEUPS];
-  st.lost += (long long)h_cnt[CNT_VALID] - nwin;
-  st.pred_fp32 += h_cnt[CNT_FP32];
-  st.pred_fp64 += h_cnt[CNT_FP64];
-  st.pred_exact += h_cnt[CNT_EXACT];
-  st.pred_dd += h_cnt[CNT_DD];
-  st.big_cavities += h_cnt[CNT_BIG];
-  st.tri_examined_seg += h_cnt[CNT_EXAM_SEG];
-  st.tri_examined_bad += h_cnt[CNT_EXAM_BAD];
-  st.ws_ints_seg += h_cnt[CNT_WS_SEG];
-  st.ws_ints_bad += h_cnt[CNT_WS_BAD];
-  st.seg_splits += nws;
-  st.inserted += nwin - nws;
   *progress = nwin + ndel + (long long)h_cnt[CNT_MARKS] + (long long)h_cnt[CNT_GIVEUPS];
   *overflowed = h_cnt[CNT_OVERFLOW] > 0;
   *nwin_seg = nws;
   return nwin;
+}
+
+// Room for a pass's claim epochs: near the wrap the claims are cleared.
+void Refiner::wrap_epoch(int iters) {
+  if (epoch + iters + 3 < (1ull << 11)) return;
+  HC(hipMemsetAsync(m.claim, 0, sizeof(unsigned long long) * 2 * capT, stream));
+  epoch = 0;
+}
+
+void Refiner::ensure_feat(int nc) {
+  if (nc <= feat_cap) return;
+  dfree(c_feat); dfree(c_score); dfree(c_deg);
+  feat_cap = std::max(nc, 2 * feat_cap);
+  dalloc(&c_feat, (size_t)feat_cap * FEAT);
+  dalloc(&c_score, (size_t)feat_cap);
+  dalloc(&c_deg, (size_t)feat_cap);
+}
+
+// A pass of nc candidates, nseg of them subsegments, that k_small_rounds
+// takes.  Vertex deletion and the training logs need the separate kernels.
+bool Refiner::small_pass(int nc, int nseg) const {
+  return nc > 0 && nc <= SR_CAP && !opt.log_training && !(del_on && nseg > 0) &&
+         (opt.priority != 2 || mlp_params);
+}
+
+// Rounds from the segment check on, while their passes are small: ne
+// encroached subsegments in enc and, unless nb < 0 (unknown), the nb bad
+// triangles in bad.  Returns false when no pass was run (the caller's next
+// pass takes the separate kernels); *done: the refinement has ended.
+bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *round,
+                        int *prev_win, bool *done) {
+  *done = false;
+  const bool seg = ne > opt.mix_below;
+  const int nc = ne + (seg ? 0 : std::max(nb, 0)), nseg = ne;
+  ensure_capacity(np + (long long)nc, nt + 2LL * nc, ns + (long long)nseg);
+  ensure_ws((long long)SR_CAP * (6LL * K + 16));
+  ensure_cand(SR_CAP);
+  ensure_mix(SR_CAP);
+  wrap_epoch(std::max(iters_for(true), iters_for(false)));
+  if (opt.priority == 2) ensure_feat(SR_CAP);
+  if (!sr_dirty) dalloc(&sr_dirty, (size_t)SR_DIRTY);
+  if (!sr_out) {
+    HC(hipHostMalloc((void **)&sr_out, sizeof(SmallOut), hipHostMallocMapped));
+    HC(hipHostGetDevicePointer((void **)&d_sr_out, sr_out, 0));
+  }
+  if (!cnt_zero) HC(hipMemsetAsync(d_cnt, 0, CNT_N * sizeof(unsigned long long), stream));
+  cnt_zero = true;
+  PassD ps = pass_base(K);
+  ps.Kf = std::min(ps.Kf, SR_K);
+  SmallArgs a{};
+  a.st.np = np;
+  a.st.nt = nt;
+  a.st.ns = ns;
+  a.st.epoch = (int)epoch;
+  a.st.pass_index = pass_index;
+  a.st.prev_win = *prev_win;
+  a.st.round = *round;
+  a.st.np_round = np_round;
+  a.st.ne = ne;
+  a.st.nb = nb;
+  a.st.status = st.status;
+  a.enc = enc;
+  a.bad = bad;
+  a.enc_out = tmp_list;
+  a.ids_out = mix_list;
+  a.dirty = sr_dirty;
+  if (opt.priority == 2) {
+    a.feat = c_feat;
+    a.score = c_score;
+    a.mlp = mlp_params;
+  }
+  a.lshift = opt.learned_shift;
+  a.mix_below = opt.mix_below;
+  a.cap = cands_per_pass(K);
+  a.cand_factor = opt.cand_factor;
+  a.cand_min = opt.cand_min;
+  a.kmax = opt.cav_cap_max;
+  a.seg_iters = iters_for(true);
+  a.bad_iters = iters_for(false);
+  a.max_rounds = opt.max_rounds;
+  a.del_on = del_on ? 1 : 0;
+  a.capP = capP;
+  a.capT = capT;
+  a.capS = capS;
+  a.out = d_sr_out;
+  const size_t lds =
+      std::max(sizeof(int) * (size_t)(SR_THREADS / SR_LG) * group_lds_ints(std::min(K, ps.Kf), SR_LG),
+               sizeof(MlpWeights) + sizeof(short) * SR_WAVES * 16 * H1_STRIDE);
+  tbegin(K_SMALL);
+  k_small_rounds<<<1, SR_THREADS, lds, stream>>>(m, pr, ps, a);
+  tend(K_SMALL, 0);
+  HC(hipGetLastError());
+  HC(hipStreamSynchronize(stream));
+  const SmallState &o = sr_out->st;
+  const unsigned long long *c = sr_out->acc;
+  np = o.np;
+  nt = o.nt;
+  ns = o.ns;
+  epoch = (unsigned long long)o.epoch;
+  pass_index = o.pass_index;
+  *prev_win = o.prev_win;
+  *round = o.round;
+  np_round = o.np_round;
+  listed_enc = o.code == SR_SLOW ? -1 : o.ne;
+  st.status = o.status;
+  st.rounds = o.code == SR_ROUNDS ? o.round : o.round + 1;
+  st.seg_passes += o.seg_passes;
+  st.bad_passes += o.bad_passes;
+  st.cand_evals += o.cand_evals;
+  add_pass_stats(c);
+  if (o.code == SR_DONE || o.code == SR_ROUNDS) {
+    *done = true;
+    return true;
+  }
+  if (o.code == SR_SLOW) {
+    long long prog = 0;
+    bool of = false;
+    int nws = 0;
+    const int nc1 = o.nc, nseg1 = o.nseg;  // the mapped copy may be rewritten
+    const bool seg1 = nseg1 > opt.mix_below;
+    const int nwin = run_pass(mix_list, nc1, nseg1, &prog, &of, &nws, true, o.stage);
+    if (seg1)
+      after_seg_pass(of);
+    else
+      *done = after_bad_pass(nseg1, nc1 - nseg1, nwin, nws, prog, of, prev_win, round);
+    return true;
+  }
+  if (o.grow) K = std::min(2 * K, opt.cav_cap_max);
+  return o.passes > 0;
+}
+
+void Refiner::after_seg_pass(bool of) {
+  st.seg_passes++;
+  if (of && K < opt.cav_cap_max) K = std::min(2 * K, opt.cav_cap_max);
+}
+
+// The end of a round: true when the refinement has ended.
+bool Refiner::after_bad_pass(int ne, int nbc, int nwin, int nws, long long prog, bool of,
+                             int *prev_win, int *round) {
+  if (ne > 0) st.seg_passes++;
+  if (nbc > 0) {
+    pass_index++;
+    st.bad_passes++;
+    st.cand_evals += nbc;
+    *prev_win = nwin - nws;
+  }
+  if (of && K < opt.cav_cap_max) {
+    K = std::min(2 * K, opt.cav_cap_max);
+    prog++;
+  }
+  if (prog == 0) {
+    st.status = 2;
+    return true;
+  }
+  if (++*round >= opt.max_rounds) return true;
+  st.rounds = *round + 1;
+  np_round = np;
+  return false;
+}
+
+// Pass counters into the run's statistics.
+void Refiner::add_pass_stats(const unsigned long long *c) {
+  st.deleted += (long long)c[CNT_DEL];
+  st.flips += (long long)c[CNT_FLIPS];
+  st.rej_overflow += c[CNT_OVERFLOW];
+  st.rej_encroach += c[CNT_REJ_ENC];
+  st.rej_blocked += c[CNT_REJ_BLOCKED];
+  st.giveups += c[CNT_GIVEUPS];
+  st.lost += (long long)c[CNT_VALID] - (long long)c[CNT_NWIN];
+  st.pred_fp32 += c[CNT_FP32];
+  st.pred_fp64 += c[CNT_FP64];
+  st.pred_exact += c[CNT_EXACT];
+  st.pred_dd += c[CNT_DD];
+  st.big_cavities += c[CNT_BIG];
+  st.tri_examined_seg += c[CNT_EXAM_SEG];
+  st.tri_examined_bad += c[CNT_EXAM_BAD];
+  st.ws_ints_seg += c[CNT_WS_SEG];
+  st.ws_ints_bad += c[CNT_WS_BAD];
+  st.seg_splits += c[CNT_SEGWIN];
+  st.inserted += (long long)c[CNT_NWIN] - (long long)c[CNT_SEGWIN];
+  if (opt.profile && !capturing) ktimes[K_APPLY].items += (long long)c[CNT_NWIN];  // winners applied
 }
 
 void Refiner::run() {
@@ -3131,35 +3679,42 @@ void Refiner::run() {
   collect_times();
 }
 
-// Host-driven rounds: the host reads every count and decides every step.
+// Host-driven rounds: the host reads every count and decides every step;
+// runs of small passes go to k_small_rounds.
 void Refiner::loop_host() {
   int prev_win = -1;
   listed_enc = -1;
   ensure_cand(std::min(cands_per_pass(K), std::max(4 * nt0, 1024)));
-  for (int round = 0; round < opt.max_rounds; round++) {
-    st.rounds = round + 1;
+  int round = 0;
+  bool done = opt.max_rounds <= 0;
+  if (!done) {
+    st.rounds = 1;
     np_round = np;
+  }
+  while (!done) {
     // segment phase: until at most mix_below subsegments are encroached
     int ne;
-    for (;;) {
-      if (listed_enc >= 0) {  // listed behind the last pass
-        ne = listed_enc;
-        listed_enc = -1;
-      } else {
-        ensure_tmp(ns);
-        ne = compact(PredSenc{m.senc}, ns, tmp_list, nullptr, nullptr);
-      }
-      if (ne <= opt.mix_below) break;
-      int nc = std::min(ne, cands_per_pass(K));
-      ensure_cand(nc);
-      long long prog = 0;
-      bool of = false;
-      int nws = 0;
-      run_pass(tmp_list, nc, nc, &prog, &of, &nws, true);
-      st.seg_passes++;
-      if (of && K < opt.cav_cap_max) K = std::min(2 * K, opt.cav_cap_max);
+    if (listed_enc >= 0) {  // listed behind the last pass
+      ne = listed_enc;
+      listed_enc = -1;
+    } else {
+      ensure_tmp(std::max(ns, SR_ENC));
+      ne = compact(PredSenc{m.senc}, ns, tmp_list, nullptr, nullptr);
     }
-    if (bad_pass(ne, &prev_win)) break;
+    if (ne <= opt.mix_below) {
+      done = bad_pass(ne, &prev_win, &round);
+      continue;
+    }
+    int nc = std::min(ne, cands_per_pass(K));
+    if (nc == ne && small_pass(nc, nc) &&
+        run_small(tmp_list, ne, nullptr, -1, &round, &prev_win, &done))
+      continue;
+    ensure_cand(nc);
+    long long prog = 0;
+    bool of = false;
+    int nws = 0;
+    run_pass(tmp_list, nc, nc, &prog, &of, &nws, true);
+    after_seg_pass(of);
   }
 }
 
@@ -3168,22 +3723,26 @@ void Refiner::loop_host() {
 void Refiner::loop_mixed() {
   int prev_win = -1;
   ensure_cand(std::min(cands_per_pass(K), std::max(4 * nt0, 1024)));
-  for (int round = 0; round < opt.max_rounds; round++) {
-    st.rounds = round + 1;
+  int round = 0;
+  bool done = opt.max_rounds <= 0;
+  if (!done) {
+    st.rounds = 1;
     np_round = np;
+  }
+  while (!done) {
     ensure_tmp(ns);
     int ne = compact(PredSenc{m.senc}, ns, tmp_list, nullptr, nullptr);
-    if (bad_pass(ne, &prev_win)) break;
+    done = bad_pass(ne, &prev_win, &round);
   }
 }
 
 // A round's bad pass: the ne encroached subsegments listed in tmp_list (none
 // in the reference's round) first, then the selected bad triangles.
 // Returns true when the refinement has ended (st.status set).
-bool Refiner::bad_pass(int ne, int *prev_win) {
+bool Refiner::bad_pass(int ne, int *prev_win, int *round) {
   const int cap = cands_per_pass(K);
   ne = std::min(ne, cap);
-  ensure_mix(std::min<long long>((long long)ns + nt, (long long)cap + 1));
+  ensure_mix(std::max<long long>(SR_CAP, std::min<long long>((long long)ns + nt, (long long)cap + 1)));
   if (ne > 0)
     HC(hipMemcpyAsync(mix_list, tmp_list, sizeof(int) * (size_t)ne, hipMemcpyDeviceToDevice, stream));
   ensure_tmp(nt);
@@ -3213,27 +3772,16 @@ bool Refiner::bad_pass(int ne, int *prev_win) {
     ids = mix_list;
   }
   const int nc = ne + nbc;
+  bool done = false;
+  if (!opt.mixed && nbc == nb && small_pass(nc, ne) &&
+      run_small(mix_list, ne, tmp_list, nb, round, prev_win, &done))
+    return done;
   ensure_cand(nc);
   long long prog = 0;
   bool of = false;
   int nws = 0;
   int nwin = run_pass(ids, nc, ne, &prog, &of, &nws, !opt.mixed);
-  if (ne > 0) st.seg_passes++;
-  if (nbc > 0) {
-    pass_index++;
-    st.bad_passes++;
-    st.cand_evals += nbc;
-    *prev_win = nwin - nws;
-  }
-  if (of && K < opt.cav_cap_max) {
-    K = std::min(2 * K, opt.cav_cap_max);
-    prog++;
-  }
-  if (prog == 0) {
-    st.status = 2;
-    return true;
-  }
-  return false;
+  return after_bad_pass(ne, nbc, nwin, nws, prog, of, prev_win, round);
 }
 
 void Refiner::ensure_mix(long long n) {
@@ -3307,7 +3855,8 @@ static void launch_cavity_t(int lg, int grid, size_t lds, hipStream_t s, const M
 
 // Filtered-predicate pass over all candidates, then the exact-predicate pass
 // over the candidates it deferred (their count stays on the device).
-void Refiner::launch_cavity(bool is_seg, int grid, const PassD &ps) {
+// resumed: the filtered pass already ran (k_small_rounds).
+void Refiner::launch_cavity(bool is_seg, int grid, const PassD &ps, bool resumed) {
   int kf = std::min(ps.K, ps.Kf);
   // the exact kernel takes a whole wave per candidate: its candidates are
   // the cavities beyond the fast kernel's LDS (33..K triangles, whose sort
@@ -3320,10 +3869,10 @@ void Refiner::launch_cavity(bool is_seg, int grid, const PassD &ps) {
   if (grid < 1) grid = 1;
   int slow_grid = std::min(grid, pws_blocks * 4);
   if (is_seg) {
-    launch_cavity_t<true, true>(lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
+    if (!resumed) launch_cavity_t<true, true>(lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
     launch_cavity_t<true, false>(lgs, slow_grid, lds_slow, stream, m, pr, ps, opt.cav_cap_max);
   } else {
-    launch_cavity_t<false, true>(lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
+    if (!resumed) launch_cavity_t<false, true>(lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
     launch_cavity_t<false, false>(lgs, slow_grid, lds_slow, stream, m, pr, ps, opt.cav_cap_max);
   }
   HC(hipGetLastError());

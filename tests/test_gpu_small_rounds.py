@@ -1,0 +1,74 @@
+"""Runs of small passes in one launch (k_small_rounds) against the separate
+kernels.  The training logs need the separate kernels, so the same options
+with log_training = 1 never take the one-launch path: mesh and statistics have
+to be equal bit for bit.  The inputs cross the limits of the path: passes of
+more and fewer candidates than it takes, cavities beyond its LDS and undecided
+signs (left to the exact kernel inside a pass), capacity doubling and mesh
+growth, the selection by priority, a round limit, and lists reallocated while
+they grow (vmm = 0)."""
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CHOSEN = dict(pred_mode=1, claim_iters=3, seg_claim_iters=2, mix_below=4, shared_ring=1,
+              cand_factor=3, learned_shift=1)
+CASES = [
+    (9, 0, {}),
+    (40, 1, {}),
+    (300, 0, {}),
+    (300, 0, dict(CHOSEN, priority=1)),
+    (301, 1, dict(CHOSEN, priority=2)),
+    (2000, 0, dict(CHOSEN, priority=2)),
+    (2000, 1, dict(CHOSEN, priority=1, vmm=0)),
+    (1203, 3, dict(CHOSEN, priority=2, theta=30.0)),
+    (1200, 2, dict(CHOSEN, priority=1)),
+    (700, 0, dict(max_rounds=7)),
+    (700, 0, dict(CHOSEN, priority=2, max_rounds=11)),
+    (900, 0, dict(cand_min=40, cand_factor=2)),
+    (900, 1, dict(cand_min=40, cand_factor=2, priority=0)),
+    (800, 1, dict(cav_cap0=4)),
+    (800, 0, dict(CHOSEN, priority=1, cav_cap0=4, cav_cap_max=8)),
+    (800, 0, dict(CHOSEN, priority=2, cav_lds_cap=6)),
+    (600, 0, dict(cand_budget=16 * 208, cav_cap_max=64)),
+    (700, 1, dict(CHOSEN, priority=2, mode=0)),
+    (1500, 0, dict(mode=0, deletion=0)),
+    (1500, 1, dict(mode=0, deletion=1, vmm=0)),
+    (500, 0, dict(mode=1, deletion=2, claim_iters=2, mix_below=300)),
+]
+SAME = ["rounds", "seg_passes", "bad_passes", "status", "seg_splits", "inserted", "lost",
+        "rej_encroach", "rej_blocked", "rej_overflow", "giveups", "cand_evals", "deleted", "flips",
+        "n_points", "n_triangles", "n_subsegs", "final_cav_cap", "pred_fp32", "pred_fp64",
+        "pred_exact", "pred_dd", "tri_examined_seg", "tri_examined_bad", "ws_ints_seg",
+        "ws_ints_bad"]
+
+
+def _run(gpu, mesh, opt, log):
+    o = dict(opt)
+    s = gpu.Session(*mesh, theta=o.pop("theta", 25.0), mode=o.pop("mode", 1), log_training=log,
+                    cav_lds_cap=o.pop("cav_lds_cap", 32), **o)
+    try:
+        if opt.get("priority") == 2:
+            s.set_priority_model(np.load(os.path.join(os.path.dirname(gpu.__file__),
+                                                      "priority_mlp.npy")))
+        s.run()
+        st = s.run()  # the second run starts from a used session
+        return s.download(), st
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("n,dist,opt", CASES)
+def test_small_rounds_equal_separate_kernels(gpu, n, dist, opt):
+    print(f"small rounds n={n} dist={dist} {opt}", flush=True)
+    P, S0 = gpu.generate_pslg(n, max(1, n // 20), L=64.0 * n ** 0.5, maxlen=1280.0, dist=dist,
+                              min_angle=5.0, seed=100 + n)
+    mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    a, sa = _run(gpu, mesh, opt, 0)
+    b, sb = _run(gpu, mesh, opt, 1)
+    assert {k: sa[k] for k in SAME} == {k: sb[k] for k in SAME}
+    assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
+    for f in ("triangles", "neighbors", "segments", "pstatus", "tstatus"):
+        assert np.array_equal(getattr(a, f), getattr(b, f)), f
