@@ -192,6 +192,8 @@ struct PassD {
   Ctl *ctl;
   const int *ids_sel;  // selected candidates when ctl->i[C_USESEL]
   int *slow;           // candidates whose filters could not decide a sign
+  int2 *cseed;         // located candidates: first cavity triangles and the
+  double *cnear;       // near-vertex distance (squared)
   int eskip;  // graph loop: the pass's vertex deletion step took an epoch
   // learned priority folded in by the first claim iteration (host loop):
   // the network's scores, and the bucket coarsening shift; nullptr: cprio

@@ -208,6 +208,8 @@ class Refiner {
   double2 *c_pt = nullptr;
   int *c_status = nullptr, *c_n = nullptr, *c_r = nullptr, *c_prio = nullptr,
       *c_win = nullptr, *c_rank = nullptr, *c_act = nullptr, *c_slow = nullptr;
+  int2 *c_seed = nullptr;
+  double *c_near = nullptr;
   int *c_ws = nullptr;
   long long ws_ints = 0;
   double *c_pws = nullptr;

@@ -446,10 +446,10 @@ __global__ __launch_bounds__(MB) void k_mark_bad_count(MeshD m, ParamsD pr, int 
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void flush_stats(unsigned long long *cnt,
                                             const PredStats &st) {
-  if (st.fp32_hits) atomicAdd(&cnt[CNT_FP32], st.fp32_hits);
-  if (st.fp64_hits) atomicAdd(&cnt[CNT_FP64], st.fp64_hits);
-  if (st.exact_calls) atomicAdd(&cnt[CNT_EXACT], st.exact_calls);
-  if (st.dd_hits) atomicAdd(&cnt[CNT_DD], st.dd_hits);
+  if (st.fp32_hits) atomicAdd(&cnt[CNT_FP32], (unsigned long long)st.fp32_hits);
+  if (st.fp64_hits) atomicAdd(&cnt[CNT_FP64], (unsigned long long)st.fp64_hits);
+  if (st.exact_calls) atomicAdd(&cnt[CNT_EXACT], (unsigned long long)st.exact_calls);
+  if (st.dd_hits) atomicAdd(&cnt[CNT_DD], (unsigned long long)st.dd_hits);
 }
 
 __device__ __forceinline__ void mark_enc(const MeshD &m, int s,
@@ -476,47 +476,44 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long x) {
   return x;
 }
 
-// Per-lane event counts of the cavity kernel, summed over the wave in LDS and
-// added to the pass counters once per wave, all counters in one instruction:
-// a counter shared by every candidate would otherwise serialise on one L2
+// Event counts of the cavity kernels: rare events (one per candidate at most)
+// straight into the block's LDS counters, the frequent ones in registers and
+// added there at the end; then all counters to the pass's in one instruction.
+// A counter shared by every candidate would otherwise serialise on one L2
 // address, and a shuffle sum per counter is a serial chain at the end of
 // every wave (segment cavities of a 10^6-point refinement 59.6 us a launch
 // with the shuffles, 49.1 without).
-enum { CC_MARKS = 0, CC_GIVEUPS, CC_OVERFLOW, CC_REJ_ENC, CC_REJ_BLOCKED, CC_VALID,
-       CC_FP32, CC_FP64, CC_DD, CC_EXACT, CC_EXAM, CC_N,
-       CC_SLOW = CC_N, CC_ALL };  // CC_SLOW: deferred (counted by ps.cnt itself)
-__device__ __forceinline__ int cc_counter(int k, bool is_seg) {
-  switch (k) {
-    case CC_MARKS: return CNT_MARKS;
-    case CC_GIVEUPS: return CNT_GIVEUPS;
-    case CC_OVERFLOW: return CNT_OVERFLOW;
-    case CC_REJ_ENC: return CNT_REJ_ENC;
-    case CC_REJ_BLOCKED: return CNT_REJ_BLOCKED;
-    case CC_VALID: return CNT_VALID;
-    case CC_FP32: return CNT_FP32;
-    case CC_FP64: return CNT_FP64;
-    case CC_DD: return CNT_DD;
-    case CC_EXACT: return CNT_EXACT;
-    default: return is_seg ? CNT_EXAM_SEG : CNT_EXAM_BAD;
-  }
-}
 struct CavCounts {
-  unsigned c[CC_ALL];
-  // sums: CC_N ints of the wave's LDS, free by now
-  __device__ void flush(unsigned long long *cnt, bool is_seg, unsigned *sums) {
-    const int lane = threadIdx.x & 63;
-    if (lane < CC_N) sums[lane] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < CC_N; k++)
-      if (c[k]) atomicAdd(&sums[k], c[k]);
-    __syncthreads();
-    if (lane < CC_N && sums[lane])
-      atomicAdd(&cnt[cc_counter(lane, is_seg)], (unsigned long long)sums[lane]);
+  PredStats signs;
+  unsigned exam;   // triangle records examined
+  unsigned *cnt;   // LDS, CNT_N counters
+  unsigned *slow;  // LDS, deferred candidates (ps.cnt counts them too)
+  __device__ CavCounts(unsigned *c, unsigned *s) : signs{0, 0, 0, 0}, exam(0), cnt(c), slow(s) {}
+  __device__ void event(int k) const { atomicAdd(&cnt[k], 1u); }
+  // the registers into the block's counters
+  __device__ void settle(bool is_seg) {
+    if (exam) atomicAdd(&cnt[is_seg ? CNT_EXAM_SEG : CNT_EXAM_BAD], exam);
+    if (signs.fp32_hits) atomicAdd(&cnt[CNT_FP32], signs.fp32_hits);
+    if (signs.fp64_hits) atomicAdd(&cnt[CNT_FP64], signs.fp64_hits);
+    if (signs.dd_hits) atomicAdd(&cnt[CNT_DD], signs.dd_hits);
+    if (signs.exact_calls) atomicAdd(&cnt[CNT_EXACT], signs.exact_calls);
+    exam = 0;
+    signs = PredStats{0, 0, 0, 0};
   }
 };
+// Block counters of a one-wave block: cleared, and added to the pass's.
+__device__ __forceinline__ void clear_block_counts(unsigned *cnt) {
+  if (threadIdx.x < CNT_N) cnt[threadIdx.x] = 0u;
+  __syncthreads();
+}
+__device__ __forceinline__ void add_block_counts(unsigned long long *dst, const unsigned *cnt) {
+  __syncthreads();
+  if (threadIdx.x < CNT_N && cnt[threadIdx.x])
+    atomicAdd(&dst[threadIdx.x], (unsigned long long)cnt[threadIdx.x]);
+}
 
-constexpr int BIG_LDS_BYTES = 160 * 1024;
+// dynamic LDS of a cavity block; the rest of 160 KiB holds its counters
+constexpr int BIG_LDS_BYTES = 160 * 1024 - 256;
 // Largest grid of the exact-predicate cavity kernel (wave64 blocks); its
 // arena holds GCDT_INCIRCLE_WS doubles per lane: 512 x 64 x 8 KiB = 256 MiB.
 constexpr int EXACT_GRID = 512;
@@ -525,23 +522,28 @@ constexpr int EXACT_GRID = 512;
 // Candidate evaluation: a wave64 evaluates 64/LG candidates at once, one per
 // group of LG lanes.
 //
-// The lanes of a group compute the Steiner / split point and the walk (same
-// loads, broadcast); the Bowyer-Watson cavity is then grown level by level,
-// the group's lanes testing the three edges of every frontier triangle in
-// parallel.  Membership is an LDS hash set (atomicCAS insert), the cavity
-// list an LDS array appended with atomicAdd and finally sorted, so the
-// result is the cavity *set* in ascending triangle order -- independent of
-// timing and of LG.  The boundary / disk / orientation checks, the ring and
-// the encroachment test run lane-parallel over the cavity's edges.  Loops
-// that contain a barrier run a wave-uniform number of times (groups with
-// nothing to do idle through them), so every barrier is reached by the whole
-// block.  Several candidates per wave keep several dependent-load chains in
-// flight per wave: the kernel is bound by memory latency, not bandwidth.
+// The point and the triangle it lies in (locate) come from a lane per
+// candidate where that pays, else from the group's lanes together (same
+// loads, broadcast).  The Bowyer-Watson cavity is a closure over a work list:
+// the three edges of every cavity triangle, LG of them tested at a time; a
+// triangle found inside adds its edges, read with the record just tested.
+// Membership is an LDS hash set (atomicCAS insert) and the cavity list an LDS
+// array appended with atomicAdd, written out in ascending triangle order, so
+// the result is the cavity *set* -- independent of timing and of LG.  The
+// boundary / disk / orientation checks, the ring and the encroachment test
+// run lane-parallel over the cavity's edges.  Loops that contain a barrier or
+// a ballot run a group-uniform number of times.  Large passes are bound by
+// instruction issue (an evaluation is a few thousand wave instructions, and 5
+// waves per SIMD hide most of the gathers), small ones by the length of the
+// chain of gathers and LDS round trips; both want fewer, wider steps.
+// On 10^6 points the work list, the lane-per-candidate location and the star
+// order by pointer doubling took bad cavities from 63.4 to 48.3 ms and segment
+// cavities from 23.1 to 17.2 ms (three refinements, small passes left out).
 // The boundary edges are also linked into the star's cyclic order here (the
 // successor of edge u->v is the boundary edge leaving v) and written to the
 // candidate's workspace, so the apply kernel only scatters records.
-// LDS per group: list (2K+2) | cavity hash (HC) | ring hash (HR) | 8 scalars |
-// boundary edges 6 x (K+2).
+// LDS per group: cavity hash (HC) | ring hash (HR) | list (2K+2) | 8 scalars |
+// boundary edges 6 x (K+2), before them the cavity triangles' edges (3K).
 // ---------------------------------------------------------------------------
 __host__ __device__ inline int pow2_at_least(int x) {
   int p = 1;
@@ -552,10 +554,11 @@ __host__ __device__ inline int pow2_at_least(int x) {
 __host__ __device__ inline int cav_hash_cap(int K, int LG) { return pow2_at_least(2 * (K + LG)); }
 // Ring inserts come from boundary edges only: at most 3K of them.
 __host__ __device__ inline int ring_hash_cap(int K) { return pow2_at_least(3 * K + 8); }
-// list | cavity hash | ring hash | 8 scalars | boundary edges (origin,
-// destination, outer otri, subsegment, successor, star order) x (K+2)
+// cavity hash | ring hash | list | 8 scalars | boundary edges (origin,
+// destination, outer otri, subsegment, successor, star order) x (K+2); a
+// multiple of 4 (the hashes are cleared 16 bytes at a time)
 __host__ __device__ inline int group_lds_ints(int K, int LG) {
-  return (2 * K + 2) + cav_hash_cap(K, LG) + ring_hash_cap(K) + 8 + 6 * (K + 2);
+  return (cav_hash_cap(K, LG) + ring_hash_cap(K) + (2 * K + 2) + 8 + 6 * (K + 2) + 3) & ~3;
 }
 
 __device__ __forceinline__ unsigned hmix(int x) {
@@ -582,7 +585,15 @@ __device__ __forceinline__ bool hset_has(const int *h, int H, int x) {
   }
 }
 
-enum { SC_N = 0, SC_R, SC_OVF, SC_GIVEUP, SC_NBND, SC_ENC, SC_DSEG, SC_SLOW };
+// The group's part of a wave ballot (groups of G lanes, aligned).
+template <int G>
+__device__ __forceinline__ unsigned long long group_bits(unsigned long long b) {
+  static_assert(G >= 1 && G <= 64 && (G & (G - 1)) == 0, "power-of-two groups");
+  const int base = (threadIdx.x & 63) & ~(G - 1);
+  return G == 64 ? b : (b >> base) & ((1ull << (G == 64 ? 0 : G)) - 1ull);
+}
+
+enum { SC_N = 0, SC_OVF, SC_DSEG, SC_SLOW };
 constexpr int ST_NONE = -1;  // lane group without a candidate
 constexpr int ST_DEFER = 7;  // not evaluated this pass (vertex deletion)
 // vertex deletion (below): largest star, subsegment candidates per pass
@@ -594,6 +605,154 @@ constexpr int DEL_WS = 4 * DEL_MAX + 3 * (DEL_MAX - 2);
 constexpr int ST_SLOW = 6;   // deferred: an undecided sign, or a cavity beyond
                              // the fast kernel's LDS capacity
 
+// A candidate's point and the triangles its cavity grows from.
+struct Located {
+  int status, prio, seed0, seed1;
+  double cx, cy;
+  double near2;  // a cavity vertex closer than this coincides with the point
+};
+
+// The Steiner or split point of candidate id and where it lies.  Every lane
+// that evaluates the candidate calls it; `lead` (one of them) marks and
+// counts.  FAST: ST_SLOW when the filters leave a sign undecided.
+template <bool IS_SEG, bool FAST, class Trace>
+__device__ __forceinline__ Located locate(const MeshD &m, const ParamsD &pr, int id, bool lead,
+                                          CavCounts &cc, PredStats &cst, const Trace &trace) {
+  Located q{ST_VALID, 0, -1, -1, 0.0, 0.0, 0.0};
+  if (IS_SEG) {
+    int t1, j1, t2, j2;
+    seg_sides(m, id, t1, j1, t2, j2);
+    if (lead) cc.exam += (t1 >= 0) + (t2 >= 0);
+    if (!split_point(m, id, q.cx, q.cy)) {
+      q.status = ST_GIVEUP;
+    } else {
+      q.seed0 = t1 >= 0 ? t1 : t2;
+      q.seed1 = t1 >= 0 ? t2 : -1;
+    }
+    return q;
+  }
+  // skipped this pass: a bad triangle whose slot the deletion step rewrote
+  if ((m.tflag[id] & (TF_ALIVE | TF_BAD)) != (TF_ALIVE | TF_BAD)) {
+    q.status = ST_DEFER;
+    return q;
+  }
+  const ParamsD lp = params_at(pr, m, id);
+  const TriRec &r0 = m.T[id];
+  const double sh2 = shortest_edge_sq(r0);
+  q.near2 = 1e-12 * sh2;
+  if (pr.priority == 1 || pr.priority == 2) q.prio = edge_bucket(sh2);
+  const int sp = steiner_point<FAST>(lp, r0, q.cx, q.cy);
+  if (sp == STEINER_DEFER) {
+    q.status = ST_SLOW;
+  } else if (!sp) {
+    q.status = ST_GIVEUP;
+  } else {
+    int tl = -1, jl = -1, sg = -1;
+    // the walk's signs are counted once per candidate
+    PredStats wst = {0, 0, 0, 0};
+    int wsteps = 0;
+    const int w = walk<FAST>(m, id, q.cx, q.cy, pr.use_fp32 != 0, &wst, tl, jl, sg, wsteps);
+    if (lead) {
+      cc.exam += (unsigned)wsteps;  // the first step reads the bad triangle
+      cst.fp32_hits += wst.fp32_hits;
+      cst.fp64_hits += wst.fp64_hits;
+      cst.dd_hits += wst.dd_hits;
+      cst.exact_calls += wst.exact_calls;
+    }
+    // Blocked by a subsegment: mark it, or give the triangle up when the
+    // subsegment was given up (it is never split, so neither is the
+    // triangle).  senc only turns 2 in segment launches, so the lanes of a
+    // candidate read the same value.
+    int blk = -1;
+    if (w == 5) {
+      q.status = ST_SLOW;
+    } else if (w == 3) {
+      blk = sg;
+    } else if (w == 2 || w == 4) {
+      q.status = ST_GIVEUP;
+    } else {
+      q.seed0 = tl;
+      if (w == 1) {
+        const int sj = comp(m.T[tl].S, jl);
+        if (sj >= 0) {
+          blk = sj;
+        } else {
+          const int nb = comp(m.T[tl].N, jl);
+          if (nb < 0) q.status = ST_GIVEUP;
+          else q.seed1 = nb >> 2;
+        }
+      }
+    }
+    if (blk >= 0) {
+      if (m.senc[blk] == 2) {
+        q.status = ST_GIVEUP;
+      } else {
+        q.status = ST_REJ_BLOCKED;
+        if (lead && mark_enc_local(m, blk)) {
+          cc.event(CNT_MARKS);
+          trace.encroached(blk);
+        }
+      }
+    }
+  }
+  return q;
+}
+
+// One lane: candidate i (of subsegment or triangle id) is evaluated.
+template <bool IS_SEG>
+__device__ __forceinline__ void finish_candidate(const MeshD &m, const PassD &ps, int i, int id,
+                                                 int status, double cx, double cy, int n, int r,
+                                                 int prio, CavCounts &cc) {
+  ps.cstatus[i] = status;
+  ps.cpt[i] = make_double2(cx, cy);
+  ps.cn[i] = status == ST_VALID ? n : 0;
+  ps.cr[i] = status == ST_VALID ? r : 0;
+  ps.cprio[i] = prio;
+  if (status == ST_VALID) cc.event(CNT_VALID);
+  else if (status == ST_OVERFLOW) cc.event(CNT_OVERFLOW);
+  else if (status == ST_REJ_ENC) cc.event(CNT_REJ_ENC);
+  else if (status == ST_REJ_BLOCKED) cc.event(CNT_REJ_BLOCKED);
+  else if (status == ST_GIVEUP) {
+    cc.event(CNT_GIVEUPS);
+    if (IS_SEG) m.senc[id] = 2;
+    else m.tflag[id] |= TF_GIVEUP;
+  }
+}
+__device__ __forceinline__ void add_signs(CavCounts &cc, const PredStats &q) {
+  cc.signs.fp32_hits += q.fp32_hits;
+  cc.signs.fp64_hits += q.fp64_hits;
+  cc.signs.dd_hits += q.dd_hits;
+  cc.signs.exact_calls += q.exact_calls;
+}
+
+// One lane locates candidate i; a candidate that gets no cavity is finished
+// here (or deferred to the exact kernel), the others are left as ST_VALID
+// with their point and seeds for cavity_wave<.., LOCATED>.
+template <bool IS_SEG, class Trace>
+__device__ __forceinline__ void locate_one(const MeshD &m, const ParamsD &pr, const PassD &ps,
+                                           int i, int id, CavCounts &cc, const Trace &trace) {
+  PredStats cst = {0, 0, 0, 0};
+  const Located q = locate<IS_SEG, true>(m, pr, id, true, cc, cst, trace);
+  if (q.status == ST_VALID) {
+    ps.cstatus[i] = ST_VALID;
+    ps.cpt[i] = make_double2(q.cx, q.cy);
+    ps.cprio[i] = q.prio;
+    ps.cseed[i] = make_int2(q.seed0, q.seed1);
+    ps.cnear[i] = q.near2;
+    ps.cn[i] = (int)cst.fp32_hits;  // counted with the cavity's, unless deferred
+    ps.cr[i] = (int)cst.fp64_hits;
+  } else if (q.status == ST_SLOW) {
+    ps.cstatus[i] = ST_SLOW;
+    ps.slow[atomicAdd(&ps.cnt[CNT_SLOW], 1ull)] = i;
+    atomicAdd(cc.slow, 1u);
+  } else {
+    add_signs(cc, cst);
+    finish_candidate<IS_SEG>(m, ps, i, id, q.status, q.cx, q.cy, 0, 0, q.prio, cc);
+    if (!IS_SEG && ps.feat)
+      for (int f = 0; f < FEAT; f++) ps.feat[(size_t)i * FEAT + f] = 0.f;
+  }
+}
+
 // FAST: every candidate of the pass, with the FP32 / FP64 filters only and
 // LDS sized for cavities of at most Kf = min(K, ps.Kf) triangles; a candidate
 // that meets an undecided sign or a larger cavity is abandoned without side
@@ -601,24 +760,29 @@ constexpr int ST_SLOW = 6;   // deferred: an undecided sign, or a cavity beyond
 // the full cascade (double-double, then exact expansions in the per-lane
 // arena) and LDS for K triangles.  Neither the rare stages' registers nor the
 // largest cavities' LDS thus limit the occupancy of the hot kernel.
-// One wave of the evaluation, number wv of nwv, with sm its LDS.
-template <bool IS_SEG, int LG, bool FAST, class Trace>
+// LOCATED: locate_one ran for every candidate.  One wave of the evaluation,
+// number wv of nwv, with sm its LDS.
+template <bool IS_SEG, int LG, bool FAST, bool LOCATED, class Trace>
 __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, const PassD &ps,
                                             int Kmax, int wv, int nwv, int *sm, CavCounts &cc,
                                             const Trace &trace) {
   static_assert(LG >= 8 && 64 % LG == 0, "lane groups of 8..64 lanes");
+  static_assert(FAST || !LOCATED, "the exact kernel locates its candidates itself");
   constexpr int NG = 64 / LG;
   // K: the cavity capacity this kernel handles (LDS layout); ps.K: the
   // pass's capacity (workspace layout, overflow rule)
   const int K = FAST ? min(ps.K, ps.Kf) : ps.K;
   const int HC = cav_hash_cap(K, LG), HR = ring_hash_cap(K);
   const int lane = threadIdx.x & 63, grp = lane / LG, gl = lane % LG;
-  int *L = sm + grp * group_lds_ints(K, LG);
-  int *hc = L + (2 * K + 2);
+  const unsigned long long below = (1ull << gl) - 1ull;  // lower lanes of the group
+  int *hc = sm + grp * group_lds_ints(K, LG);
   int *hr = hc + HC;
-  int *sc = hr + HR;
+  int *L = hr + HR;
+  int *sc = L + (2 * K + 2);
   int *eu = sc + 8, *ev = eu + (K + 2), *eo = ev + (K + 2), *es = eo + (K + 2);
   int *esucc = es + (K + 2), *eord = esucc + (K + 2);
+  int *adj = eu;  // while the cavity grows: entry 3p + j, the otri across edge
+                  // j of cavity triangle p (-1: hull or subsegment)
   const bool fp32 = pr.use_fp32 != 0;
   // the exact stages' arena: only the exact kernel (whose grid the arena
   // covers) uses it
@@ -643,6 +807,12 @@ __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, c
     if (sg == PRED_UNSURE) { unsure = true; sg = 0; }
     return sg;
   };
+  // edges of cavity triangle t, list entry p
+  auto put_adj = [&](int p, const int4 &N, const int4 &S) {
+    adj[3 * p] = S.x >= 0 ? -1 : N.x;  // subsegments are never crossed
+    adj[3 * p + 1] = S.y >= 0 ? -1 : N.y;
+    adj[3 * p + 2] = S.z >= 0 ? -1 : N.z;
+  };
   for (int base = wv * NG; base < nwork; base += nwv * NG) {
     bool act = base + grp < nwork;
     int i = nc;
@@ -653,156 +823,105 @@ __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, c
         i = nc;
       }
     }
-    PredStats cst = {0, 0, 0, 0};  // this candidate's predicate counts
+    // empty sets
+    const int4 none = make_int4(-1, -1, -1, -1);
+    for (int k = gl; k < (HC + HR) / 4; k += LG) reinterpret_cast<int4 *>(hc)[k] = none;
+    if (gl < 8) sc[gl] = gl == SC_DSEG ? 0x7f7fffff : 0;  // +FLT_MAX bits: no subsegment yet
     // ---- point + seeds (uniform across the group) ----
-    int status = act ? ST_VALID : ST_NONE, prio = 0, seed0 = -1, seed1 = -1, split_s = -1,
-        t0 = -1;
-    double cx = 0.0, cy = 0.0;
-    double near2 = 0.0;  // a cavity vertex closer than this coincides with the point
-    ParamsD lp = pr;
+    PredStats cst = {0, 0, 0, 0};  // this candidate's predicate counts
+    const int id = act ? ids[i] : -1;
+    const int split_s = IS_SEG ? id : -1;
+    Located loc{ST_NONE, 0, -1, -1, 0.0, 0.0, 0.0};
     if (act) {
-      // skipped this pass: a bad triangle whose slot the deletion step
-      // rewrote
-      if (!IS_SEG && (m.tflag[ids[i]] & (TF_ALIVE | TF_BAD)) != (TF_ALIVE | TF_BAD)) {
-        status = ST_DEFER;
-      } else if (IS_SEG) {
-        split_s = ids[i];
-        int t1, j1, t2, j2;
-        seg_sides(m, split_s, t1, j1, t2, j2);
-        if (gl == 0) cc.c[CC_EXAM] += (t1 >= 0) + (t2 >= 0);
-        lp = params_at(pr, m, t1 >= 0 ? t1 : t2);
-        if (!split_point(m, split_s, cx, cy)) {
-          status = ST_GIVEUP;
+      if (LOCATED) {
+        loc.status = ps.cstatus[i];
+        if (loc.status == ST_VALID) {
+          const double2 c = ps.cpt[i];
+          const int2 sd = ps.cseed[i];
+          loc.cx = c.x;
+          loc.cy = c.y;
+          loc.seed0 = sd.x;
+          loc.seed1 = sd.y;
+          loc.prio = ps.cprio[i];
+          loc.near2 = ps.cnear[i];
+          if (gl == 0) {
+            cst.fp32_hits = (unsigned)ps.cn[i];
+            cst.fp64_hits = (unsigned)ps.cr[i];
+          }
         } else {
-          seed0 = t1 >= 0 ? t1 : t2;
-          seed1 = t1 >= 0 ? t2 : -1;
+          act = false;  // finished or deferred by locate_one
+          loc.status = ST_NONE;
         }
       } else {
-        t0 = ids[i];
-        lp = params_at(pr, m, t0);
-        const TriRec &r0 = m.T[t0];
-        const double sh2 = shortest_edge_sq(r0);
-        near2 = 1e-12 * sh2;
-        if (pr.priority == 1 || pr.priority == 2) prio = edge_bucket(sh2);
-        const int sp = steiner_point<FAST>(lp, r0, cx, cy);
-        if (sp == STEINER_DEFER) {
-          status = ST_SLOW;
-        } else if (!sp) {
-          status = ST_GIVEUP;
-        } else {
-          int tl = -1, jl = -1, sg = -1;
-          // the walk's signs are counted once per group (every lane walks)
-          PredStats wst = {0, 0, 0, 0};
-          int wsteps = 0;
-          int w = walk<FAST>(m, t0, cx, cy, fp32, &wst, tl, jl, sg, wsteps);
-          if (gl == 0) {
-            cc.c[CC_EXAM] += (unsigned)wsteps;  // the first step reads the bad triangle
-            cst.fp32_hits += wst.fp32_hits;
-            cst.fp64_hits += wst.fp64_hits;
-            cst.dd_hits += wst.dd_hits;
-            cst.exact_calls += wst.exact_calls;
-          }
-          // Blocked by a subsegment: mark it, or give the triangle up when
-          // the subsegment was given up (it is never split, so neither is
-          // the triangle).  senc only turns 2 in segment launches, so the
-          // group's lanes read the same value.
-          if (w == 5) {
-            status = ST_SLOW;
-          } else if (w == 3) {
-            if (m.senc[sg] == 2) {
-              status = ST_GIVEUP;
-            } else {
-              status = ST_REJ_BLOCKED;
-              if (gl == 0 && mark_enc_local(m, sg)) {
-                cc.c[CC_MARKS]++;
-                trace.encroached(sg);
-              }
-            }
-          } else if (w == 2 || w == 4) {
-            status = ST_GIVEUP;
-          } else {
-            seed0 = tl;
-            if (w == 1) {
-              int s = comp(m.T[tl].S, jl);
-              if (s >= 0 && m.senc[s] == 2) {
-                status = ST_GIVEUP;
-              } else if (s >= 0) {
-                status = ST_REJ_BLOCKED;
-                if (gl == 0 && mark_enc_local(m, s)) {
-                  cc.c[CC_MARKS]++;
-                  trace.encroached(s);
-                }
-              } else {
-                int nb = comp(m.T[tl].N, jl);
-                if (nb < 0) status = ST_GIVEUP;
-                else seed1 = nb >> 2;
-              }
-            }
-          }
-        }
+        loc = locate<IS_SEG, FAST>(m, pr, id, gl == 0, cc, cst, trace);
       }
     }
-    // ---- breadth-first growth of the cavity ----
+    int status = loc.status;
+    const double cx = loc.cx, cy = loc.cy;
     const bool grow = status == ST_VALID;
-    for (int k = gl; k < HC; k += LG) hc[k] = -1;
-    for (int k = gl; k < HR; k += LG) hr[k] = -1;
-    if (gl < 8) sc[gl] = 0;
-    if (gl == 0) sc[SC_DSEG] = 0x7f7fffff;  // +FLT_MAX bits: no subsegment yet
+    const ParamsD lp = grow ? params_at(pr, m, loc.seed0) : pr;
     wave_sync();
-    if (grow && gl == 0) {
-      L[0] = seed0;
-      hset_insert(hc, HC, seed0);
-      int c0 = 1;
-      if (seed1 >= 0) {
-        L[1] = seed1;
-        hset_insert(hc, HC, seed1);
-        c0 = 2;
-      }
-      sc[SC_N] = c0;
+    // ---- closure: the cavity ----
+    if (grow && gl < (loc.seed1 >= 0 ? 2 : 1)) {
+      const int t = gl == 0 ? loc.seed0 : loc.seed1;
+      L[gl] = t;
+      hset_insert(hc, HC, t);
+      put_adj(gl, m.T[t].N, m.T[t].S);
+      if (gl == 0) sc[SC_N] = loc.seed1 >= 0 ? 2 : 1;
     }
     wave_sync();
-    int fb = 0;
-    for (;;) {
-      int fe = sc[SC_N];
-      int ovf = sc[SC_OVF] | sc[SC_SLOW];
-      bool more = grow && !ovf && fb < fe;
+    for (int q0 = 0;;) {  // q0: edges tested
+      const int fe = sc[SC_N], stop = sc[SC_OVF] | sc[SC_SLOW];
+      const bool more = grow && !stop && q0 < 3 * fe;
       wave_sync();
       if (__ballot(more) == 0ull) break;  // wave-uniform exit
       if (more) {
-        int items = (fe - fb) * 3;
-        for (int it = gl; it < items; it += LG) {
-          int t = L[fb + it / 3], j = it % 3;
-          if (comp(m.T[t].S, j) >= 0) continue;  // subsegments are never crossed
-          int nb = comp(m.T[t].N, j);
-          if (nb < 0) continue;
-          int u = nb >> 2;
-          if (hset_has(hc, HC, u)) continue;
+        const int it = q0 + gl;
+        const int nb = it < 3 * fe ? adj[it] : -1;
+        if (nb >= 0) {
+          const int u = nb >> 2;
           const TriRec &ru = m.T[u];
-          double2 a = ru.X[0], b = ru.X[1], c = ru.X[2];
-          cc.c[CC_EXAM]++;
-          int ins = in_circle(a, b, c, cx, cy, &cst);
-          if (FAST && unsure) {
-            sc[SC_SLOW] = 1;
-            unsure = false;
-            continue;
-          }
-          if (ins > 0) {
-            // u is in the cavity.  Once K triangles are in, a triangle that is
-            // still absent proves the cavity larger than K; inserts stay
-            // below K + LG, so the hash set never fills.
-            if (hset_has(hc, HC, u)) continue;
-            if (sc[SC_N] >= K) {
-              sc[SC_OVF] = 1;
-            } else if (hset_insert(hc, HC, u)) {
-              int pos = atomicAdd(&sc[SC_N], 1);
-              if (pos < K) L[pos] = u;
-              else sc[SC_OVF] = 1;
+          const double2 a = ru.X[0], b = ru.X[1], c = ru.X[2];
+          const int4 uN = ru.N, uS = ru.S;
+          const int a0 = uS.x >= 0 ? -1 : uN.x, a1 = uS.y >= 0 ? -1 : uN.y,
+                    a2 = uS.z >= 0 ? -1 : uN.z;
+          if (!hset_has(hc, HC, u)) {
+            cc.exam++;
+            const int ins = in_circle(a, b, c, cx, cy, &cst);
+            if (FAST && unsure) {
+              sc[SC_SLOW] = 1;
+              unsure = false;
+            } else if (ins > 0) {
+              // u is in the cavity.  Once K triangles are in, a triangle that
+              // is still absent proves the cavity larger than K; inserts stay
+              // below K + LG, so the hash set never fills.  The check is
+              // needed only where this step's inserts could pass K.
+              bool add = true;
+              if (fe + LG > K) {
+                if (hset_has(hc, HC, u)) {
+                  add = false;
+                } else if (sc[SC_N] >= K) {
+                  sc[SC_OVF] = 1;
+                  add = false;
+                }
+              }
+              if (add && hset_insert(hc, HC, u)) {
+                const int pos = atomicAdd(&sc[SC_N], 1);
+                if (pos < K) {
+                  L[pos] = u;
+                  adj[3 * pos] = a0;
+                  adj[3 * pos + 1] = a1;
+                  adj[3 * pos + 2] = a2;
+                } else {
+                  sc[SC_OVF] = 1;
+                }
+              }
             }
           }
         }
+        q0 = min(q0 + LG, 3 * fe);
       }
       wave_sync();
-      if (more) fb = fe;
     }
     int n = 0, r = 0;
     bool cav_ok = false;
@@ -813,74 +932,83 @@ __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, c
       else if (sc[SC_OVF] || n > K) status = (K >= Kmax) ? ST_GIVEUP : ST_OVERFLOW;
       else cav_ok = true;
     }
-    // ---- sort the cavity (rank sort into the free half of L) ----
-    int *tmp = L + K + 2;
-    if (cav_ok)
-      for (int e = gl; e < n; e += LG) {
-        int v = L[e], rank = 0;
-        for (int x = 0; x < n; x++) rank += L[x] < v;
-        tmp[rank] = v;
-      }
-    wave_sync();
-    if (cav_ok)
-      for (int e = gl; e < n; e += LG) L[e] = tmp[e];
-    wave_sync();
+    wave_sync();  // adj is rewritten as the boundary
     // ---- disk and star checks over every cavity edge ----
-    if (cav_ok)
-      for (int it = gl; it < 3 * n; it += LG) {
-        int t = L[it / 3], j = it % 3;
-        const TriRec &rt = m.T[t];
-        int s = comp(rt.S, j);
-        int nb = comp(rt.N, j);
-        bool inside = nb >= 0 && hset_has(hc, HC, nb >> 2);
-        if (s >= 0 && s != split_s && inside) sc[SC_GIVEUP] = 1;
-        bool bnd = (s >= 0 && s != split_s) || nb < 0 || !inside;
+    if (cav_ok) {
+      bool give = false, enc_any = false, slow = false;
+      int nbnd = 0;
+      for (int q = 0; q < 3 * n; q += LG) {
+        const int it = q + gl;
+        bool bnd = false, ring = false;
+        int t = -1, j = 0, s = -1, nb = -1;
+        if (it < 3 * n) {
+          t = L[it / 3];
+          j = it % 3;
+          const TriRec &rt = m.T[t];
+          s = (&rt.S.x)[j];
+          nb = (&rt.N.x)[j];
+        }
+        if (t >= 0) {
+          const bool inside = nb >= 0 && hset_has(hc, HC, nb >> 2);
+          const bool other = s >= 0 && s != split_s;  // a subsegment not being split
+          if (other && inside) give = true;
+          bnd = other || nb < 0 || !inside;
+          ring = nb >= 0 && !inside;
+        }
+        const unsigned long long bb = group_bits<LG>(__ballot(bnd));
+        const int bpos = nbnd + __popcll(bb & below);
+        nbnd += __popcll(bb);
+        const int j1 = j == 2 ? 0 : j + 1, j2 = j == 0 ? 2 : j - 1;
         if (bnd) {
-          int4 tv = rt.V;
+          const TriRec &rt = m.T[t];
+          const double2 u = rt.X[j1], v = rt.X[j2];
           if (!IS_SEG) {
             // Steiner point on an existing vertex up to rounding: give up
             // (in exact arithmetic the empty circumcircle keeps every vertex
             // at least half the shortest edge away)
-            double2 q = rt.X[(j + 1) % 3];
-            double dx = cx - q.x, dy = cy - q.y;
-            if (dx * dx + dy * dy < near2) sc[SC_GIVEUP] = 1;
+            const double dx = cx - u.x, dy = cy - u.y;
+            if (dx * dx + dy * dy < loc.near2) give = true;
           }
-          int bpos = atomicAdd(&sc[SC_NBND], 1);
           if (bpos < K + 2) {
-            eu[bpos] = comp(tv, (j + 1) % 3);
-            ev[bpos] = comp(tv, (j + 2) % 3);
+            eu[bpos] = (&rt.V.x)[j1];
+            ev[bpos] = (&rt.V.x)[j2];
             eo[bpos] = nb;
             es[bpos] = s;
           }
           if (!(s >= 0 && s == split_s)) {
-            double2 u = rt.X[(j + 1) % 3], v = rt.X[(j + 2) % 3];
-            int o = orient(cx, cy, u, v, &cst);
+            const int o = orient(cx, cy, u, v, &cst);
             if (FAST && unsure) {
-              sc[SC_SLOW] = 1;
+              slow = true;
               unsure = false;
             } else if (o <= 0) {
-              sc[SC_GIVEUP] = 1;
+              give = true;
             }
           }
-          if (nb >= 0 && !inside && hset_insert(hr, HR, nb >> 2)) {
-            int pos = atomicAdd(&sc[SC_R], 1);
-            if (pos < K + 2) L[n + pos] = nb >> 2;
-          }
+          ring = ring && hset_insert(hr, HR, nb >> 2);
+        } else {
+          ring = false;
         }
+        const unsigned long long rb = group_bits<LG>(__ballot(ring));
+        if (ring) {
+          const int pos = r + __popcll(rb & below);
+          if (pos < K + 2) L[n + pos] = nb >> 2;
+        }
+        r += __popcll(rb);
         if (!IS_SEG && s >= 0) {
+          const TriRec &rt = m.T[t];
           // The subsegment is this edge.  Ruppert's test (dot < 0) is exactly
           // symmetric in the endpoints, so the record's coordinates serve;
           // Chew's lens product is not, so it takes the subsegment's order.
           double2 A, B;
           if (lp.ruppert) {
-            A = rt.X[(j + 1) % 3];
-            B = rt.X[(j + 2) % 3];
+            A = rt.X[j1];
+            B = rt.X[j2];
           } else {
             const int2 sv = m.SV[s];
             A = m.P[sv.x];
             B = m.P[sv.y];
           }
-          if (encroaches_xy(lp, A, B, cx, cy)) sc[SC_ENC] = 1;
+          if (encroaches_xy(lp, A, B, cx, cy)) enc_any = true;
           if (ps.feat) {  // distance of the Steiner point to this subsegment
             float ex = (float)(B.x - A.x), ey = (float)(B.y - A.y);
             float px = (float)(cx - A.x), py = (float)(cy - A.y);
@@ -891,14 +1019,11 @@ __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, c
           }
         }
       }
-    wave_sync();
-    if (cav_ok) {
-      r = sc[SC_R];
-      if (FAST && sc[SC_SLOW]) {
+      if (group_bits<LG>(__ballot(slow)) != 0ull && FAST) {
         status = ST_SLOW;
-      } else if (sc[SC_GIVEUP] || sc[SC_NBND] != n + 2 || r > n + 2) {
+      } else if (group_bits<LG>(__ballot(give)) != 0ull || nbnd != n + 2 || r > n + 2) {
         status = ST_GIVEUP;
-      } else if (!IS_SEG && sc[SC_ENC]) {
+      } else if (!IS_SEG && group_bits<LG>(__ballot(enc_any)) != 0ull) {
         // Ruppert/Chew rule: a Steiner point that encroaches a subsegment on
         // its cavity boundary is not inserted; every such subsegment is
         // marked.  When every subsegment it encroaches was given up, the
@@ -919,83 +1044,124 @@ __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, c
           if (enc) {
             live |= m.senc[s] != 2;
             if (mark_enc_local(m, s)) {
-              cc.c[CC_MARKS]++;
+              cc.event(CNT_MARKS);
               trace.encroached(s);
             }
           }
         }
         // every lane of this group is here (the branch is group-uniform)
-        const unsigned long long gmask = LG == 64 ? ~0ull : ((1ull << (LG % 64)) - 1ull);
-        const bool any_live = ((__ballot(live) >> (grp * LG)) & gmask) != 0ull;
-        status = any_live ? ST_REJ_ENC : ST_GIVEUP;
+        status = group_bits<LG>(__ballot(live)) != 0ull ? ST_REJ_ENC : ST_GIVEUP;
       }
     }
+    wave_sync();
     // ---- star order of the boundary (valid candidates) ----
     // The n+2 boundary edges form one cycle.  Closed star: it starts at the
     // edge with the smallest origin vertex; a hull subsegment split (open
     // star) starts after the split edge and leaves it out.
     const bool star = status == ST_VALID;
     const int nbe = n + 2;
-    if (star)
-      for (int e = gl; e < nbe; e += LG) {
-        int v = ev[e], f = 0;
-        while (f < nbe && eu[f] != v) f++;
-        esucc[e] = f < nbe ? f : 0;
+    int *G = ps.ws + (size_t)i * ps.R + (2 * ps.K + 2);
+    if (star && nbe <= LG) {
+      // one edge per lane: its distance along the cycle to the start by
+      // pointer doubling, no serial chase
+      const int e = gl < nbe ? gl : 0;
+      const int U = eu[e], V = ev[e], O = eo[e], S = es[e];
+      int succ = 0, start = 0, umin = INT_MAX;
+      for (int f = 0; f < nbe; f++) {
+        const int x = eu[f];
+        if (x == V) succ = f;
+        if (x < umin) {
+          umin = x;
+          start = f;
+        }
       }
-    wave_sync();
-    int nstar = 0;
-    if (star) {
-      int start = 0;
       bool open = false;
-      for (int e = 0; e < nbe; e++) {
-        if (IS_SEG && es[e] == split_s) {  // only a hull split edge is on the boundary
-          open = true;
-          start = esucc[e];
-          break;
-        }
-        if (eu[e] < eu[start]) start = e;
+      if (IS_SEG) {  // only a hull split edge is on the boundary
+        const unsigned long long ob = group_bits<LG>(__ballot(gl < nbe && S == split_s));
+        open = ob != 0ull;
+        if (open) start = __shfl(succ, __builtin_ctzll(ob), LG);
       }
-      nstar = open ? nbe - 1 : nbe;
-      if (gl == 0) {
-        int e = start;
-        for (int q = 0; q < nstar; q++) {
-          eord[q] = e;
-          e = esucc[e];
+      int dist = 1, nxt = succ == start ? -1 : succ;
+      for (int step = 1; step < LG; step <<= 1) {
+        const int at = nxt < 0 ? 0 : nxt;
+        const int d2 = __shfl(dist, at, LG), n2 = __shfl(nxt, at, LG);
+        if (nxt >= 0) {
+          dist += d2;
+          nxt = n2;
         }
+      }
+      const int rank = nbe - dist;
+      if (gl < nbe && rank >= 0 && rank < (open ? nbe - 1 : nbe)) {
+        G[rank] = U;
+        G[(ps.K + 2) + rank] = V;
+        G[2 * (ps.K + 2) + rank] = O;
+        G[3 * (ps.K + 2) + rank] = S;
       }
     }
-    wave_sync();
+    const bool longstar = star && nbe > LG;
+    if (__ballot(longstar) != 0ull) {
+      if (longstar)
+        for (int e = gl; e < nbe; e += LG) {
+          int v = ev[e], f = 0;
+          while (f < nbe && eu[f] != v) f++;
+          esucc[e] = f < nbe ? f : 0;
+        }
+      wave_sync();
+      int nstar = 0;
+      if (longstar) {
+        int start = 0;
+        bool open = false;
+        for (int e = 0; e < nbe; e++) {
+          if (IS_SEG && es[e] == split_s) {
+            open = true;
+            start = esucc[e];
+            break;
+          }
+          if (eu[e] < eu[start]) start = e;
+        }
+        nstar = open ? nbe - 1 : nbe;
+        if (gl == 0) {
+          int e = start;
+          for (int q = 0; q < nstar; q++) {
+            eord[q] = e;
+            e = esucc[e];
+          }
+        }
+      }
+      wave_sync();
+      if (longstar)
+        for (int q = gl; q < nstar; q += LG) {
+          int e = eord[q];
+          G[q] = eu[e];
+          G[(ps.K + 2) + q] = ev[e];
+          G[2 * (ps.K + 2) + q] = eo[e];
+          G[3 * (ps.K + 2) + q] = es[e];
+        }
+    }
+    // ---- outputs: the cavity in ascending order, the ring ----
     if (star) {
-      int *G = ps.ws + (size_t)i * ps.R + (2 * ps.K + 2);
-      for (int q = gl; q < nstar; q += LG) {
-        int e = eord[q];
-        G[q] = eu[e];
-        G[(ps.K + 2) + q] = ev[e];
-        G[2 * (ps.K + 2) + q] = eo[e];
-        G[3 * (ps.K + 2) + q] = es[e];
+      int *W = ps.ws + (size_t)i * ps.R;
+      for (int e = gl; e < n; e += LG) {
+        const int v = L[e];
+        int rank = 0;
+        for (int x = 0; x < n; x++) rank += L[x] < v;
+        W[rank] = v;
       }
-    }
-    // ---- outputs ----
-    if (status == ST_VALID) {
-      int *G = ps.ws + (size_t)i * ps.R;
-      for (int q = gl; q < n + r; q += LG) G[q] = L[q];
+      for (int q = gl; q < r; q += LG) W[n + q] = L[n + q];
     }
     if (status == ST_SLOW) {  // defer: no output, no side effect, no counts
       if (gl == 0) {
         ps.slow[atomicAdd(&ps.cnt[CNT_SLOW], 1ull)] = i;
-        cc.c[CC_SLOW]++;
+        atomicAdd(cc.slow, 1u);
       }
     } else {
-      cc.c[CC_FP32] += (unsigned)cst.fp32_hits;
-      cc.c[CC_FP64] += (unsigned)cst.fp64_hits;
-      cc.c[CC_DD] += (unsigned)cst.dd_hits;
-      cc.c[CC_EXACT] += (unsigned)cst.exact_calls;
+      add_signs(cc, cst);
     }
     if (!IS_SEG && ps.feat && act && status != ST_SLOW) {
       // per-candidate features of the learned priority
       float l0 = 0.f, l1 = 0.f, l2 = 0.f, area2 = 0.f;
       if (status == ST_VALID) {
-        const TriRec &r0 = m.T[t0];
+        const TriRec &r0 = m.T[id];
         double2 A = r0.X[0], O = r0.X[1], D = r0.X[2];
         l0 = (float)((O.x - D.x) * (O.x - D.x) + (O.y - D.y) * (O.y - D.y));
         l1 = (float)((D.x - A.x) * (D.x - A.x) + (D.y - A.y) * (D.y - A.y));
@@ -1022,51 +1188,55 @@ __device__ __forceinline__ void cavity_wave(const MeshD &m, const ParamsD &pr, c
         ps.feat[(size_t)i * FEAT + f] = fv;
       }
     }
-    if (act && gl == 0 && status != ST_SLOW) {
-      ps.cstatus[i] = status;
-      ps.cpt[i] = make_double2(cx, cy);
-      ps.cn[i] = status == ST_VALID ? n : 0;
-      ps.cr[i] = status == ST_VALID ? r : 0;
-      ps.cprio[i] = prio;
-      if (status == ST_VALID) cc.c[CC_VALID]++;
-      else if (status == ST_OVERFLOW) cc.c[CC_OVERFLOW]++;
-      else if (status == ST_REJ_ENC) cc.c[CC_REJ_ENC]++;
-      else if (status == ST_REJ_BLOCKED) cc.c[CC_REJ_BLOCKED]++;
-      else if (status == ST_GIVEUP) {
-        cc.c[CC_GIVEUPS]++;
-        if (IS_SEG) m.senc[split_s] = 2;
-        else m.tflag[t0] |= TF_GIVEUP;
-      }
-    }
+    if (act && gl == 0 && status != ST_SLOW)
+      finish_candidate<IS_SEG>(m, ps, i, id, status, cx, cy, n, r, loc.prio, cc);
     wave_sync();  // LDS is reused by the next candidates
   }
 }
 
 // A kernel of one wave per block.
-template <bool IS_SEG, int LG, bool FAST>
+template <bool IS_SEG, int LG, bool FAST, bool LOCATED>
 __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr, const PassD &ps,
                                             int Kmax) {
-  extern __shared__ int sm[];
+  extern __shared__ __align__(16) int sm[];
   if (!FAST) {  // most passes defer nothing
     if (pass_nc(ps) <= 0 || ps.cnt[CNT_SLOW] == 0ull) return;
   }
-  CavCounts cc;
-  for (int k = 0; k < CC_ALL; k++) cc.c[k] = 0u;
-  cavity_wave<IS_SEG, LG, FAST>(m, pr, ps, Kmax, (int)blockIdx.x, (int)gridDim.x, sm, cc,
-                                NoTrace{});
-  cc.flush(ps.cnt, IS_SEG, (unsigned *)sm);
+  __shared__ unsigned s_cnt[CNT_N], s_slow;
+  clear_block_counts(s_cnt);
+  CavCounts cc(s_cnt, &s_slow);
+  cavity_wave<IS_SEG, LG, FAST, LOCATED>(m, pr, ps, Kmax, (int)blockIdx.x, (int)gridDim.x, sm, cc,
+                                         NoTrace{});
+  cc.settle(IS_SEG);
+  add_block_counts(ps.cnt, s_cnt);
 }
 
-// The filtered kernel is held to 5 waves per SIMD (<= 96 VGPRs, no spills);
-// the exact kernel runs on few candidates and keeps its full register file.
-template <bool IS_SEG, int LG>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5))) void k_cavity_fast(
+// The filtered kernel is held to 4 waves per SIMD (at most 128 VGPRs, no
+// spills; LDS allows 4.4): 10^6 points 100.6 ms a call, 102.2 with 5 waves and
+// spills.  The exact kernel runs on few candidates and keeps its full register
+// file.
+template <bool IS_SEG, int LG, bool LOCATED>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_cavity_fast(
     MeshD m, ParamsD pr, PassD ps, int Kmax) {
-  cavity_body<IS_SEG, LG, true>(m, pr, ps, Kmax);
+  cavity_body<IS_SEG, LG, true, LOCATED>(m, pr, ps, Kmax);
 }
 template <bool IS_SEG, int LG>
 __global__ __launch_bounds__(64) void k_cavity_slow(MeshD m, ParamsD pr, PassD ps, int Kmax) {
-  cavity_body<IS_SEG, LG, false>(m, pr, ps, Kmax);
+  cavity_body<IS_SEG, LG, false, false>(m, pr, ps, Kmax);
+}
+
+// A lane per candidate ahead of k_cavity_fast<.., LOCATED>.
+constexpr int LOC_BLOCK = 64;
+template <bool IS_SEG>
+__global__ __launch_bounds__(LOC_BLOCK) void k_locate(MeshD m, ParamsD pr, PassD ps) {
+  __shared__ unsigned s_cnt[CNT_N], s_slow;
+  clear_block_counts(s_cnt);
+  const int n = IS_SEG ? ps.nseg : ps.nc - ps.nseg;
+  const int w = blockIdx.x * LOC_BLOCK + threadIdx.x, i = IS_SEG ? w : ps.nseg + w;
+  CavCounts cc(s_cnt, &s_slow);
+  if (w < n) locate_one<IS_SEG>(m, pr, ps, i, ps.ids[i], cc, NoTrace{});
+  cc.settle(IS_SEG);
+  add_block_counts(ps.cnt, s_cnt);
 }
 
 // Claim key: higher wins.  Epoch in the top 11 bits makes older claims lose
@@ -1090,13 +1260,6 @@ constexpr int LIST_BLOCK = 256;
 static_assert(LIST_BLOCK == CB, "k_rank_apply ranks the winners with the compaction's tile");
 constexpr int CLAIM_LANES = 16;
 constexpr int APPLY_LANES = 4;
-
-template <int G>
-__device__ __forceinline__ unsigned long long group_bits(unsigned long long b) {
-  static_assert(G >= 1 && G <= 64 && (G & (G - 1)) == 0, "power-of-two groups");
-  const int base = (threadIdx.x & 63) & ~(G - 1);
-  return G == 64 ? b : (b >> base) & ((1ull << (G == 64 ? 0 : G)) - 1ull);
-}
 
 // Claim iteration ps.iter.  Iteration 0: every valid candidate claims its
 // cavity and ring.  Later iterations: a candidate still in play (cact) whose
@@ -1464,17 +1627,6 @@ struct ListTrace {
   __device__ void seg_winners(const PassD &, unsigned n) const { atomicAdd(&cnt[CNT_SEGWIN], n); }
 };
 
-// One pass's counts of this thread into the block's LDS counters; deferred
-// candidates to a counter of their kind (read by all between two barriers).
-__device__ __forceinline__ void add_counts(CavCounts &cc, bool is_seg, unsigned *cnt,
-                                           unsigned *slow) {
-#pragma unroll
-  for (int k = 0; k < CC_N; k++)
-    if (cc.c[k]) atomicAdd(&cnt[cc_counter(k, is_seg)], cc.c[k]);
-  if (cc.c[CC_SLOW]) atomicAdd(&slow[is_seg ? 0 : 1], cc.c[CC_SLOW]);
-  for (int k = 0; k < CC_ALL; k++) cc.c[k] = 0u;
-}
-
 // Ascending order of the n distinct values in src (LDS, n <= SR_THREADS), to
 // dst: each thread counts the smaller values.  The caller synchronises.
 __device__ __forceinline__ void rank_sort(const int *src, int n, int *dst) {
@@ -1492,6 +1644,8 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
   extern __shared__ __align__(16) int sm[];
   __shared__ int s_enc[SR_ENC], s_bad[SR_CAP], s_ids[SR_CAP];
   __shared__ double2 s_pt[SR_CAP];
+  __shared__ double s_near[SR_CAP];
+  __shared__ int2 s_seed[SR_CAP];
   __shared__ int s_status[SR_CAP], s_n[SR_CAP], s_r[SR_CAP], s_prio[SR_CAP], s_win[SR_CAP],
       s_rank[SR_CAP], s_act[SR_CAP];
   __shared__ unsigned s_cnt[CNT_N], s_slow[2];
@@ -1516,8 +1670,6 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
     s_slow[0] = s_slow[1] = 0u;
   }
   __syncthreads();
-  CavCounts cc;
-  for (int k = 0; k < CC_ALL; k++) cc.c[k] = 0u;
   for (; passes < SR_PASSES; passes++) {
     nseg = st.ne;
     int nbc = 0;
@@ -1582,6 +1734,8 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
     ps.cprio = s_prio;
     ps.cwin = s_win;
     ps.crank = s_rank;
+    ps.cseed = s_seed;
+    ps.cnear = s_near;
     ps.feat = nbc > 0 ? a.feat : nullptr;
     ps.pass_index = st.pass_index;
     const ListTrace trace{s_enc, &s_ne, a.dirty, &s_nd, s_cnt, st.nt, known};
@@ -1589,8 +1743,11 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
     // ---- cavities ----
     int *cav = sm + wave * (64 / SR_LG) * group_lds_ints(min(ps.K, ps.Kf), SR_LG);
     if (nseg > 0) {
-      cavity_wave<true, SR_LG, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
-      add_counts(cc, true, s_cnt, s_slow);
+      CavCounts cc(s_cnt, &s_slow[0]);
+      if (tid < nseg) locate_one<true>(m, pr, ps, tid, s_ids[tid], cc, trace);
+      __syncthreads();
+      cavity_wave<true, SR_LG, true, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
+      cc.settle(true);
       __syncthreads();
       if (s_slow[0] != 0u) {
         code = SR_SLOW;
@@ -1599,8 +1756,11 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
       }
     }
     if (nbc > 0) {
-      cavity_wave<false, SR_LG, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
-      add_counts(cc, false, s_cnt, s_slow);
+      CavCounts cc(s_cnt, &s_slow[1]);
+      if (tid < nbc) locate_one<false>(m, pr, ps, nseg + tid, s_ids[nseg + tid], cc, trace);
+      __syncthreads();
+      cavity_wave<false, SR_LG, true, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
+      cc.settle(false);
       __syncthreads();
       if (s_slow[1] != 0u) {
         code = SR_SLOW;
@@ -2516,6 +2676,12 @@ __global__ void k_dicut(const int *sel_tmp, Ctl *c) {
 // ===========================================================================
 // Host side
 // ===========================================================================
+// Dynamic LDS of k_small_rounds for cavities of up to K triangles.
+static size_t small_lds(int K) {
+  return std::max(sizeof(int) * (size_t)(SR_THREADS / SR_LG) * group_lds_ints(K, SR_LG),
+                  sizeof(MlpWeights) + sizeof(short) * SR_WAVES * 16 * H1_STRIDE);
+}
+
 static void hip_check(hipError_t e, const char *what) {
   if (e != hipSuccess)
     throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
@@ -2565,16 +2731,19 @@ Refiner::Refiner(const gcdt_options &o) : opt(o) {
   HC(hipEventCreate(&ev1));
   // cavity and apply kernels take up to BIG_LDS_BYTES of dynamic LDS
   const void *cav[] = {
-      (const void *)k_cavity_fast<true, 8>,  (const void *)k_cavity_fast<false, 8>,
-      (const void *)k_cavity_fast<true, 16>, (const void *)k_cavity_fast<false, 16>,
-      (const void *)k_cavity_fast<true, 32>, (const void *)k_cavity_fast<false, 32>,
-      (const void *)k_cavity_fast<true, 64>, (const void *)k_cavity_fast<false, 64>,
-      (const void *)k_cavity_slow<true, 8>,  (const void *)k_cavity_slow<false, 8>,
-      (const void *)k_cavity_slow<true, 16>, (const void *)k_cavity_slow<false, 16>,
-      (const void *)k_cavity_slow<true, 32>, (const void *)k_cavity_slow<false, 32>,
-      (const void *)k_cavity_slow<true, 64>, (const void *)k_cavity_slow<false, 64>};
+      (const void *)k_cavity_fast<true, 8, false>,  (const void *)k_cavity_fast<false, 8, false>,
+      (const void *)k_cavity_fast<true, 16, false>, (const void *)k_cavity_fast<false, 16, false>,
+      (const void *)k_cavity_fast<true, 32, false>, (const void *)k_cavity_fast<false, 32, false>,
+      (const void *)k_cavity_fast<true, 64, false>, (const void *)k_cavity_fast<false, 64, false>,
+      (const void *)k_cavity_fast<true, 8, true>,   (const void *)k_cavity_fast<false, 8, true>,
+      (const void *)k_cavity_fast<true, 16, true>,  (const void *)k_cavity_fast<false, 16, true>,
+      (const void *)k_cavity_fast<true, 32, true>,  (const void *)k_cavity_fast<false, 32, true>,
+      (const void *)k_cavity_fast<true, 64, true>,  (const void *)k_cavity_fast<false, 64, true>,
+      (const void *)k_cavity_slow<true, 64>,        (const void *)k_cavity_slow<false, 64>};
   for (const void *f : cav)
     HC(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, BIG_LDS_BYTES));
+  HC(hipFuncSetAttribute((const void *)k_small_rounds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                         (int)small_lds(SR_K)));
 
   dalloc(&d_total, 4);
   dalloc(&d_cnt, CNT_N);
@@ -2620,7 +2789,7 @@ Refiner::~Refiner() {
   dfree(seg_in);
   dfree(c_pt); dfree(c_status); dfree(c_n); dfree(c_r);
   dfree(c_prio); dfree(c_win); dfree(c_rank); dfree(c_ws); dfree(c_pws);
-  dfree(c_act); dfree(c_slow); dfree(tmp_list); dfree(mix_list);
+  dfree(c_act); dfree(c_slow); dfree(c_seed); dfree(c_near); dfree(tmp_list); dfree(mix_list);
   dfree(sel_prio); dfree(sel_tmp); dfree(sel_list); dfree(d_hist);
   dfree(c_feat); dfree(c_score); dfree(c_deg); dfree(t_cnt); dfree(mlp_params);
   dfree(cb_cnt); dfree(cb_off); dfree(d_total); dfree(d_cnt);
@@ -3044,6 +3213,9 @@ void Refiner::ensure_cand(int nc) {
   dfree(c_prio); dfree(c_win); dfree(c_rank); dfree(c_act); dfree(c_slow);
   dalloc(&c_act, (size_t)c);
   dalloc(&c_slow, (size_t)c);
+  dfree(c_seed); dfree(c_near);
+  dalloc(&c_seed, (size_t)c);
+  dalloc(&c_near, (size_t)c);
   dalloc(&c_pt, (size_t)c);
   dalloc(&c_status, (size_t)c);
   dalloc(&c_n, (size_t)c);
@@ -3138,6 +3310,8 @@ PassD Refiner::pass_base(int Kc) const {
   ps.ctl = nullptr;
   ps.ids_sel = nullptr;
   ps.slow = c_slow;
+  ps.cseed = c_seed;
+  ps.cnear = c_near;
   ps.iters = std::max(1, opt.claim_iters);
   ps.shared_ring = opt.shared_ring;
   return ps;
@@ -3428,9 +3602,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   a.capT = capT;
   a.capS = capS;
   a.out = d_sr_out;
-  const size_t lds =
-      std::max(sizeof(int) * (size_t)(SR_THREADS / SR_LG) * group_lds_ints(std::min(K, ps.Kf), SR_LG),
-               sizeof(MlpWeights) + sizeof(short) * SR_WAVES * 16 * H1_STRIDE);
+  const size_t lds = small_lds(std::min(K, ps.Kf));
   tbegin(K_SMALL);
   k_small_rounds<<<1, SR_THREADS, lds, stream>>>(m, pr, ps, a);
   tend(K_SMALL, 0);
@@ -3824,6 +3996,13 @@ void Refiner::size_pass_buffers() {
   }
 }
 
+// Passes of at least this many candidates of a kind locate them in a launch
+// of their own, a lane per candidate.  A wave then does 64
+// points and walks in the instructions of 4, at the price of a launch and of
+// the longest of 64 walks: 10^6 points 103.5 -> 102.2 ms a call, 150,001
+// points (plain path) 87.3 -> 85.7; at 41,003 points even.
+constexpr int LOCATE_MIN = 16384;
+
 // Lanes per candidate in the cavity kernel: the configured group size,
 // widened until the groups' LDS fits one block.
 int Refiner::cavity_lanes(int Kc) const {
@@ -3833,23 +4012,26 @@ int Refiner::cavity_lanes(int Kc) const {
   return lg;
 }
 
-template <bool IS_SEG, bool FAST>
-static void launch_cavity_t(int lg, int grid, size_t lds, hipStream_t s, const MeshD &m,
-                            const ParamsD &pr, const PassD &ps, int kmax) {
-  if (FAST) {
-    switch (lg) {
-      case 8: k_cavity_fast<IS_SEG, 8><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-      case 16: k_cavity_fast<IS_SEG, 16><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-      case 32: k_cavity_fast<IS_SEG, 32><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-      default: k_cavity_fast<IS_SEG, 64><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-    }
+template <bool IS_SEG, bool LOCATED>
+static void launch_cavity_fast(int lg, int grid, size_t lds, hipStream_t s, const MeshD &m,
+                               const ParamsD &pr, const PassD &ps, int kmax) {
+  switch (lg) {
+    case 8: k_cavity_fast<IS_SEG, 8, LOCATED><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
+    case 16: k_cavity_fast<IS_SEG, 16, LOCATED><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
+    case 32: k_cavity_fast<IS_SEG, 32, LOCATED><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
+    default: k_cavity_fast<IS_SEG, 64, LOCATED><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
+  }
+}
+
+template <bool IS_SEG>
+static void launch_cavity_t(bool located, int lg, int grid, size_t lds, hipStream_t s,
+                            const MeshD &m, const ParamsD &pr, const PassD &ps, int kmax) {
+  if (located) {
+    const int n = IS_SEG ? ps.nseg : ps.nc - ps.nseg;
+    k_locate<IS_SEG><<<(n + LOC_BLOCK - 1) / LOC_BLOCK, LOC_BLOCK, 0, s>>>(m, pr, ps);
+    launch_cavity_fast<IS_SEG, true>(lg, grid, lds, s, m, pr, ps, kmax);
   } else {
-    switch (lg) {
-      case 8: k_cavity_slow<IS_SEG, 8><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-      case 16: k_cavity_slow<IS_SEG, 16><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-      case 32: k_cavity_slow<IS_SEG, 32><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-      default: k_cavity_slow<IS_SEG, 64><<<grid, 64, lds, s>>>(m, pr, ps, kmax); break;
-    }
+    launch_cavity_fast<IS_SEG, false>(lg, grid, lds, s, m, pr, ps, kmax);
   }
 }
 
@@ -3861,7 +4043,8 @@ void Refiner::launch_cavity(bool is_seg, int grid, const PassD &ps, bool resumed
   // the exact kernel takes a whole wave per candidate: its candidates are
   // the cavities beyond the fast kernel's LDS (33..K triangles, whose sort
   // and boundary cycle cost O(n^2 / lanes)) and the undecided signs
-  int lg = cavity_lanes(kf), lgs = 64;
+  int lg = cavity_lanes(kf);
+  const int lgs = 64;
   size_t lds = sizeof(int) * (size_t)(64 / lg) * group_lds_ints(kf, lg);
   size_t lds_slow = sizeof(int) * (size_t)(64 / lgs) * group_lds_ints(ps.K, lgs);
   if (lds_slow > (size_t)BIG_LDS_BYTES)
@@ -3869,11 +4052,13 @@ void Refiner::launch_cavity(bool is_seg, int grid, const PassD &ps, bool resumed
   if (grid < 1) grid = 1;
   int slow_grid = std::min(grid, pws_blocks * 4);
   if (is_seg) {
-    if (!resumed) launch_cavity_t<true, true>(lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
-    launch_cavity_t<true, false>(lgs, slow_grid, lds_slow, stream, m, pr, ps, opt.cav_cap_max);
+    const bool located = !ps.ctl && ps.nseg >= LOCATE_MIN;
+    if (!resumed) launch_cavity_t<true>(located, lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
+    k_cavity_slow<true, 64><<<slow_grid, 64, lds_slow, stream>>>(m, pr, ps, opt.cav_cap_max);
   } else {
-    if (!resumed) launch_cavity_t<false, true>(lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
-    launch_cavity_t<false, false>(lgs, slow_grid, lds_slow, stream, m, pr, ps, opt.cav_cap_max);
+    const bool located = !ps.ctl && ps.nc - ps.nseg >= LOCATE_MIN;
+    if (!resumed) launch_cavity_t<false>(located, lg, grid, lds, stream, m, pr, ps, opt.cav_cap_max);
+    k_cavity_slow<false, 64><<<slow_grid, 64, lds_slow, stream>>>(m, pr, ps, opt.cav_cap_max);
   }
   HC(hipGetLastError());
 }

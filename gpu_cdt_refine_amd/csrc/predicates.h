@@ -52,7 +52,7 @@ namespace gcdt {
 
 // Per-thread counters for the predicate stages (filter hit rates).
 struct PredStats {
-  unsigned long long fp32_hits, fp64_hits, exact_calls, dd_hits;
+  unsigned fp32_hits, fp64_hits, exact_calls, dd_hits;  // of one lane or candidate
 };
 
 GCDT_HD void two_sum(double a, double b, double &x, double &y) {
