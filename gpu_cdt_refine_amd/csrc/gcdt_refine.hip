@@ -1589,18 +1589,17 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_rank_apply(MeshD m, ParamsD pr, 
 // or the refinement ends; and inside a pass, after the cavities, when a
 // candidate needs the exact-predicate kernel, which the host then launches
 // (Refiner::run_pass with that pass to resume).
-// Bound by the cavities' dependent gathers and LDS chains (about 60% of a
-// pass); 16 waves of one CU.  A pass of 300 points' refinement takes 56 us
-// where the launches took 85 to 110 with the round trip; 8 waves (twice the
-// registers) took 59.  SR_CAP: a second and third batch of 64 cavities on the
-// one CU still costs less than the launches saved; at four batches the two
-// sides meet.
+// Bound by the chain of gathers and LDS round trips of the cavities (about half
+// of a pass), on one CU.  A pass of a 300-point refinement takes 50 us, where
+// its launches took 85 to 110 with the round trip.  8 waves with 256 registers:
+// 41,003 points 22.1 ms a call, 22.8 with 16 waves and spills.  SR_CAP: a few
+// batches of cavities on the one CU still cost less than the launches saved.
 // ---------------------------------------------------------------------------
-constexpr int SR_WAVES = 16, SR_THREADS = 64 * SR_WAVES;
+constexpr int SR_WAVES = 8, SR_THREADS = 64 * SR_WAVES;
 constexpr int SR_LG = 16;        // lanes per cavity
 constexpr int SR_K = 32;         // largest cavity held in LDS
 constexpr int SR_CAP = 256;      // candidates of a pass
-constexpr int SR_ENC = 1024;     // encroached subsegments listed
+constexpr int SR_ENC = 512;      // encroached subsegments listed
 constexpr int SR_DIRTY = 8192;   // rewritten triangles listed between two bad passes
 constexpr int SR_PASSES = 128;   // passes of one launch
 static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
