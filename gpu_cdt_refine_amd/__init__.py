@@ -16,6 +16,7 @@ Main entry points
 """
 import ctypes as C
 import os
+import weakref
 
 import numpy as np
 
@@ -377,13 +378,31 @@ def dropin_reset():
     L.gcdt_dropin_release()
 
 
+def _adopt(n, width, **field):
+    """The new[] array of one triangulateio field as a numpy array (n, width)
+    that frees it with its last reference: a copy of a mesh of 10^7 triangles
+    costs a quarter of the call that made it (10^6 points: 99.9 ms with
+    copies, 74.5 without)."""
+    (name, ptr), = field.items()
+    kind = ptr._type_
+    owned = TriangulateIO()
+    setattr(owned, name, ptr)
+    if not n or not ptr:
+        lib().gcdt_dropin_free(C.byref(owned), None, None)
+        return np.zeros((0, width), kind)
+    buf = (kind * (n * width)).from_address(C.addressof(ptr.contents))
+    free = weakref.finalize(buf, lib().gcdt_dropin_free, C.byref(owned), None, None)
+    free.atexit = False  # arrays may still be read by other exit handlers
+    return np.ctypeslib.as_array(buf).reshape(n, width)
+
+
 def dropin_refine(points, triangles, neighbors, segments, theta=25.0, insert=Offcenter,
                   mode=RUPPERT, debug=False):
     """Calls the C++ drop-in GPU_Refine_Quality on triangulateio records built
     from the arrays and returns (RefineResult, seconds): the wall time of the
     call alone (host arrays in, host arrays out, the reference's timing,
-    main.cpp:1860-1868).  The result arrays are copied out and the call's
-    new[] arrays freed."""
+    main.cpp:1860-1868).  The result arrays are the call's own new[] arrays,
+    each freed with its last reference."""
     P, T, N, S = _as_inputs(points, triangles, neighbors, segments)
     L = lib()
     f = getattr(L, DROPIN_SYMBOL)
@@ -404,16 +423,15 @@ def dropin_refine(points, triangles, neighbors, segments, theta=25.0, insert=Off
       C.byref(ts) if debug else None)
     dt = time.perf_counter() - t0
     np_, nt, ns = res.numberofpoints, res.numberoftriangles, res.numberofsegments
-    Po = np.ctypeslib.as_array(res.pointlist, shape=(np_, 2)).copy()
-    To = np.ctypeslib.as_array(res.trianglelist, shape=(nt, 3)).copy()
-    No = np.ctypeslib.as_array(res.neighborlist, shape=(nt, 3)).copy()
-    So = (np.ctypeslib.as_array(res.segmentlist, shape=(ns, 2)).copy() if ns
-          else np.zeros((0, 2), np.int32))
+    Po = _adopt(np_, 2, pointlist=res.pointlist)
+    To = _adopt(nt, 3, trianglelist=res.trianglelist)
+    No = _adopt(nt, 3, neighborlist=res.neighborlist)
+    So = _adopt(ns, 2, segmentlist=res.segmentlist)
     pst = tst = None
     if debug:
         pst = np.ctypeslib.as_array(C.cast(ps, C.POINTER(C.c_uint8)), shape=(np_,)).copy()
         tst = np.ctypeslib.as_array(C.cast(ts, C.POINTER(C.c_uint8)), shape=(nt,)).copy()
-    L.gcdt_dropin_free(C.byref(res), ps if debug else None, ts if debug else None)
+        L.gcdt_dropin_free(C.byref(TriangulateIO()), ps, ts)
     st = Stats()
     L.gcdt_dropin_last_stats(C.byref(st))
     d = st.as_dict()
