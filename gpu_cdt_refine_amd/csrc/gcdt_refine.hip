@@ -1919,8 +1919,7 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
 // The ear rule: repeatedly cut the first ear of the remaining link polygon
 // that turns left and whose circumcircle holds no other remaining vertex
 // strictly inside (exact signs); the cut triangles are the constrained
-// Delaunay triangles inside the star once the vertex is gone.  One lane per
-// candidate: stars are small and deletions rare.
+// Delaunay triangles inside the star once the vertex is gone.
 // ---------------------------------------------------------------------------
 
 struct DelD {
@@ -1943,248 +1942,274 @@ __device__ __forceinline__ unsigned long long del_epoch(const DelD &d) {
   return d.ctl ? (unsigned long long)d.ctl->i[C_EPOCH] + 1ull : d.epoch;
 }
 
+// A group of DEL_G lanes serves a nomination: a lane per ear, per claim and
+// per cut triangle; only the walk around the vertex is a serial chain of
+// gathers.  Per launch, against a lane per nomination: 2,999 points in Chew mode
+// scan 21.3 -> 15.8 us, apply 16.6 -> 6.3; 150,001 points 23.6 -> 20.5 and
+// 23.1 -> 7.9.
+constexpr int DEL_G = 16, DEL_BLOCK = 64;
+// LDS of a group: scan -- link coordinates (2 doubles) and indices, remaining
+// polygon; apply -- link, outer otri, subsegments, slots, sorted slots, cut
+// triangles
+constexpr int DEL_LDS_INTS = 256;
+static_assert(6 * DEL_MAX <= DEL_LDS_INTS && 5 * DEL_MAX + 3 * (DEL_MAX - 2) <= DEL_LDS_INTS,
+              "both kernels' arrays fit");
+
 // Apex of triangle t (corner j) on subsegment s: a deletion candidate?
-// Writes the star, link, outer otri, subsegments and the cut triangles to W
-// and the star size to *kout; returns the vertex or -1.  The link's indices,
-// coordinates (taken from the star's records) and the ear bookkeeping live
-// in this lane's column of the block's LDS arrays (lane-interleaved: entry i
-// of lane l at i * 64 + l).
-constexpr int DEL_LANES = 64;
-__device__ int del_candidate(const MeshD &m, int s, int t, int j, int *W, int *kout,
-                             double *pws, bool fp32, int *lp, double2 *lc,
-                             unsigned char *lrem) {
-  const int ln = threadIdx.x;
+// Writes the star, link, outer otri, subsegments and the cut triangles to W;
+// returns the star size, 0 if not, and the vertex in *vout.  Uniform across
+// the group (lane gl of it); lds: the group's, 16-byte aligned.
+__device__ int del_candidate(const MeshD &m, int s, int t, int j, int *W, int *vout, double *pws,
+                             bool fp32, int *lds, int gl) {
+  double2 *lc = reinterpret_cast<double2 *>(lds);
+  int *lp = lds + 4 * DEL_MAX, *rem = lp + DEL_MAX;
   int *star = W, *p = W + DEL_MAX, *o = W + 2 * DEL_MAX, *sg = W + 3 * DEL_MAX;
   int *nt = W + 4 * DEL_MAX;
   const TriRec &r0 = m.T[t];
   const int v = comp(r0.V, j);
-  if ((m.pflag[v] & (PF_FREE | PF_DEAD)) != PF_FREE) return -1;
+  *vout = v;
+  if ((m.pflag[v] & (PF_FREE | PF_DEAD)) != PF_FREE) return 0;
   const int2 sv = m.SV[s];
   const double2 O = m.P[sv.x], D = m.P[sv.y], V = r0.X[j];
-  if (!((O.x - V.x) * (D.x - V.x) + (O.y - V.y) * (D.y - V.y) < 0.0)) return -1;
-  int cur = t, jc = j, k = 0;
+  if (!((O.x - V.x) * (D.x - V.x) + (O.y - V.y) * (D.y - V.y) < 0.0)) return 0;
+  int cur = t, jc = j, k = 0, first = -1, prev = -1;
   for (;;) {
-    if (k == DEL_MAX) return -1;
+    if (k == DEL_MAX) return 0;
     const TriRec &r = m.T[cur];
     const int4 rv = r.V, rn = r.N, rs = r.S;
     const int x = comp(rv, (jc + 1) % 3), y = comp(rv, (jc + 2) % 3);
-    if (k == 0) {
-      lp[ln] = x;
-      lc[ln] = r.X[(jc + 1) % 3];
-    } else if (lp[k * DEL_LANES + ln] != x) {
-      return -1;
+    if (k == 0) first = x;
+    else if (prev != x) return 0;
+    prev = y;
+    if (gl == 0) {
+      lp[k] = x;
+      lc[k] = r.X[(jc + 1) % 3];
+      rem[k] = k;
+      star[k] = cur;
+      p[k] = x;
+      o[k] = comp(rn, jc);
+      sg[k] = comp(rs, jc);
     }
-    star[k] = cur;
-    o[k] = comp(rn, jc);
-    sg[k] = comp(rs, jc);
-    if (comp(rs, (jc + 1) % 3) >= 0) return -1;  // edge (v, y) is a subsegment
+    if (comp(rs, (jc + 1) % 3) >= 0) return 0;  // edge (v, y) is a subsegment
     const int nb = comp(rn, (jc + 1) % 3);
-    if (nb < 0) return -1;
+    if (nb < 0) return 0;
     k++;
     const int nx = nb >> 2;
     if (nx == t) {
-      if (y != lp[ln]) return -1;
+      if (y != first) return 0;
       break;
-    }
-    if (k < DEL_MAX) {
-      lp[k * DEL_LANES + ln] = y;
-      lc[k * DEL_LANES + ln] = r.X[(jc + 2) % 3];
     }
     const int4 vn = m.T[nx].V;
     const int jn = vn.x == v ? 0 : (vn.y == v ? 1 : (vn.z == v ? 2 : -1));
-    if (jn < 0) return -1;
+    if (jn < 0) return 0;
     cur = nx;
     jc = jn;
   }
-  if (k < 3) return -1;
-  for (int q = 0; q < k; q++) p[q] = lp[q * DEL_LANES + ln];
-  auto REM = [&](int q) -> int { return lrem[q * DEL_LANES + ln]; };
-  auto PT = [&](int q) -> double2 { return lc[REM(q) * DEL_LANES + ln]; };
-  auto ID = [&](int q) -> int { return lp[REM(q) * DEL_LANES + ln]; };
+  if (k < 3) return 0;
+  wave_sync();
   int r = k, ne = 0;
-  for (int q = 0; q < k; q++) lrem[q * DEL_LANES + ln] = (unsigned char)q;
   while (r > 3) {
     int found = -1;
-    for (int q = 0; q < r && found < 0; q++) {
-      const int qa = (q + r - 1) % r, qc = (q + 1) % r;
-      const double2 A = PT(qa), B = PT(q), C = PT(qc);
-      if (orient2d_sign(A.x, A.y, B.x, B.y, C.x, C.y, fp32, nullptr) <= 0) continue;
-      bool ok = true;
-      for (int w = 0; w < r && ok; w++) {
-        if (w == qa || w == q || w == qc) continue;
-        const double2 E = PT(w);
-        if (incircle_sign(A.x, A.y, B.x, B.y, C.x, C.y, E.x, E.y, pws, fp32, nullptr) > 0) ok = false;
+    for (int q0 = 0; q0 < r && found < 0; q0 += DEL_G) {
+      const int q = q0 + gl;
+      bool ok = false;
+      if (q < r) {
+        const int qa = q == 0 ? r - 1 : q - 1, qc = q + 1 == r ? 0 : q + 1;
+        const double2 A = lc[rem[qa]], B = lc[rem[q]], C = lc[rem[qc]];
+        ok = orient2d_sign(A.x, A.y, B.x, B.y, C.x, C.y, fp32, nullptr) > 0;
+        for (int w = 0; w < r && ok; w++) {
+          if (w == qa || w == q || w == qc) continue;
+          const double2 E = lc[rem[w]];
+          if (incircle_sign(A.x, A.y, B.x, B.y, C.x, C.y, E.x, E.y, pws, fp32, nullptr) > 0)
+            ok = false;
+        }
       }
-      if (ok) found = q;
+      const unsigned long long b = group_bits<DEL_G>(__ballot(ok));
+      if (b != 0ull) found = q0 + __builtin_ctzll(b);
     }
-    if (found < 0) return -1;
-    nt[3 * ne] = ID((found + r - 1) % r);
-    nt[3 * ne + 1] = ID(found);
-    nt[3 * ne + 2] = ID((found + 1) % r);
+    if (found < 0) return 0;
+    if (gl < 3) {
+      const int q = found + gl - 1;
+      nt[3 * ne + gl] = lp[rem[q < 0 ? r - 1 : (q == r ? 0 : q)]];
+    }
     ne++;
-    for (int q = found; q + 1 < r; q++) lrem[q * DEL_LANES + ln] = lrem[(q + 1) * DEL_LANES + ln];
+    // close the gap: entries after the ear move down
+    constexpr int PER = (DEL_MAX + DEL_G - 1) / DEL_G;
+    int mv[PER];
+    for (int e = 0; e < PER; e++) {
+      const int q = e * DEL_G + gl;
+      mv[e] = q >= found && q + 1 < r ? rem[q + 1] : -1;
+    }
+    wave_sync();
+    for (int e = 0; e < PER; e++)
+      if (mv[e] >= 0) rem[e * DEL_G + gl] = mv[e];
     r--;
+    wave_sync();
   }
   {
-    const double2 A = PT(0), B = PT(1), C = PT(2);
-    if (orient2d_sign(A.x, A.y, B.x, B.y, C.x, C.y, fp32, nullptr) <= 0) return -1;
+    const double2 A = lc[rem[0]], B = lc[rem[1]], C = lc[rem[2]];
+    if (orient2d_sign(A.x, A.y, B.x, B.y, C.x, C.y, fp32, nullptr) <= 0) return 0;
   }
-  nt[3 * ne] = ID(0);
-  nt[3 * ne + 1] = ID(1);
-  nt[3 * ne + 2] = ID(2);
-  *kout = k;
-  return v;
+  if (gl < 3) nt[3 * ne + gl] = lp[rem[gl]];
+  return k;
 }
 
-// Nominations, stars and retriangulations, one lane per nomination (both
-// sides of a subsegment in parallel); a candidate then claims its star and
-// the outer triangles across its link (claims commute, so no other lane's
-// star needs to be known).
-__global__ __launch_bounds__(DEL_LANES) void k_del_scan(MeshD m, ParamsD pr, DelD dd) {
-  __shared__ int s_lp[DEL_MAX * DEL_LANES];
-  __shared__ double2 s_lc[DEL_MAX * DEL_LANES];
-  __shared__ unsigned char s_rem[DEL_MAX * DEL_LANES];
+// Nomination d (both sides of a subsegment are nominations of their own): its
+// star and retriangulation; a candidate then claims its star and the outer
+// triangles across its link (claims commute, so no other group's star needs
+// to be known).
+__device__ __forceinline__ void del_scan_one(const MeshD &m, const ParamsD &pr, const DelD &dd,
+                                             int d, unsigned long long ep, double *pws, int *lds,
+                                             int gl) {
+  const int s = dd.ids[d >> 1], side = d & 1;
+  int t1, j1, t2, j2;
+  seg_sides(m, s, t1, j1, t2, j2);
+  const int t = side ? t2 : t1, j = side ? j2 : j1;
+  int v = -1, k = 0;
+  int *W = dd.ws + (size_t)d * DEL_WS;
+  if (t >= 0) {
+    const ParamsD lp = params_at(pr, m, t);
+    if (dd.policy == 2 || (dd.policy == 1 && !lp.ruppert))
+      k = del_candidate(m, s, t, j, W, &v, pws, dd.use_fp32 != 0, lds, gl);
+  }
+  if (gl == 0) {
+    dd.dv[d] = k > 0 ? v : -1;
+    dd.dk[d] = k;
+  }
+  if (k > 0) {
+    // the star was written by lane 0; a wave's accesses to one address keep
+    // their order
+    wave_sync();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const unsigned long long key = claim_key(ep, 0, d);
+    for (int q = gl; q < k; q += DEL_G) {
+      atomicMax(&m.claim[2 * (size_t)W[q]], key);
+      const int o = W[2 * DEL_MAX + q];
+      if (o >= 0) atomicMax(&m.claim[2 * (size_t)(o >> 2)], key);
+    }
+  }
+}
+
+__global__ __launch_bounds__(DEL_BLOCK) void k_del_scan(MeshD m, ParamsD pr, DelD dd) {
+  __shared__ __align__(16) int s_lds[(DEL_BLOCK / DEL_G) * DEL_LDS_INTS];
   const int nd = 2 * del_nseg(dd);
   const unsigned long long ep = del_epoch(dd);
-  const int lane = blockIdx.x * blockDim.x + threadIdx.x;
-  double *pws = dd.pws + (size_t)lane * GCDT_INCIRCLE_WS;
-  for (int d = lane; d < nd; d += gridDim.x * blockDim.x) {
-    const int s = dd.ids[d >> 1], side = d & 1;
-    int t1, j1, t2, j2;
-    seg_sides(m, s, t1, j1, t2, j2);
-    const int t = side ? t2 : t1, j = side ? j2 : j1;
-    int v = -1;
-    int *W = dd.ws + (size_t)d * DEL_WS;
-    if (t >= 0) {
-      const ParamsD lp = params_at(pr, m, t);
-      if (dd.policy == 2 || (dd.policy == 1 && !lp.ruppert))
-        v = del_candidate(m, s, t, j, W, dd.dk + d, pws, dd.use_fp32 != 0, s_lp, s_lc, s_rem);
-    }
-    dd.dv[d] = v;
-    if (v >= 0) {
-      const int k = dd.dk[d];
-      const unsigned long long key = claim_key(ep, 0, d);
-      for (int q = 0; q < k; q++) {
-        atomicMax(&m.claim[2 * (size_t)W[q]], key);
-        const int o = W[2 * DEL_MAX + q];
-        if (o >= 0) atomicMax(&m.claim[2 * (size_t)(o >> 2)], key);
-      }
-    }
+  const int grp = threadIdx.x / DEL_G, gl = threadIdx.x % DEL_G;
+  constexpr int per = DEL_BLOCK / DEL_G;
+  double *pws = dd.pws + ((size_t)blockIdx.x * DEL_BLOCK + threadIdx.x) * GCDT_INCIRCLE_WS;
+  for (int d = blockIdx.x * per + grp; d < nd; d += gridDim.x * per) {
+    del_scan_one(m, pr, dd, d, ep, pws, s_lds + grp * DEL_LDS_INTS, gl);
+    wave_sync();
   }
 }
 
 // A candidate holding every triangle of its star and ring deletes its
-// vertex right away: winners' regions are disjoint and the other lanes' win
+// vertex right away: winners' regions are disjoint and the other groups' win
 // tests read only claim words, which no apply writes.  The cut triangles
 // take the star's slots in ascending order (the two largest slots die);
 // links inside the star are matched edge by edge, link edges take the outer
 // triangle (whose back-link is repaired) and the subsegment (whose adjacent
-// otri is repaired).
-__global__ __launch_bounds__(DEL_LANES) void k_del_apply(MeshD m, DelD dd) {
-  // this lane's link, outer otri, subsegments, sorted slots and cut
-  // triangles, lane-interleaved in LDS for the edge matching below
-  __shared__ int a_p[DEL_MAX * DEL_LANES], a_o[DEL_MAX * DEL_LANES], a_s[DEL_MAX * DEL_LANES],
-      a_sl[DEL_MAX * DEL_LANES], a_nt[3 * (DEL_MAX - 2) * DEL_LANES];
-  const int ln = threadIdx.x;
+// otri is repaired).  Returns the star size, 0 if the vertex stays.
+template <class Trace>
+__device__ __forceinline__ int del_apply_one(const MeshD &m, const DelD &dd, int d,
+                                             unsigned long long ep, int *lds, int gl,
+                                             const Trace &trace) {
+  const int v = dd.dv[d];
+  if (v < 0) return 0;
+  const int *W = dd.ws + (size_t)d * DEL_WS;
+  const int k = dd.dk[d];
+  int *P_ = lds, *O_ = P_ + DEL_MAX, *S_ = O_ + DEL_MAX, *U_ = S_ + DEL_MAX, *SL = U_ + DEL_MAX,
+      *NT = SL + DEL_MAX;
+  const unsigned long long key = claim_key(ep, 0, d);
+  bool lose = false;
+  for (int q = gl; q < k; q += DEL_G) {
+    const int st = W[q], o = W[2 * DEL_MAX + q];
+    U_[q] = st;
+    O_[q] = o;
+    P_[q] = W[DEL_MAX + q];
+    S_[q] = W[3 * DEL_MAX + q];
+    lose |= m.claim[2 * (size_t)st] != key;
+    if (o >= 0) lose |= m.claim[2 * (size_t)(o >> 2)] != key;
+  }
+  for (int q = gl; q < 3 * (k - 2); q += DEL_G) NT[q] = W[4 * DEL_MAX + q];
+  if (group_bits<DEL_G>(__ballot(lose)) != 0ull) return 0;
+  wave_sync();
+  for (int q = gl; q < k; q += DEL_G) {
+    const int x = U_[q];
+    int rank = 0;
+    for (int w = 0; w < k; w++) rank += U_[w] < x;
+    SL[rank] = x;
+  }
+  wave_sync();
+  const int inst = m.batched ? m.T[SL[0]].V.w : 0;
+  wave_sync();  // the instance is read before any record is rewritten
+  for (int q = gl; q < k - 2; q += DEL_G) {
+    const int st = SL[q];
+    const int V0 = NT[3 * q], V1 = NT[3 * q + 1], V2 = NT[3 * q + 2];
+    int nn[3], ss[3];
+    for (int e = 0; e < 3; e++) {
+      const int u = e == 0 ? V1 : (e == 1 ? V2 : V0);
+      const int w = e == 0 ? V2 : (e == 1 ? V0 : V1);
+      int nb = -2, sgv = -1;
+      for (int i = 0; i < k && nb == -2; i++)
+        if (P_[i] == u && P_[i + 1 == k ? 0 : i + 1] == w) {
+          nb = O_[i];
+          sgv = S_[i];
+          if (nb >= 0) *nbr_slot(m.T, nb >> 2, nb & 3) = (st << 2) | e;
+          if (sgv >= 0) m.ST[sgv] = (st << 2) | e;
+        }
+      for (int q2 = 0; q2 < k - 2 && nb == -2; q2++) {
+        if (q2 == q) continue;
+        for (int e2 = 0; e2 < 3; e2++)
+          if (NT[3 * q2 + (e2 + 1) % 3] == w && NT[3 * q2 + (e2 + 2) % 3] == u) {
+            nb = (SL[q2] << 2) | e2;
+            break;
+          }
+      }
+      nn[e] = nb;
+      ss[e] = sgv;
+    }
+    TriRec r;
+    r.V = make_int4(V0, V1, V2, inst);
+    r.N = make_int4(nn[0], nn[1], nn[2], 0);
+    r.S = make_int4(ss[0], ss[1], ss[2], 0);
+    r.X[0] = m.P[V0];
+    r.X[1] = m.P[V1];
+    r.X[2] = m.P[V2];
+    r.pad[0] = r.pad[1] = make_int4(0, 0, 0, 0);
+    m.T[st] = r;
+    trace.rewritten(m, st);
+    m.tflag[st] = TF_ALIVE | TF_CHECK;
+  }
+  if (gl < 2) {
+    const int st = SL[k - 2 + gl];
+    TriRec r;
+    r.V = make_int4(-1, -1, -1, 0);
+    r.N = make_int4(-1, -1, -1, 0);
+    r.S = make_int4(-1, -1, -1, 0);
+    r.X[0] = r.X[1] = r.X[2] = make_double2(0.0, 0.0);
+    r.pad[0] = r.pad[1] = make_int4(0, 0, 0, 0);
+    m.T[st] = r;
+    m.tflag[st] = 0;
+  }
+  if (gl == 0) m.pflag[v] |= PF_DEAD;
+  return k;
+}
+
+__global__ __launch_bounds__(DEL_BLOCK) void k_del_apply(MeshD m, DelD dd) {
+  __shared__ __align__(16) int s_lds[(DEL_BLOCK / DEL_G) * DEL_LDS_INTS];
   const int nd = 2 * del_nseg(dd);
   const unsigned long long ep = del_epoch(dd);
+  const int grp = threadIdx.x / DEL_G, gl = threadIdx.x % DEL_G;
+  constexpr int per = DEL_BLOCK / DEL_G;
   unsigned long long ndel = 0, nflip = 0;
-  for (int d = blockIdx.x * blockDim.x + threadIdx.x; d < nd; d += gridDim.x * blockDim.x) {
-    if (dd.dv[d] < 0) continue;
-    const int *W = dd.ws + (size_t)d * DEL_WS;
-    const int k = dd.dk[d];
-    auto P_ = [&](int i) -> int & { return a_p[i * DEL_LANES + ln]; };
-    auto O_ = [&](int i) -> int & { return a_o[i * DEL_LANES + ln]; };
-    auto S_ = [&](int i) -> int & { return a_s[i * DEL_LANES + ln]; };
-    auto SL = [&](int i) -> int & { return a_sl[i * DEL_LANES + ln]; };
-    auto NT = [&](int i) -> int & { return a_nt[i * DEL_LANES + ln]; };
-    // the workspace first (independent loads), then every claim word of the
-    // star and ring (independent again): two round trips, not two per entry
-    // (unrolled by 8: eight loads in flight before their first use)
-#pragma unroll 8
-    for (int q = 0; q < k; q++) {
-      SL(q) = W[q];
-      O_(q) = W[2 * DEL_MAX + q];
+  for (int d = blockIdx.x * per + grp; d < nd; d += gridDim.x * per) {
+    const int k = del_apply_one(m, dd, d, ep, s_lds + grp * DEL_LDS_INTS, gl, NoTrace{});
+    if (k > 0 && gl == 0) {
+      ndel++;
+      nflip += (unsigned long long)(k - 3);
     }
-    {
-      const unsigned long long key = claim_key(ep, 0, d);
-      bool w = true;
-#pragma unroll 8
-      for (int q = 0; q < k; q++) {
-        const int o = O_(q);
-        const bool a = m.claim[2 * (size_t)SL(q)] == key;
-        const bool b = o < 0 || m.claim[2 * (size_t)(o >> 2)] == key;
-        w = w & a & b;
-      }
-      if (!w) continue;
-    }
-#pragma unroll 8
-    for (int q = 0; q < k; q++) {
-      P_(q) = W[DEL_MAX + q];
-      S_(q) = W[3 * DEL_MAX + q];
-    }
-#pragma unroll 8
-    for (int q = 0; q < 3 * (k - 2); q++) NT(q) = W[4 * DEL_MAX + q];
-    const int inst = m.batched ? m.T[SL(0)].V.w : 0;
-    for (int q = 1; q < k; q++) {
-      const int x = SL(q);
-      int w = q - 1;
-      while (w >= 0 && SL(w) > x) {
-        SL(w + 1) = SL(w);
-        w--;
-      }
-      SL(w + 1) = x;
-    }
-    for (int q = 0; q < k - 2; q++) {
-      const int st = SL(q);
-      const int V0 = NT(3 * q), V1 = NT(3 * q + 1), V2 = NT(3 * q + 2);
-      int nn[3], ss[3];
-      for (int e = 0; e < 3; e++) {
-        const int u = e == 0 ? V1 : (e == 1 ? V2 : V0);
-        const int w = e == 0 ? V2 : (e == 1 ? V0 : V1);
-        int nb = -2, sgv = -1;
-        for (int i = 0; i < k && nb == -2; i++)
-          if (P_(i) == u && P_((i + 1) % k) == w) {
-            nb = O_(i);
-            sgv = S_(i);
-            if (nb >= 0) *nbr_slot(m.T, nb >> 2, nb & 3) = (st << 2) | e;
-            if (sgv >= 0) m.ST[sgv] = (st << 2) | e;
-          }
-        for (int q2 = 0; q2 < k - 2 && nb == -2; q2++) {
-          if (q2 == q) continue;
-          for (int e2 = 0; e2 < 3; e2++)
-            if (NT(3 * q2 + (e2 + 1) % 3) == w && NT(3 * q2 + (e2 + 2) % 3) == u) {
-              nb = (SL(q2) << 2) | e2;
-              break;
-            }
-        }
-        nn[e] = nb;
-        ss[e] = sgv;
-      }
-      TriRec r;
-      r.V = make_int4(V0, V1, V2, inst);
-      r.N = make_int4(nn[0], nn[1], nn[2], 0);
-      r.S = make_int4(ss[0], ss[1], ss[2], 0);
-      r.X[0] = m.P[V0];
-      r.X[1] = m.P[V1];
-      r.X[2] = m.P[V2];
-      r.pad[0] = r.pad[1] = make_int4(0, 0, 0, 0);
-      m.T[st] = r;
-      m.tflag[st] = TF_ALIVE | TF_CHECK;
-    }
-    for (int q = k - 2; q < k; q++) {
-      TriRec r;
-      r.V = make_int4(-1, -1, -1, 0);
-      r.N = make_int4(-1, -1, -1, 0);
-      r.S = make_int4(-1, -1, -1, 0);
-      r.X[0] = r.X[1] = r.X[2] = make_double2(0.0, 0.0);
-      r.pad[0] = r.pad[1] = make_int4(0, 0, 0, 0);
-      m.T[SL(q)] = r;
-      m.tflag[SL(q)] = 0;
-    }
-    m.pflag[dd.dv[d]] |= PF_DEAD;
-    ndel++;
-    nflip += (unsigned long long)(k - 3);
+    wave_sync();
   }
   ndel = wave_sum(ndel);
   nflip = wave_sum(nflip);
@@ -3335,13 +3360,14 @@ void Refiner::enqueue_deletion(const DelD &dd) {
   // host loop: grids sized by the pass's subsegment candidates (most
   // segment passes hold few); graph loop: sized for the largest pass
   const long long n = dd.ctl ? DEL_CANDS : std::min(dd.nseg, DEL_CANDS);
-  const int gs = (int)std::max(1LL, std::min<long long>(pws_blocks * 4, (2 * n + 63) / 64));
-  const int g = (int)std::max(1LL, std::min<long long>(2048, (2 * n + 63) / 64));
+  constexpr int per = DEL_BLOCK / DEL_G;
+  const int gs = (int)std::max(1LL, std::min<long long>(pws_blocks * 4, (2 * n + per - 1) / per));
+  const int g = (int)std::max(1LL, std::min<long long>(4096, (2 * n + per - 1) / per));
   tbegin(K_DEL_SCAN);
-  k_del_scan<<<gs, DEL_LANES, 0, stream>>>(m, pr, dd);
+  k_del_scan<<<gs, DEL_BLOCK, 0, stream>>>(m, pr, dd);
   tend(K_DEL_SCAN, dd.ctl ? 0 : n);
   tbegin(K_DEL_APPLY);
-  k_del_apply<<<g, DEL_LANES, 0, stream>>>(m, dd);
+  k_del_apply<<<g, DEL_BLOCK, 0, stream>>>(m, dd);
   tend(K_DEL_APPLY, 0);
   HC(hipGetLastError());
 }
