@@ -29,85 +29,7 @@
 
 namespace gcdt {
 
-// One wave computes the forward pass of 16 samples starting at row0.
-// Outputs D-layout activations (pre-ReLU kept implicitly by value > 0).
-struct Fwd {
-  floatx4 h1[4], h2[4];  // post-ReLU activations, D layout, 4 column blocks
-  float y[4];            // lane l: outputs of rows 4*(l/16)+j (all 16 lanes of a group hold the same)
-};
-
-__device__ __forceinline__ void mlp_forward16(const float *__restrict__ X,
-                                              int n, int row0,
-                                              const float *__restrict__ P,
-                                              short *lds /* 16*64 */,
-                                              Fwd &f) {
-  int l = threadIdx.x & 63;
-  int r = l % 16, kb = l / 16;
-  // layer 1: A = X[row0 + r][4kb..4kb+3]
-  bf16x4 a;
-  for (int j = 0; j < 4; j++) {
-    int row = row0 + r;
-    a[j] = row < n ? f2bf(X[(size_t)row * MLP_IN + 4 * kb + j]) : (short)0;
-  }
-  for (int cb = 0; cb < 4; cb++) {
-    bf16x4 b;
-    for (int j = 0; j < 4; j++) b[j] = f2bf(P[OFF_W1 + (4 * kb + j) * MLP_H + cb * 16 + r]);
-    floatx4 z = {0.f, 0.f, 0.f, 0.f};
-    z = mfma(a, b, z);
-    float bias = P[OFF_B1 + cb * 16 + r];
-    for (int j = 0; j < 4; j++) z[j] = fmaxf(z[j] + bias, 0.f);
-    f.h1[cb] = z;
-  }
-  // stage H1 (bf16) through LDS to re-read it in A layout
-  for (int cb = 0; cb < 4; cb++)
-    for (int j = 0; j < 4; j++) lds[(4 * kb + j) * MLP_H + cb * 16 + r] = f2bf(f.h1[cb][j]);
-  __syncthreads();
-  for (int cb = 0; cb < 4; cb++) {
-    floatx4 z = {0.f, 0.f, 0.f, 0.f};
-    for (int kk = 0; kk < 4; kk++) {  // K blocks of 16 over the 64 hidden units
-      bf16x4 a2, b2;
-      for (int j = 0; j < 4; j++) {
-        a2[j] = lds[r * MLP_H + kk * 16 + 4 * kb + j];
-        b2[j] = f2bf(P[OFF_W2 + (kk * 16 + 4 * kb + j) * MLP_H + cb * 16 + r]);
-      }
-      z = mfma(a2, b2, z);
-    }
-    float bias = P[OFF_B2 + cb * 16 + r];
-    for (int j = 0; j < 4; j++) z[j] = fmaxf(z[j] + bias, 0.f);
-    f.h2[cb] = z;
-  }
-  __syncthreads();
-  // layer 3: y[row] = sum_c H2[row][c] W3[c] + b3, reduced over the 16 lanes
-  // of a group (they hold the 16 columns of each block)
-  for (int j = 0; j < 4; j++) {
-    float s = 0.f;
-    for (int cb = 0; cb < 4; cb++) s += f.h2[cb][j] * bf2f(f2bf(P[OFF_W3 + cb * 16 + r]));
-    for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
-    f.y[j] = s + P[OFF_B3];
-  }
-}
-
-// dn (optional): the row count is read from device memory, and the kernel
-// does nothing unless *dgo is set (graph-driven refinement loop).
-__global__ __launch_bounds__(64) void k_mlp_forward(const float *X, int n,
-                                                    const float *P, float *y,
-                                                    const int *dn, const int *dgo) {
-  __shared__ short lds[16 * MLP_H];
-  if (dn) n = *dgo ? *dn : 0;
-  int l = threadIdx.x;
-  for (int row0 = blockIdx.x * 16; row0 < n; row0 += gridDim.x * 16) {
-    Fwd f;
-    mlp_forward16(X, n, row0, P, lds, f);
-    if (l % 16 == 0)
-      for (int j = 0; j < 4; j++) {
-        int row = row0 + 4 * (l / 16) + j;
-        if (row < n) y[row] = f.y[j];
-      }
-    __syncthreads();
-  }
-}
-
-// Inference: the forward pass above with the weights converted to BF16 once
+// Inference: the weights converted to BF16 once
 // per block and kept in LDS, four waves per block, each wave taking 16 rows
 // at a time; layer 2 on the 16x16x32 MFMA.  Same roundings as the training
 // forward (inputs, weights and hidden activations in BF16, FP32 accumulate);
@@ -135,100 +57,150 @@ __global__ __launch_bounds__(64 * INF_WAVES) void k_mlp_infer(const float *X, in
 
 // Mean-squared-error gradient over n samples, accumulated into G (MLP_NPARAM
 // floats, zeroed by the caller) and the loss sum into *loss.
-__global__ __launch_bounds__(64) void k_mlp_grad(const float *X, const float *t,
-                                                 int n, const float *P, float *G,
-                                                 float *loss) {
-  __shared__ short lds[16 * MLP_H];
+//
+// A wave takes 16 rows at a time and keeps its share of every gradient in
+// registers from tile to tile (the weight gradients as MFMA accumulators); the
+// block sums its waves in LDS once and adds to G with one atomic per
+// parameter.  Weights are converted to BF16 once per block.  200,003 rows: 515 -> 100 us,
+// where every tile had added 85 values per lane to LDS and converted its
+// weights again from global memory.
+constexpr int GRAD_WAVES = 4, GRAD_BLOCKS = 256;
+__global__ __launch_bounds__(64 * GRAD_WAVES) void k_mlp_grad(const float *X, const float *t,
+                                                              int n, const float *P, float *G,
+                                                              float *loss) {
+  __shared__ MlpWeights w;
+  __shared__ __align__(16) short w2n[MLP_H * W2T_STRIDE];          // W2 [k][c]
+  __shared__ __align__(16) short hs[GRAD_WAVES][16 * H1_STRIDE];  // per wave: [row][unit]
   __shared__ float gsh[MLP_NPARAM];
-  int l = threadIdx.x, r = l % 16, kb = l / 16;
-  for (int k = l; k < MLP_NPARAM; k += 64) gsh[k] = 0.f;
+  const int tid = threadIdx.x, wv = tid / 64, l = tid & 63, r = l % 16, kb = l / 16;
+  mlp_stage<64 * GRAD_WAVES>(P, w, tid);
+  for (int i = tid; i < MLP_H * MLP_H; i += 64 * GRAD_WAVES)
+    w2n[(i / MLP_H) * W2T_STRIDE + i % MLP_H] = f2bf(P[OFF_W2 + i]);
+  for (int k = tid; k < MLP_NPARAM; k += 64 * GRAD_WAVES) gsh[k] = 0.f;
   __syncthreads();
-  float lsum = 0.f;
-  for (int row0 = blockIdx.x * 16; row0 < n; row0 += gridDim.x * 16) {
-    Fwd f;
-    mlp_forward16(X, n, row0, P, lds, f);
-    // dy for the 4 rows of this lane group
+  short *H = hs[wv];
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  floatx4 g1[4], g2[4][4];
+  float gb1[4], gb2[4], gw3[4], gb3 = 0.f, lsum = 0.f;
+  for (int a = 0; a < 4; a++) {
+    g1[a] = zero;
+    gb1[a] = gb2[a] = gw3[a] = 0.f;
+    for (int b = 0; b < 4; b++) g2[a][b] = zero;
+  }
+  for (int row0 = (blockIdx.x * GRAD_WAVES + wv) * 16; row0 < n;
+       row0 += gridDim.x * GRAD_WAVES * 16) {
+    // ---- forward (D layout: lane l holds column l % 16, rows 4 (l / 16) + j) ----
+    floatx4 h1[4], h2[4];
+    bf16x4 ax0;
+    {
+      const int row = row0 + r;
+      for (int j = 0; j < 4; j++)
+        ax0[j] = row < n ? f2bf(X[(size_t)row * MLP_IN + 4 * kb + j]) : (short)0;
+    }
+    bf16x4 a1[4];  // H1 in BF16
+    for (int cb = 0; cb < 4; cb++) {
+      bf16x4 b;
+      for (int j = 0; j < 4; j++) b[j] = w.w1[(4 * kb + j) * MLP_H + cb * 16 + r];
+      floatx4 z = mfma(ax0, b, zero);
+      const float bias = w.b1[cb * 16 + r];
+      for (int j = 0; j < 4; j++) {
+        z[j] = fmaxf(z[j] + bias, 0.f);
+        a1[cb][j] = f2bf(z[j]);
+        H[(4 * kb + j) * H1_STRIDE + cb * 16 + r] = a1[cb][j];
+      }
+      h1[cb] = z;
+    }
+    wave_sync();
+    for (int cb = 0; cb < 4; cb++) {
+      floatx4 z = zero;
+      for (int kk = 0; kk < 2; kk++) {
+        const shortx8 a2 =
+            *reinterpret_cast<const shortx8 *>(&H[r * H1_STRIDE + kk * 32 + 8 * kb]);
+        const shortx8 b2v = *reinterpret_cast<const shortx8 *>(
+            &w.w2t[(cb * 16 + r) * W2T_STRIDE + kk * 32 + 8 * kb]);
+        z = mfma32(a2, b2v, z);
+      }
+      const float bias = w.b2[cb * 16 + r];
+      for (int j = 0; j < 4; j++) z[j] = fmaxf(z[j] + bias, 0.f);
+      h2[cb] = z;
+    }
+    // ---- output, its error and layer 3 ----
     float dy[4];
     for (int j = 0; j < 4; j++) {
-      int row = row0 + 4 * kb + j;
-      float e = row < n ? f.y[j] - t[row] : 0.f;
+      float y = 0.f;
+      for (int cb = 0; cb < 4; cb++) y += h2[cb][j] * w.w3[cb * 16 + r];
+      for (int off = 8; off > 0; off >>= 1) y += __shfl_xor(y, off, 16);
+      const int row = row0 + 4 * kb + j;
+      const float e = row < n ? y + w.b3 - t[row] : 0.f;
       dy[j] = 2.f * e / (float)n;
       if (r == 0) lsum += e * e;
     }
-    // layer 3: dW3[c] = sum_rows H2[row][c] dy[row]; db3 = sum dy
-    for (int cb = 0; cb < 4; cb++) {
-      float s = 0.f;
-      for (int j = 0; j < 4; j++) s += f.h2[cb][j] * dy[j];
-      atomicAdd(&gsh[OFF_W3 + cb * 16 + r], s);
-    }
-    if (r == 0) atomicAdd(&gsh[OFF_B3], dy[0] + dy[1] + dy[2] + dy[3]);
-    // dH2 = dy * W3 (.) relu'
-    floatx4 dh2[4];
-    for (int cb = 0; cb < 4; cb++) {
-      float w3 = bf2f(f2bf(P[OFF_W3 + cb * 16 + r]));
-      for (int j = 0; j < 4; j++) dh2[cb][j] = f.h2[cb][j] > 0.f ? dy[j] * w3 : 0.f;
-    }
-    // dW2 = H1^T dH2: A = H1^T block (D layout of H1), B = dH2 (D layout)
-    for (int mb = 0; mb < 4; mb++) {
-      bf16x4 a;
-      for (int j = 0; j < 4; j++) a[j] = f2bf(f.h1[mb][j]);
-      for (int nb = 0; nb < 4; nb++) {
-        bf16x4 b;
-        for (int j = 0; j < 4; j++) b[j] = f2bf(dh2[nb][j]);
-        floatx4 z = {0.f, 0.f, 0.f, 0.f};
-        z = mfma(a, b, z);  // rows: hidden1 unit mb*16 + 4kb + j, col: hidden2 nb*16 + r
-        for (int j = 0; j < 4; j++)
-          atomicAdd(&gsh[OFF_W2 + (mb * 16 + 4 * kb + j) * MLP_H + nb * 16 + r], z[j]);
-      }
-      // db2: column sums of dH2
-    }
-    for (int cb = 0; cb < 4; cb++) {
-      float s = dh2[cb][0] + dh2[cb][1] + dh2[cb][2] + dh2[cb][3];
-      atomicAdd(&gsh[OFF_B2 + cb * 16 + r], s);
-    }
-    // dH1 = dH2 W2^T (.) relu'(H1): stage dH2 (bf16) through LDS for A layout
     for (int cb = 0; cb < 4; cb++)
-      for (int j = 0; j < 4; j++) lds[(4 * kb + j) * MLP_H + cb * 16 + r] = f2bf(dh2[cb][j]);
-    __syncthreads();
-    floatx4 dh1[4];
-    for (int cb = 0; cb < 4; cb++) {  // output: hidden1 block cb
-      floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      for (int kk = 0; kk < 4; kk++) {  // K: hidden2 units
-        bf16x4 a2, b2;
-        for (int j = 0; j < 4; j++) {
-          a2[j] = lds[r * MLP_H + kk * 16 + 4 * kb + j];
-          // B[k][n] = W2^T[k][n] = W2[n][k], n = hidden1 unit cb*16 + r
-          b2[j] = f2bf(P[OFF_W2 + (cb * 16 + r) * MLP_H + kk * 16 + 4 * kb + j]);
-        }
-        z = mfma(a2, b2, z);
+      for (int j = 0; j < 4; j++) gw3[cb] += h2[cb][j] * dy[j];
+    if (r == 0) gb3 += dy[0] + dy[1] + dy[2] + dy[3];
+    // ---- dH2 = dy W3 (.) relu', dW2 = H1^T dH2 (the D layout of 16 rows is
+    // the A / B layout of a product over them) ----
+    bf16x4 d2[4];
+    wave_sync();  // H1 was read
+    for (int cb = 0; cb < 4; cb++) {
+      const float w3 = w.w3[cb * 16 + r];
+      for (int j = 0; j < 4; j++) {
+        const float d = h2[cb][j] > 0.f ? dy[j] * w3 : 0.f;
+        gb2[cb] += d;
+        d2[cb][j] = f2bf(d);
+        H[(4 * kb + j) * H1_STRIDE + cb * 16 + r] = d2[cb][j];
       }
-      for (int j = 0; j < 4; j++) z[j] = f.h1[cb][j] > 0.f ? z[j] : 0.f;
-      dh1[cb] = z;
     }
-    __syncthreads();
-    // dW1 = X^T dH1: A = X^T (lane l: feature l%16, samples 4kb+j), B = dH1 (D layout)
+    for (int mb = 0; mb < 4; mb++)
+      for (int nb = 0; nb < 4; nb++) g2[mb][nb] = mfma(a1[mb], d2[nb], g2[mb][nb]);
+    wave_sync();
+    // ---- dH1 = dH2 W2^T (.) relu', dW1 = X^T dH1 ----
     bf16x4 ax;
     for (int j = 0; j < 4; j++) {
-      int row = row0 + 4 * kb + j;
+      const int row = row0 + 4 * kb + j;
       ax[j] = row < n ? f2bf(X[(size_t)row * MLP_IN + r]) : (short)0;
     }
-    for (int nb = 0; nb < 4; nb++) {
+    for (int cb = 0; cb < 4; cb++) {
+      floatx4 z = zero;
+      for (int kk = 0; kk < 2; kk++) {
+        const shortx8 a2 =
+            *reinterpret_cast<const shortx8 *>(&H[r * H1_STRIDE + kk * 32 + 8 * kb]);
+        const shortx8 b2v = *reinterpret_cast<const shortx8 *>(
+            &w2n[(cb * 16 + r) * W2T_STRIDE + kk * 32 + 8 * kb]);
+        z = mfma32(a2, b2v, z);
+      }
       bf16x4 b;
-      for (int j = 0; j < 4; j++) b[j] = f2bf(dh1[nb][j]);
-      floatx4 z = {0.f, 0.f, 0.f, 0.f};
-      z = mfma(ax, b, z);  // rows: feature 4kb+j, col: hidden1 nb*16 + r
-      for (int j = 0; j < 4; j++)
-        atomicAdd(&gsh[OFF_W1 + (4 * kb + j) * MLP_H + nb * 16 + r], z[j]);
-      float s = dh1[nb][0] + dh1[nb][1] + dh1[nb][2] + dh1[nb][3];
-      atomicAdd(&gsh[OFF_B1 + nb * 16 + r], s);
+      for (int j = 0; j < 4; j++) {
+        const float d = h1[cb][j] > 0.f ? z[j] : 0.f;
+        gb1[cb] += d;
+        b[j] = f2bf(d);
+      }
+      g1[cb] = mfma(ax, b, g1[cb]);
     }
-    __syncthreads();
+    wave_sync();  // H is rewritten by the next rows
   }
-  __syncthreads();
-  for (int k = l; k < MLP_NPARAM; k += 64)
-    if (gsh[k] != 0.f) atomicAdd(&G[k], gsh[k]);
+  // ---- the block's sum ----
+  for (int cb = 0; cb < 4; cb++) {
+    for (int j = 0; j < 4; j++) {
+      atomicAdd(&gsh[OFF_W1 + (4 * kb + j) * MLP_H + cb * 16 + r], g1[cb][j]);
+      for (int mb = 0; mb < 4; mb++)
+        atomicAdd(&gsh[OFF_W2 + (mb * 16 + 4 * kb + j) * MLP_H + cb * 16 + r], g2[mb][cb][j]);
+    }
+    atomicAdd(&gsh[OFF_B1 + cb * 16 + r], gb1[cb]);
+    atomicAdd(&gsh[OFF_B2 + cb * 16 + r], gb2[cb]);
+    atomicAdd(&gsh[OFF_W3 + cb * 16 + r], gw3[cb]);
+  }
+  if (r == 0) atomicAdd(&gsh[OFF_B3], gb3);
   for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off, 64);
   if (l == 0) atomicAdd(loss, lsum);
+  __syncthreads();
+  for (int k = tid; k < MLP_NPARAM; k += 64 * GRAD_WAVES)
+    if (gsh[k] != 0.f) atomicAdd(&G[k], gsh[k]);
+}
+
+// Blocks of the gradient kernel for n > 0 rows.
+static int grad_blocks(int n) {
+  return std::min((n + 16 * GRAD_WAVES - 1) / (16 * GRAD_WAVES), GRAD_BLOCKS);
 }
 
 // Adam step on the FP32 master weights.
@@ -345,8 +317,7 @@ int gcdt_mlp_grad(const float *X, const float *t, int n, const float *params,
     hc(hipMemcpy(dP, params, sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice), "copy");
     hc(hipMemset(dG, 0, sizeof(float) * MLP_NPARAM), "memset");
     hc(hipMemset(dl, 0, sizeof(float)), "memset");
-    int blocks = std::min((n + 15) / 16, 1024);
-    if (blocks > 0) k_mlp_grad<<<blocks, 64>>>(dX, dt, n, dP, dG, dl);
+    if (n > 0) k_mlp_grad<<<grad_blocks(n), 64 * GRAD_WAVES>>>(dX, dt, n, dP, dG, dl);
     hc(hipGetLastError(), "launch");
     hc(hipDeviceSynchronize(), "sync");
     hc(hipMemcpy(grad, dG, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost), "copy");
@@ -405,7 +376,8 @@ int gcdt_mlp_train(const float *X, const float *t, int n, int epochs, int batch,
       for (int b0 = 0; b0 < n; b0 += batch) {
         int nb = std::min(batch, n - b0);
         hc(hipMemset(dG, 0, sizeof(float) * MLP_NPARAM), "memset");
-        k_mlp_grad<<<std::min((nb + 15) / 16, 256), 64>>>(dX + (size_t)b0 * MLP_IN, dt + b0, nb, dP, dG, dl);
+        k_mlp_grad<<<grad_blocks(nb), 64 * GRAD_WAVES>>>(dX + (size_t)b0 * MLP_IN, dt + b0, nb, dP,
+                                                         dG, dl);
         step++;
         k_adam<<<(MLP_NPARAM + 255) / 256, 256>>>(dP, dG, dm1, dm2, MLP_NPARAM, lr, 0.9f, 0.999f, 1e-8f, step);
       }
