@@ -202,6 +202,19 @@ struct PassD {
   int lshift;
 };
 
+// Vertex deletion step of a pass.
+struct DelD {
+  const int *ids;  // subsegment candidates of the pass
+  int nseg;        // host loop: their number (graph loop: from ctl)
+  Ctl *ctl;
+  unsigned long long epoch;  // host loop: the claim epoch
+  int policy;                // 1: Chew-mode instances only, 2: every instance
+  int *ws, *dv, *dk;
+  double *pws;               // exact-predicate arena, one slot per lane
+  unsigned long long *cnt;
+  int use_fp32;
+};
+
 // State of the host loop that k_small_rounds carries from pass to pass, and
 // hands back.
 enum : int {
@@ -231,6 +244,7 @@ struct SmallArgs {
   const float *mlp;  // priority network (nullptr: none)
   int lshift, mix_below, cap, cand_factor, cand_min, kmax, seg_iters, bad_iters, max_rounds;
   int del_on;
+  DelD del;
   long long capP, capT, capS;
   SmallOut *out;  // mapped host memory
 };

@@ -32,8 +32,6 @@ struct MeshHost {
 };
 
 // One device-resident input CDT (a single mesh, or the union of a batch).
-struct DelD;  // vertex deletion step of a pass (gcdt_refine.hip)
-
 struct InputSet {
   int np = 0, nt = 0, ns = 0, n_inst = 0;
   int capP = 0, capT = 0, capS = 0;  // allocated sizes (reuse on upload)

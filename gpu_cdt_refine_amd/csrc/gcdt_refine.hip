@@ -1575,332 +1575,6 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_rank_apply(MeshD m, ParamsD pr, 
 }
 
 // ---------------------------------------------------------------------------
-// Small passes: whole rounds in one launch of one block.
-//
-// A pass over few candidates is a chain of 8 to 16 dependent launches (about
-// 4 us each for almost no work) and a host round trip.  Here one block of 16
-// waves runs the same steps with block barriers between them, pass after
-// pass, while every pass has at most SR_CAP candidates.  Steps and order are
-// the separate kernels' (the same device functions), so the mesh is the same
-// bit for bit.  Per-candidate arrays and the lists live in LDS; the
-// encroached subsegments and the triangles to test are listed as they change,
-// so no step scans the mesh.  The block returns to the host, at a pass
-// boundary, when a pass is larger, needs more mesh capacity, a list overflows
-// or the refinement ends; and inside a pass, after the cavities, when a
-// candidate needs the exact-predicate kernel, which the host then launches
-// (Refiner::run_pass with that pass to resume).
-// Bound by the chain of gathers and LDS round trips of the cavities (about half
-// of a pass), on one CU.  A pass of a 300-point refinement takes 50 us, where
-// its launches took 85 to 110 with the round trip.  8 waves with 256 registers:
-// 41,003 points 22.1 ms a call, 22.8 with 16 waves and spills.  SR_CAP: a few
-// batches of cavities on the one CU still cost less than the launches saved.
-// ---------------------------------------------------------------------------
-constexpr int SR_WAVES = 8, SR_THREADS = 64 * SR_WAVES;
-constexpr int SR_LG = 16;        // lanes per cavity
-constexpr int SR_K = 32;         // largest cavity held in LDS
-constexpr int SR_CAP = 256;      // candidates of a pass
-constexpr int SR_ENC = 512;      // encroached subsegments listed
-constexpr int SR_DIRTY = 8192;   // rewritten triangles listed between two bad passes
-constexpr int SR_PASSES = 128;   // passes of one launch
-static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
-
-// The lists k_small_rounds keeps as passes change the mesh.
-struct ListTrace {
-  int *enc, *n_enc;      // LDS
-  int *dirty, *n_dirty;  // global list, LDS count
-  unsigned *cnt;         // LDS counters of the pass
-  int nt;                // slots from here on are new
-  bool track;            // the bad list is known: list what changes
-  __device__ void encroached(int s) const {
-    const int p = atomicAdd(n_enc, 1);
-    if (p < SR_ENC) enc[p] = s;
-  }
-  // once per slot between two marking passes: the first rewrite finds the
-  // check flag clear (a new slot's flags are not initialised)
-  __device__ void rewritten(const MeshD &m, int t) const {
-    if (track && (t >= nt || !(m.tflag[t] & TF_CHECK))) {
-      const int p = atomicAdd(n_dirty, 1);
-      if (p < SR_DIRTY) dirty[p] = t;
-    }
-  }
-  __device__ void seg_winners(const PassD &, unsigned n) const { atomicAdd(&cnt[CNT_SEGWIN], n); }
-};
-
-// Ascending order of the n distinct values in src (LDS, n <= SR_THREADS), to
-// dst: each thread counts the smaller values.  The caller synchronises.
-__device__ __forceinline__ void rank_sort(const int *src, int n, int *dst) {
-  if ((int)threadIdx.x < n) {
-    const int v = src[threadIdx.x];
-    int r = 0;
-    for (int x = 0; x < n; x++) r += src[x] < v;
-    dst[r] = v;
-  }
-}
-
-__global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr, PassD base,
-                                                             SmallArgs a) {
-  // the cavities' LDS; between them the network's and the sorts'
-  extern __shared__ __align__(16) int sm[];
-  __shared__ int s_enc[SR_ENC], s_bad[SR_CAP], s_ids[SR_CAP];
-  __shared__ double2 s_pt[SR_CAP];
-  __shared__ double s_near[SR_CAP];
-  __shared__ int2 s_seed[SR_CAP];
-  __shared__ int s_status[SR_CAP], s_n[SR_CAP], s_r[SR_CAP], s_prio[SR_CAP], s_win[SR_CAP],
-      s_rank[SR_CAP], s_act[SR_CAP];
-  __shared__ unsigned s_cnt[CNT_N], s_slow[2];
-  __shared__ unsigned long long s_acc[CNT_N];
-  __shared__ int s_wave[SR_WAVES];
-  __shared__ int s_ne, s_nd, s_k;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  // uniform state
-  SmallState st = a.st;
-  bool known = st.nb >= 0;
-  int nb = known ? st.nb : 0;
-  int code = SR_BOUNDARY, stage = 0, nc = 0, nseg = 0, passes = 0;
-  if (tid < st.ne) s_enc[tid] = a.enc[tid];
-  if (tid < nb) s_bad[tid] = a.bad[tid];
-  if (tid < CNT_N) {
-    s_cnt[tid] = 0u;
-    s_acc[tid] = 0ull;
-  }
-  if (tid == 0) {
-    s_ne = st.ne;
-    s_nd = 0;
-    s_slow[0] = s_slow[1] = 0u;
-  }
-  __syncthreads();
-  for (; passes < SR_PASSES; passes++) {
-    nseg = st.ne;
-    int nbc = 0;
-    const bool seg_pass = st.ne > a.mix_below;
-    if (!seg_pass) {
-      // ---- bad triangles: the old list's survivors and the rewritten ones ----
-      const int nd = s_nd;
-      if (!known || nd > SR_DIRTY) break;
-      const int t0 = tid < nb ? s_bad[tid] : -1;
-      const uint8_t f0 = t0 >= 0 ? m.tflag[t0] : 0;
-      if (tid == 0) s_k = 0;
-      __syncthreads();
-      if ((f0 & (TF_ALIVE | TF_BAD | TF_GIVEUP | TF_CHECK)) == (TF_ALIVE | TF_BAD))
-        sm[atomicAdd(&s_k, 1)] = t0;
-      for (int q = tid; q < nd; q += SR_THREADS) {
-        const int t = a.dirty[q];
-        const uint8_t f = mark_bad_one(m, pr, t, m.tflag[t]);
-        if ((f & (TF_ALIVE | TF_BAD | TF_GIVEUP)) == (TF_ALIVE | TF_BAD)) {
-          const int p = atomicAdd(&s_k, 1);
-          if (p < 2 * SR_CAP) sm[p] = t;
-        }
-      }
-      __syncthreads();
-      nb = s_k;
-      if (nb > SR_CAP) {
-        known = false;
-        break;
-      }
-      rank_sort(sm, nb, s_bad);
-      if (tid == 0) s_nd = 0;
-      __syncthreads();
-      if (st.ne == 0 && nb == 0) {
-        code = SR_DONE;
-        st.status = 0;
-        break;
-      }
-      long long capb = (long long)a.cap - st.ne;
-      if (a.cand_factor > 0 && st.prev_win >= 0)
-        capb = min(capb, max((long long)a.cand_min, (long long)a.cand_factor * st.prev_win));
-      if (nb > capb) break;  // needs the selection by priority
-      nbc = nb;
-    }
-    nc = nseg + nbc;
-    const int iters = nbc == 0 ? a.seg_iters : a.bad_iters;
-    if (nc > SR_CAP || nc > a.cap || (a.del_on && nseg > 0) ||
-        st.epoch + iters + 3 >= (1 << 11) || st.np + (long long)nc > a.capP ||
-        st.nt + 2ll * nc > a.capT || st.ns + (long long)nseg > a.capS)
-      break;
-    if (tid < nseg) s_ids[tid] = s_enc[tid];
-    if (tid < nbc) s_ids[nseg + tid] = s_bad[tid];
-    PassD ps = base;
-    ps.ids = s_ids;
-    ps.nc = nc;
-    ps.nseg = nseg;
-    ps.iters = iters;
-    ps.epoch0 = ps.epoch = (unsigned long long)st.epoch + 1ull;
-    ps.iter = 0;
-    ps.cpt = s_pt;
-    ps.cstatus = s_status;
-    ps.cn = s_n;
-    ps.cr = s_r;
-    ps.cprio = s_prio;
-    ps.cwin = s_win;
-    ps.crank = s_rank;
-    ps.cseed = s_seed;
-    ps.cnear = s_near;
-    ps.feat = nbc > 0 ? a.feat : nullptr;
-    ps.pass_index = st.pass_index;
-    const ListTrace trace{s_enc, &s_ne, a.dirty, &s_nd, s_cnt, st.nt, known};
-    __syncthreads();
-    // ---- cavities ----
-    int *cav = sm + wave * (64 / SR_LG) * group_lds_ints(min(ps.K, ps.Kf), SR_LG);
-    if (nseg > 0) {
-      CavCounts cc(s_cnt, &s_slow[0]);
-      if (tid < nseg) locate_one<true>(m, pr, ps, tid, s_ids[tid], cc, trace);
-      __syncthreads();
-      cavity_wave<true, SR_LG, true, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
-      cc.settle(true);
-      __syncthreads();
-      if (s_slow[0] != 0u) {
-        code = SR_SLOW;
-        stage = 1;
-        break;
-      }
-    }
-    if (nbc > 0) {
-      CavCounts cc(s_cnt, &s_slow[1]);
-      if (tid < nbc) locate_one<false>(m, pr, ps, nseg + tid, s_ids[nseg + tid], cc, trace);
-      __syncthreads();
-      cavity_wave<false, SR_LG, true, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
-      cc.settle(false);
-      __syncthreads();
-      if (s_slow[1] != 0u) {
-        code = SR_SLOW;
-        stage = 2;
-        break;
-      }
-      if (a.mlp) {
-        MlpWeights &w = *reinterpret_cast<MlpWeights *>(sm);
-        short *H = reinterpret_cast<short *>(sm) + sizeof(MlpWeights) / sizeof(short) +
-                   wave * 16 * H1_STRIDE;
-        mlp_stage<SR_THREADS>(a.mlp, w, tid);
-        __syncthreads();
-        for (int row0 = wave * 16; row0 < nbc; row0 += SR_WAVES * 16) {
-          mlp_rows16(a.feat + (size_t)nseg * FEAT, nbc, row0, w, H, a.score + nseg);
-          wave_sync();
-        }
-        ps.score = a.score;
-        ps.lshift = a.lshift;
-        __syncthreads();
-      }
-    }
-    // ---- claims ----
-    unsigned ws_seg = 0, ws_bad = 0;
-    for (int it = 0; it < iters; it++) {
-      ps.epoch = (unsigned long long)++st.epoch;
-      ps.iter = it;
-      claim_body<CLAIM_LANES>(m, ps, s_act, tid, SR_THREADS, ws_seg, ws_bad);
-      __syncthreads();
-      win_body<CLAIM_LANES>(m, ps, s_act, tid, SR_THREADS);
-      __syncthreads();
-    }
-    ++st.epoch;  // the winners' stamp epoch
-    if (ws_seg) atomicAdd(&s_cnt[CNT_WS_SEG], ws_seg);
-    if (ws_bad) atomicAdd(&s_cnt[CNT_WS_BAD], ws_bad);
-    // ---- ranks and apply ----
-    const bool win = tid < nc && s_win[tid] != 0;
-    const unsigned long long wb = __ballot(win);
-    if (lane == 0) s_wave[wave] = __popcll(wb);
-    __syncthreads();
-    int before = 0, nwin = 0;
-    for (int w = 0; w < SR_WAVES; w++) {
-      const int c = s_wave[w];
-      if (w < wave) before += c;
-      nwin += c;
-    }
-    if (win) s_rank[tid] = before + __popcll(wb & ((1ull << lane) - 1ull));
-    __syncthreads();
-    unsigned long long nflip = 0;
-    for (int i = tid / APPLY_LANES; i < nc; i += SR_THREADS / APPLY_LANES)
-      apply_one<APPLY_LANES>(m, pr, ps, i, tid % APPLY_LANES, nseg, s_ids, st.np, st.nt, st.ns,
-                             nflip, trace);
-    if (nflip) atomicAdd(&s_cnt[CNT_FLIPS], (unsigned)nflip);
-    if (tid == 0) s_cnt[CNT_NWIN] = (unsigned)nwin;
-    __syncthreads();
-    // ---- what the pass did ----
-    const int nws = (int)s_cnt[CNT_SEGWIN], listed = s_ne;
-    const bool ovf = s_cnt[CNT_OVERFLOW] > 0;
-    long long prog = (long long)nwin + s_cnt[CNT_MARKS] + s_cnt[CNT_GIVEUPS];
-    st.np += nwin;
-    st.nt += 2 * nwin;
-    st.ns += nws;
-    const int es = tid < min(listed, SR_ENC) ? s_enc[tid] : -1;
-    const bool still = es >= 0 && __hip_atomic_load(&m.senc[es], __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT) == 1;
-    if (tid == 0) s_k = 0;
-    __syncthreads();
-    if (still) sm[atomicAdd(&s_k, 1)] = es;
-    if (tid < CNT_N) {
-      s_acc[tid] += s_cnt[tid];
-      s_cnt[tid] = 0u;
-    }
-    __syncthreads();
-    st.ne = s_k;
-    rank_sort(sm, st.ne, s_enc);
-    if (tid == 0) s_ne = st.ne;
-    __syncthreads();
-    if (listed > SR_ENC) st.ne = -1;
-    const bool grow = ovf && base.K < a.kmax;
-    if (seg_pass) {
-      st.seg_passes++;
-    } else {
-      if (nseg > 0) st.seg_passes++;
-      if (nbc > 0) {
-        st.pass_index++;
-        st.bad_passes++;
-        st.cand_evals += nbc;
-        st.prev_win = nwin - nws;
-      }
-      if (grow) prog++;
-      if (prog == 0) {
-        code = SR_DONE;
-        st.status = 2;
-        passes++;
-        break;
-      }
-      st.round++;
-      if (st.round >= a.max_rounds) {
-        code = SR_ROUNDS;
-        passes++;
-        break;
-      }
-      st.np_round = st.np;
-    }
-    st.grow = grow ? 1 : 0;
-    if (grow || st.ne < 0) {
-      passes++;
-      break;
-    }
-  }
-  // ---- back to the host ----
-  __syncthreads();
-  if (code == SR_SLOW) {  // this pass's candidates and counts, for the separate kernels
-    if (tid < nc) {
-      a.ids_out[tid] = s_ids[tid];
-      base.cpt[tid] = s_pt[tid];
-      base.cstatus[tid] = s_status[tid];
-      base.cn[tid] = s_n[tid];
-      base.cr[tid] = s_r[tid];
-      base.cprio[tid] = s_prio[tid];
-    }
-    if (tid < CNT_N && tid != CNT_SLOW) base.cnt[tid] = s_cnt[tid];
-  } else if (tid < st.ne) {
-    a.enc_out[tid] = s_enc[tid];
-  }
-  if (tid < CNT_N)
-    __hip_atomic_store(&a.out->acc[tid], s_acc[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  if (tid == 0) {
-    st.code = code;
-    st.stage = stage;
-    st.nc = nc;
-    st.nseg = nseg;
-    st.passes = passes;
-    const int *src = reinterpret_cast<const int *>(&st);
-    int *dst = reinterpret_cast<int *>(&a.out->st);
-    for (int k = 0; k < (int)(sizeof(SmallState) / sizeof(int)); k++)
-      __hip_atomic_store(dst + k, src[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
-  __threadfence_system();
-}
-
-// ---------------------------------------------------------------------------
 // Vertex deletion (Chew's rule as Triangle applies it before splitting an
 // encroached subsegment, triangle.cpp:13319-13357; the reference marks the
 // same vertices and removes them by flips, refine.cu:604-677, 778-1070).
@@ -1921,18 +1595,6 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
 // strictly inside (exact signs); the cut triangles are the constrained
 // Delaunay triangles inside the star once the vertex is gone.
 // ---------------------------------------------------------------------------
-
-struct DelD {
-  const int *ids;  // subsegment candidates of the pass
-  int nseg;        // host loop: their number (graph loop: from ctl)
-  Ctl *ctl;
-  unsigned long long epoch;  // host loop: the claim epoch
-  int policy;                // 1: Chew-mode instances only, 2: every instance
-  int *ws, *dv, *dk;
-  double *pws;               // exact-predicate arena, one slot per lane
-  unsigned long long *cnt;
-  int use_fp32;
-};
 
 __device__ __forceinline__ int del_nseg(const DelD &d) {
   const int n = d.ctl ? (d.ctl->i[C_GO] ? d.ctl->i[C_NC] : 0) : d.nseg;
@@ -2217,6 +1879,357 @@ __global__ __launch_bounds__(DEL_BLOCK) void k_del_apply(MeshD m, DelD dd) {
     if (ndel) atomicAdd(&dd.cnt[CNT_DEL], ndel);
     if (nflip) atomicAdd(&dd.cnt[CNT_FLIPS], nflip);
   }
+}
+
+// ---------------------------------------------------------------------------
+// Small passes: whole rounds in one launch of one block.
+//
+// A pass over few candidates is a chain of 8 to 16 dependent launches (about
+// 4 us each for almost no work) and a host round trip.  Here one block of 16
+// waves runs the same steps with block barriers between them, pass after
+// pass, while every pass has at most SR_CAP candidates.  Steps and order are
+// the separate kernels' (the same device functions), so the mesh is the same
+// bit for bit.  Per-candidate arrays and the lists live in LDS; the
+// encroached subsegments and the triangles to test are listed as they change,
+// so no step scans the mesh.  The block returns to the host, at a pass
+// boundary, when a pass is larger, needs more mesh capacity, a list overflows
+// or the refinement ends; and inside a pass, after the cavities, when a
+// candidate needs the exact-predicate kernel, which the host then launches
+// (Refiner::run_pass with that pass to resume).
+// Bound by the chain of gathers and LDS round trips of the cavities (about half
+// of a pass), on one CU.  A pass of a 300-point refinement takes 50 us, where
+// its launches took 85 to 110 with the round trip.  8 waves with 256 registers:
+// 41,003 points 22.1 ms a call, 22.8 with 16 waves and spills.  SR_CAP: a few
+// batches of cavities on the one CU still cost less than the launches saved.
+// ---------------------------------------------------------------------------
+constexpr int SR_WAVES = 8, SR_THREADS = 64 * SR_WAVES;
+constexpr int SR_LG = 16;        // lanes per cavity
+constexpr int SR_K = 32;         // largest cavity held in LDS
+constexpr int SR_CAP = 256;      // candidates of a pass
+// subsegments of a pass that deletes vertices: 32 groups of lanes serve their
+// 2 nominations each, 4 rounds of walks around a vertex (2,999 points in Chew
+// mode 12.1 ms a call with no such limit, 11.1 with 64, 10.9 to 11.1 with 32)
+constexpr int SR_DEL = 64;
+constexpr int SR_ENC = 512;      // encroached subsegments listed
+constexpr int SR_DIRTY = 8192;   // rewritten triangles listed between two bad passes
+constexpr int SR_PASSES = 128;   // passes of one launch
+static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
+
+// The lists k_small_rounds keeps as passes change the mesh.
+struct ListTrace {
+  int *enc, *n_enc;      // LDS
+  int *dirty, *n_dirty;  // global list, LDS count
+  unsigned *cnt;         // LDS counters of the pass
+  int nt;                // slots from here on are new
+  bool track;            // the bad list is known: list what changes
+  __device__ void encroached(int s) const {
+    const int p = atomicAdd(n_enc, 1);
+    if (p < SR_ENC) enc[p] = s;
+  }
+  // once per slot between two marking passes: the first rewrite finds the
+  // check flag clear (a new slot's flags are not initialised)
+  __device__ void rewritten(const MeshD &m, int t) const {
+    if (track && (t >= nt || !(m.tflag[t] & TF_CHECK))) {
+      const int p = atomicAdd(n_dirty, 1);
+      if (p < SR_DIRTY) dirty[p] = t;
+    }
+  }
+  __device__ void seg_winners(const PassD &, unsigned n) const { atomicAdd(&cnt[CNT_SEGWIN], n); }
+};
+
+// Ascending order of the n distinct values in src (LDS, n <= SR_THREADS), to
+// dst: each thread counts the smaller values.  The caller synchronises.
+__device__ __forceinline__ void rank_sort(const int *src, int n, int *dst) {
+  if ((int)threadIdx.x < n) {
+    const int v = src[threadIdx.x];
+    int r = 0;
+    for (int x = 0; x < n; x++) r += src[x] < v;
+    dst[r] = v;
+  }
+}
+
+__global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr, PassD base,
+                                                             SmallArgs a) {
+  // the cavities' LDS; between them the network's and the sorts'
+  extern __shared__ __align__(16) int sm[];
+  __shared__ int s_enc[SR_ENC], s_bad[SR_CAP], s_ids[SR_CAP];
+  __shared__ double2 s_pt[SR_CAP];
+  __shared__ double s_near[SR_CAP];
+  __shared__ int2 s_seed[SR_CAP];
+  __shared__ int s_status[SR_CAP], s_n[SR_CAP], s_r[SR_CAP], s_prio[SR_CAP], s_win[SR_CAP],
+      s_rank[SR_CAP], s_act[SR_CAP];
+  __shared__ unsigned s_cnt[CNT_N], s_slow[2];
+  __shared__ unsigned long long s_acc[CNT_N];
+  __shared__ int s_wave[SR_WAVES];
+  __shared__ int s_ne, s_nd, s_k;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  // uniform state
+  SmallState st = a.st;
+  bool known = st.nb >= 0;
+  int nb = known ? st.nb : 0;
+  int code = SR_BOUNDARY, stage = 0, nc = 0, nseg = 0, passes = 0;
+  if (tid < st.ne) s_enc[tid] = a.enc[tid];
+  if (tid < nb) s_bad[tid] = a.bad[tid];
+  if (tid < CNT_N) {
+    s_cnt[tid] = 0u;
+    s_acc[tid] = 0ull;
+  }
+  if (tid == 0) {
+    s_ne = st.ne;
+    s_nd = 0;
+    s_slow[0] = s_slow[1] = 0u;
+  }
+  __syncthreads();
+  for (; passes < SR_PASSES; passes++) {
+    nseg = st.ne;
+    int nbc = 0;
+    const bool seg_pass = st.ne > a.mix_below;
+    if (!seg_pass) {
+      // ---- bad triangles: the old list's survivors and the rewritten ones ----
+      const int nd = s_nd;
+      if (!known || nd > SR_DIRTY) break;
+      const int t0 = tid < nb ? s_bad[tid] : -1;
+      const uint8_t f0 = t0 >= 0 ? m.tflag[t0] : 0;
+      if (tid == 0) s_k = 0;
+      __syncthreads();
+      if ((f0 & (TF_ALIVE | TF_BAD | TF_GIVEUP | TF_CHECK)) == (TF_ALIVE | TF_BAD))
+        sm[atomicAdd(&s_k, 1)] = t0;
+      for (int q = tid; q < nd; q += SR_THREADS) {
+        const int t = a.dirty[q];
+        const uint8_t f = mark_bad_one(m, pr, t, m.tflag[t]);
+        if ((f & (TF_ALIVE | TF_BAD | TF_GIVEUP)) == (TF_ALIVE | TF_BAD)) {
+          const int p = atomicAdd(&s_k, 1);
+          if (p < 2 * SR_CAP) sm[p] = t;
+        }
+      }
+      __syncthreads();
+      nb = s_k;
+      if (nb > SR_CAP) {
+        known = false;
+        break;
+      }
+      rank_sort(sm, nb, s_bad);
+      if (tid == 0) s_nd = 0;
+      __syncthreads();
+      if (st.ne == 0 && nb == 0) {
+        code = SR_DONE;
+        st.status = 0;
+        break;
+      }
+      long long capb = (long long)a.cap - st.ne;
+      if (a.cand_factor > 0 && st.prev_win >= 0)
+        capb = min(capb, max((long long)a.cand_min, (long long)a.cand_factor * st.prev_win));
+      if (nb > capb) break;  // needs the selection by priority
+      nbc = nb;
+    }
+    nc = nseg + nbc;
+    const int iters = nbc == 0 ? a.seg_iters : a.bad_iters;
+    if (nc > SR_CAP || (a.del_on && nseg > SR_DEL) || nc > a.cap || st.epoch + iters + 3 >= (1 << 11) || st.np + (long long)nc > a.capP ||
+        st.nt + 2ll * nc > a.capT || st.ns + (long long)nseg > a.capS)
+      break;
+    if (tid < nseg) s_ids[tid] = s_enc[tid];
+    if (tid < nbc) s_ids[nseg + tid] = s_bad[tid];
+    PassD ps = base;
+    ps.ids = s_ids;
+    ps.nc = nc;
+    ps.nseg = nseg;
+    ps.iters = iters;
+    ps.iter = 0;
+    ps.cpt = s_pt;
+    ps.cstatus = s_status;
+    ps.cn = s_n;
+    ps.cr = s_r;
+    ps.cprio = s_prio;
+    ps.cwin = s_win;
+    ps.crank = s_rank;
+    ps.cseed = s_seed;
+    ps.cnear = s_near;
+    ps.feat = nbc > 0 ? a.feat : nullptr;
+    ps.pass_index = st.pass_index;
+    const ListTrace trace{s_enc, &s_ne, a.dirty, &s_nd, s_cnt, st.nt, known};
+    __syncthreads();
+    // ---- vertex deletion, with a claim epoch of its own ----
+    if (a.del_on && nseg > 0) {
+      DelD dd = a.del;
+      dd.ids = s_ids;
+      const unsigned long long ep = (unsigned long long)++st.epoch;
+      const int grp = tid / DEL_G, gl = tid % DEL_G;
+      int *lds = sm + grp * DEL_LDS_INTS;
+      for (int d = grp; d < 2 * nseg; d += SR_THREADS / DEL_G) {
+        del_scan_one(m, pr, dd, d, ep, dd.pws + (size_t)tid * GCDT_INCIRCLE_WS, lds, gl);
+        wave_sync();
+      }
+      __syncthreads();
+      for (int d = grp; d < 2 * nseg; d += SR_THREADS / DEL_G) {
+        const int k = del_apply_one(m, dd, d, ep, lds, gl, trace);
+        if (k > 0 && gl == 0) {
+          atomicAdd(&s_cnt[CNT_DEL], 1u);
+          atomicAdd(&s_cnt[CNT_FLIPS], (unsigned)(k - 3));
+        }
+        wave_sync();
+      }
+      __syncthreads();
+    }
+    ps.epoch0 = ps.epoch = (unsigned long long)st.epoch + 1ull;
+    // ---- cavities ----
+    int *cav = sm + wave * (64 / SR_LG) * group_lds_ints(min(ps.K, ps.Kf), SR_LG);
+    if (nseg > 0) {
+      CavCounts cc(s_cnt, &s_slow[0]);
+      if (tid < nseg) locate_one<true>(m, pr, ps, tid, s_ids[tid], cc, trace);
+      __syncthreads();
+      cavity_wave<true, SR_LG, true, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
+      cc.settle(true);
+      __syncthreads();
+      if (s_slow[0] != 0u) {
+        code = SR_SLOW;
+        stage = 1;
+        break;
+      }
+    }
+    if (nbc > 0) {
+      CavCounts cc(s_cnt, &s_slow[1]);
+      if (tid < nbc) locate_one<false>(m, pr, ps, nseg + tid, s_ids[nseg + tid], cc, trace);
+      __syncthreads();
+      cavity_wave<false, SR_LG, true, true>(m, pr, ps, a.kmax, wave, SR_WAVES, cav, cc, trace);
+      cc.settle(false);
+      __syncthreads();
+      if (s_slow[1] != 0u) {
+        code = SR_SLOW;
+        stage = 2;
+        break;
+      }
+      if (a.mlp) {
+        MlpWeights &w = *reinterpret_cast<MlpWeights *>(sm);
+        short *H = reinterpret_cast<short *>(sm) + sizeof(MlpWeights) / sizeof(short) +
+                   wave * 16 * H1_STRIDE;
+        mlp_stage<SR_THREADS>(a.mlp, w, tid);
+        __syncthreads();
+        for (int row0 = wave * 16; row0 < nbc; row0 += SR_WAVES * 16) {
+          mlp_rows16(a.feat + (size_t)nseg * FEAT, nbc, row0, w, H, a.score + nseg);
+          wave_sync();
+        }
+        ps.score = a.score;
+        ps.lshift = a.lshift;
+        __syncthreads();
+      }
+    }
+    // ---- claims ----
+    unsigned ws_seg = 0, ws_bad = 0;
+    for (int it = 0; it < iters; it++) {
+      ps.epoch = (unsigned long long)++st.epoch;
+      ps.iter = it;
+      claim_body<CLAIM_LANES>(m, ps, s_act, tid, SR_THREADS, ws_seg, ws_bad);
+      __syncthreads();
+      win_body<CLAIM_LANES>(m, ps, s_act, tid, SR_THREADS);
+      __syncthreads();
+    }
+    ++st.epoch;  // the winners' stamp epoch
+    if (ws_seg) atomicAdd(&s_cnt[CNT_WS_SEG], ws_seg);
+    if (ws_bad) atomicAdd(&s_cnt[CNT_WS_BAD], ws_bad);
+    // ---- ranks and apply ----
+    const bool win = tid < nc && s_win[tid] != 0;
+    const unsigned long long wb = __ballot(win);
+    if (lane == 0) s_wave[wave] = __popcll(wb);
+    __syncthreads();
+    int before = 0, nwin = 0;
+    for (int w = 0; w < SR_WAVES; w++) {
+      const int c = s_wave[w];
+      if (w < wave) before += c;
+      nwin += c;
+    }
+    if (win) s_rank[tid] = before + __popcll(wb & ((1ull << lane) - 1ull));
+    __syncthreads();
+    unsigned long long nflip = 0;
+    for (int i = tid / APPLY_LANES; i < nc; i += SR_THREADS / APPLY_LANES)
+      apply_one<APPLY_LANES>(m, pr, ps, i, tid % APPLY_LANES, nseg, s_ids, st.np, st.nt, st.ns,
+                             nflip, trace);
+    if (nflip) atomicAdd(&s_cnt[CNT_FLIPS], (unsigned)nflip);
+    if (tid == 0) s_cnt[CNT_NWIN] = (unsigned)nwin;
+    __syncthreads();
+    // ---- what the pass did ----
+    const int nws = (int)s_cnt[CNT_SEGWIN], listed = s_ne;
+    const bool ovf = s_cnt[CNT_OVERFLOW] > 0;
+    long long prog = (long long)nwin + s_cnt[CNT_DEL] + s_cnt[CNT_MARKS] + s_cnt[CNT_GIVEUPS];
+    st.np += nwin;
+    st.nt += 2 * nwin;
+    st.ns += nws;
+    const int es = tid < min(listed, SR_ENC) ? s_enc[tid] : -1;
+    const bool still = es >= 0 && __hip_atomic_load(&m.senc[es], __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT) == 1;
+    if (tid == 0) s_k = 0;
+    __syncthreads();
+    if (still) sm[atomicAdd(&s_k, 1)] = es;
+    if (tid < CNT_N) {
+      s_acc[tid] += s_cnt[tid];
+      s_cnt[tid] = 0u;
+    }
+    __syncthreads();
+    st.ne = s_k;
+    rank_sort(sm, st.ne, s_enc);
+    if (tid == 0) s_ne = st.ne;
+    __syncthreads();
+    if (listed > SR_ENC) st.ne = -1;
+    const bool grow = ovf && base.K < a.kmax;
+    if (seg_pass) {
+      st.seg_passes++;
+    } else {
+      if (nseg > 0) st.seg_passes++;
+      if (nbc > 0) {
+        st.pass_index++;
+        st.bad_passes++;
+        st.cand_evals += nbc;
+        st.prev_win = nwin - nws;
+      }
+      if (grow) prog++;
+      if (prog == 0) {
+        code = SR_DONE;
+        st.status = 2;
+        passes++;
+        break;
+      }
+      st.round++;
+      if (st.round >= a.max_rounds) {
+        code = SR_ROUNDS;
+        passes++;
+        break;
+      }
+      st.np_round = st.np;
+    }
+    st.grow = grow ? 1 : 0;
+    if (grow || st.ne < 0) {
+      passes++;
+      break;
+    }
+  }
+  // ---- back to the host ----
+  __syncthreads();
+  if (code == SR_SLOW) {  // this pass's candidates and counts, for the separate kernels
+    if (tid < nc) {
+      a.ids_out[tid] = s_ids[tid];
+      base.cpt[tid] = s_pt[tid];
+      base.cstatus[tid] = s_status[tid];
+      base.cn[tid] = s_n[tid];
+      base.cr[tid] = s_r[tid];
+      base.cprio[tid] = s_prio[tid];
+    }
+    if (tid < CNT_N && tid != CNT_SLOW) base.cnt[tid] = s_cnt[tid];
+  } else if (tid < st.ne) {
+    a.enc_out[tid] = s_enc[tid];
+  }
+  if (tid < CNT_N)
+    __hip_atomic_store(&a.out->acc[tid], s_acc[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (tid == 0) {
+    st.code = code;
+    st.stage = stage;
+    st.nc = nc;
+    st.nseg = nseg;
+    st.passes = passes;
+    const int *src = reinterpret_cast<const int *>(&st);
+    int *dst = reinterpret_cast<int *>(&a.out->st);
+    for (int k = 0; k < (int)(sizeof(SmallState) / sizeof(int)); k++)
+      __hip_atomic_store(dst + k, src[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  __threadfence_system();
 }
 
 // Export with deleted vertices: live points keep their order (input points
@@ -2702,8 +2715,9 @@ __global__ void k_dicut(const int *sel_tmp, Ctl *c) {
 // ===========================================================================
 // Dynamic LDS of k_small_rounds for cavities of up to K triangles.
 static size_t small_lds(int K) {
-  return std::max(sizeof(int) * (size_t)(SR_THREADS / SR_LG) * group_lds_ints(K, SR_LG),
-                  sizeof(MlpWeights) + sizeof(short) * SR_WAVES * 16 * H1_STRIDE);
+  return std::max({sizeof(int) * (size_t)(SR_THREADS / SR_LG) * group_lds_ints(K, SR_LG),
+                   sizeof(int) * (size_t)(SR_THREADS / DEL_G) * DEL_LDS_INTS,
+                   sizeof(MlpWeights) + sizeof(short) * SR_WAVES * 16 * H1_STRIDE});
 }
 
 static void hip_check(hipError_t e, const char *what) {
@@ -3561,10 +3575,9 @@ void Refiner::ensure_feat(int nc) {
 }
 
 // A pass of nc candidates, nseg of them subsegments, that k_small_rounds
-// takes.  Vertex deletion and the training logs need the separate kernels.
+// takes (the training logs need the separate kernels).
 bool Refiner::small_pass(int nc, int nseg) const {
-  return nc > 0 && nc <= SR_CAP && !opt.log_training && !(del_on && nseg > 0) &&
-         (opt.priority != 2 || mlp_params);
+  return nc > 0 && nc <= SR_CAP && !(del_on && nseg > SR_DEL) && !opt.log_training && (opt.priority != 2 || mlp_params);
 }
 
 // Rounds from the segment check on, while their passes are small: ne
@@ -3623,6 +3636,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   a.bad_iters = iters_for(false);
   a.max_rounds = opt.max_rounds;
   a.del_on = del_on ? 1 : 0;
+  a.del = del_base();
   a.capP = capP;
   a.capT = capT;
   a.capS = capS;
