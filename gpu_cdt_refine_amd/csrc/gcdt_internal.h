@@ -234,6 +234,7 @@ class Refiner {
   int *h_total = nullptr;       // pinned, host-coherent: compaction totals
   int *d_host_total = nullptr;  // its device address
   unsigned long long *d_cnt = nullptr;
+  unsigned long long *d_cntr = nullptr;  // the counters' copies (pass_cnt), zero between passes
   int *h_scalar = nullptr;
   unsigned long long *h_cnt = nullptr;
   unsigned long long *d_host_cnt = nullptr;  // h_cnt as the device sees it (mapped)

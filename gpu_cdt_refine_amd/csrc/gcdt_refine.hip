@@ -467,7 +467,8 @@ struct NoTrace {
   __device__ void encroached(int) const {}           // senc[s] went 0 -> 1
   __device__ void rewritten(const MeshD &, int) const {}  // slot about to be rewritten
   __device__ void seg_winners(const PassD &ps, unsigned n) const {
-    atomicAdd(&ps.cnt[CNT_SEGWIN], (unsigned long long)n);
+    // host loop: all winners of a pass without bad triangles (CNT_NWIN)
+    if (ps.ctl || ps.nseg < ps.nc) atomicAdd(&ps.cnt[CNT_SEGWIN], (unsigned long long)n);
   }
 };
 
@@ -1208,7 +1209,7 @@ __device__ __forceinline__ void cavity_body(const MeshD &m, const ParamsD &pr, c
   cavity_wave<IS_SEG, LG, FAST, LOCATED>(m, pr, ps, Kmax, (int)blockIdx.x, (int)gridDim.x, sm, cc,
                                          NoTrace{});
   cc.settle(IS_SEG);
-  add_block_counts(ps.cnt, s_cnt);
+  add_block_counts(pass_cnt(ps), s_cnt);
 }
 
 // The filtered kernel is held to 4 waves per SIMD (at most 128 VGPRs, no
@@ -1236,7 +1237,7 @@ __global__ __launch_bounds__(LOC_BLOCK) void k_locate(MeshD m, ParamsD pr, PassD
   CavCounts cc(s_cnt, &s_slow);
   if (w < n) locate_one<IS_SEG>(m, pr, ps, i, ps.ids[i], cc, NoTrace{});
   cc.settle(IS_SEG);
-  add_block_counts(ps.cnt, s_cnt);
+  add_block_counts(pass_cnt(ps), s_cnt);
 }
 
 // Claim key: higher wins.  Epoch in the top 11 bits makes older claims lose
@@ -1330,8 +1331,8 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_claim(MeshD m, PassD ps, int *ca
   if (ps.iter == 0) {
     const unsigned long long a = wave_sum(ws_seg), b = wave_sum(ws_bad);
     if ((threadIdx.x & 63) == 0) {
-      if (a) atomicAdd(&ps.cnt[CNT_WS_SEG], a);
-      if (b) atomicAdd(&ps.cnt[CNT_WS_BAD], b);
+      if (a) atomicAdd(&pass_cnt(ps)[CNT_WS_SEG], a);
+      if (b) atomicAdd(&pass_cnt(ps)[CNT_WS_BAD], b);
     }
   }
 }
@@ -1551,7 +1552,7 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_apply(MeshD m, ParamsD pr, PassD
   for (int i = blockIdx.x * per + threadIdx.x / G; i < nc; i += gridDim.x * per)
     apply_one<G>(m, pr, ps, i, gl, nseg, ids, pbase, tbase, sbase, nflip, NoTrace{});
   nflip = wave_sum(nflip);
-  if ((threadIdx.x & 63) == 0 && nflip) atomicAdd(&ps.cnt[CNT_FLIPS], nflip);
+  if ((threadIdx.x & 63) == 0 && nflip) atomicAdd(&pass_cnt(ps)[CNT_FLIPS], nflip);
 }
 
 // Small host-loop passes (nc <= SMALL_PASS): one block ranks the winners
@@ -1571,7 +1572,7 @@ __global__ __launch_bounds__(LIST_BLOCK) void k_rank_apply(MeshD m, ParamsD pr, 
   for (int i = threadIdx.x / G; i < nc; i += per)
     apply_one<G>(m, pr, ps, i, gl, ps.nseg, ps.ids, pbase, tbase, sbase, nflip, NoTrace{});
   nflip = wave_sum(nflip);
-  if ((threadIdx.x & 63) == 0 && nflip) atomicAdd(&ps.cnt[CNT_FLIPS], nflip);
+  if ((threadIdx.x & 63) == 0 && nflip) atomicAdd(&pass_cnt(ps)[CNT_FLIPS], nflip);
 }
 
 // ---------------------------------------------------------------------------
@@ -2785,6 +2786,8 @@ Refiner::Refiner(const gcdt_options &o) : opt(o) {
 
   dalloc(&d_total, 4);
   dalloc(&d_cnt, CNT_N);
+  dalloc(&d_cntr, (size_t)CNT_REP * CNT_STRIDE);
+  HC(hipMemset(d_cntr, 0, sizeof(unsigned long long) * CNT_REP * CNT_STRIDE));
   dalloc(&d_ctl, 1);
   dalloc(&g_cnt, GC);
   dalloc(&g_off, GC);
@@ -2830,7 +2833,7 @@ Refiner::~Refiner() {
   dfree(c_act); dfree(c_slow); dfree(c_seed); dfree(c_near); dfree(tmp_list); dfree(mix_list);
   dfree(sel_prio); dfree(sel_tmp); dfree(sel_list); dfree(d_hist);
   dfree(c_feat); dfree(c_score); dfree(c_deg); dfree(t_cnt); dfree(mlp_params);
-  dfree(cb_cnt); dfree(cb_off); dfree(d_total); dfree(d_cnt);
+  dfree(cb_cnt); dfree(cb_off); dfree(d_total); dfree(d_cnt); dfree(d_cntr);
   dfree(o_T); dfree(o_N); dfree(o_tstat); dfree(o_pstat); dfree(newid);
   dfree(h_key); dfree(h_val);
   dfree(d_ctl); dfree(g_cnt); dfree(g_off);
@@ -3214,20 +3217,34 @@ void Refiner::read_counters() {
   cnt_zero = false;
 }
 
-// End of a pass: the counters to the host's mapped copy (read after the
-// stream synchronisation) and back to zero for the next pass -- one launch
-// in place of a copy and a fill.
-__global__ void k_flush_counters(unsigned long long *cnt, unsigned long long *host) {
-  const int k = threadIdx.x;
-  if (k < CNT_N) {
-    __hip_atomic_store(host + k, cnt[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    cnt[k] = 0ull;
+// End of a pass: the counters, their copies added, to the host's mapped copy
+// (read after the stream synchronisation) and back to zero for the next pass
+// -- one launch in place of a copy and a fill.
+__global__ __launch_bounds__(1024) void k_flush_counters(unsigned long long *cnt,
+                                                         unsigned long long *rep,
+                                                         unsigned long long *host) {
+  __shared__ unsigned long long sum[CNT_STRIDE];
+  constexpr int PER = CNT_REP * CNT_STRIDE / 1024;
+  static_assert(CNT_REP * CNT_STRIDE % 1024 == 0 && 1024 % CNT_STRIDE == 0, "whole copies");
+  const int t = threadIdx.x, k = t % CNT_STRIDE;
+  unsigned long long v = 0ull;
+  for (int q = 0; q < PER; q++) {
+    v += rep[q * 1024 + t];
+    rep[q * 1024 + t] = 0ull;
   }
-  __threadfence_system();
+  if (t < CNT_STRIDE) sum[t] = t < CNT_N ? cnt[t] : 0ull;
+  __syncthreads();
+  if (v) atomicAdd(&sum[k], v);
+  __syncthreads();
+  if (t < CNT_N) {
+    __hip_atomic_store(host + t, sum[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    cnt[t] = 0ull;
+    __threadfence_system();
+  }
 }
 
 void Refiner::flush_counters() {
-  k_flush_counters<<<1, 64, 0, stream>>>(d_cnt, d_host_cnt);
+  k_flush_counters<<<1, 1024, 0, stream>>>(d_cnt, d_cntr, d_host_cnt);
   HC(hipGetLastError());
   HC(hipStreamSynchronize(stream));
   cnt_zero = true;
@@ -3345,6 +3362,7 @@ PassD Refiner::pass_base(int Kc) const {
   ps.pws = c_pws;
   ps.cnt = d_cnt;
   ps.feat = nullptr;
+  ps.cntr = d_cntr;
   ps.ctl = nullptr;
   ps.ids_sel = nullptr;
   ps.slow = c_slow;
@@ -3541,9 +3559,10 @@ int Refiner::run_pass(const int *ids, int nc, int nseg, long long *progress, boo
   // grown here (the pass may still read it)
   const bool listed = list_enc && (long long)ns + nseg <= tmp_list_cap;
   if (listed)
-    compact(PredSencN{m.senc, ns, d_cnt + CNT_SEGWIN}, ns + nseg, tmp_list, nullptr, nullptr,
+    compact(PredSencN{m.senc, ns, d_cnt + (nseg == nc ? CNT_NWIN : CNT_SEGWIN)}, ns + nseg, tmp_list, nullptr, nullptr,
             d_cnt + CNT_NENC);
   flush_counters();
+  if (nseg == nc) h_cnt[CNT_SEGWIN] = h_cnt[CNT_NWIN];
   listed_enc = listed ? (int)h_cnt[CNT_NENC] : -1;
   const int nwin = (int)h_cnt[CNT_NWIN];
   const int nws = (int)h_cnt[CNT_SEGWIN];
@@ -3783,6 +3802,7 @@ void Refiner::run() {
   m.SEG = seg_in;
   pr.ipar = d_ipar;
   HC(hipMemsetAsync(d_cnt, 0, CNT_N * sizeof(unsigned long long), stream));
+  HC(hipMemsetAsync(d_cntr, 0, sizeof(unsigned long long) * CNT_REP * CNT_STRIDE, stream));
   tbegin(K_INIT);
   HC(hipMemcpyAsync(m.P, in_P, sizeof(double2) * np0, hipMemcpyDeviceToDevice, stream));
   m.batched = want_inst ? 1 : 0;
@@ -4119,6 +4139,7 @@ void Refiner::enqueue_seg_pass() {
   ps.nseg = -1;
   ps.ctl = d_ctl;
   ps.cnt = ctl_cnt_ptr();
+  ps.cntr = nullptr;
   if (del_on) {  // vertex deletion first, with its own claim epoch
     DelD dd = del_base();
     dd.ids = tmp_list;
@@ -4167,6 +4188,7 @@ void Refiner::enqueue_bad_pass() {
   ps.ids_sel = sel_list;
   ps.ctl = d_ctl;
   ps.cnt = ctl_cnt_ptr();
+  ps.cntr = nullptr;
   ps.feat = opt.priority == 2 ? c_feat : nullptr;
   launch_cavity(false, opt.grid_cavity, ps);
   if (opt.priority == 2) {
