@@ -485,7 +485,8 @@ __global__ void k_ck_quality(View v, Scratch s, double ga) {
   }
   // one atomic per block and counter: updates of one word cost about 20 ns
   // each, one after the other:
-  // 99 us on 300,000 triangles with one per wave, 20 to 40 with 512 blocks
+  // with one per wave the check of a 30,003-point refinement took 592 us, with
+  // 512 blocks 514
   __shared__ unsigned long long sb, se, sm;
   if (threadIdx.x == 0) {
     sb = se = 0ull;
