@@ -72,3 +72,22 @@ def test_small_rounds_equal_separate_kernels(gpu, n, dist, opt):
     assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
     for f in ("triangles", "neighbors", "segments", "pstatus", "tstatus"):
         assert np.array_equal(getattr(a, f), getattr(b, f)), f
+
+
+@pytest.mark.parametrize("dist,opt", [(0, dict(CHOSEN, priority=1, mix_below=0)),
+                                      (1, dict(claim_iters=2)), (0, dict(mode=0))])
+def test_located_candidates_equal_inline(gpu, dist, opt):
+    """A first bad pass of more than 16,384 candidates is located by a lane per
+    candidate in the host loop; the graph loop's cavities locate their own."""
+    print(f"located dist={dist} {opt}", flush=True)
+    n = 14000
+    P, S0 = gpu.generate_pslg(n, n // 20, L=64.0 * n ** 0.5, maxlen=1280.0, dist=dist,
+                              min_angle=5.0, seed=77)
+    mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    a, sa = _run(gpu, mesh, dict(opt, graph=0, cand_min=1 << 20), 0)
+    b, sb = _run(gpu, mesh, dict(opt, graph=1, cand_min=1 << 20), 0)
+    for k in ("rounds", "inserted", "seg_splits", "giveups", "flips", "cand_evals"):
+        assert sa[k] == sb[k], k
+    assert sa["cand_evals"] > 16384
+    assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
+    assert np.array_equal(a.triangles, b.triangles) and np.array_equal(a.neighbors, b.neighbors)
