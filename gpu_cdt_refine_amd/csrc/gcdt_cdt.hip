@@ -1821,13 +1821,13 @@ void build_cdt_device(const double *points, int np, const int *segs, int ns,
   const int PCAP = 4 * ns + 16;
   Piece *pieces = B.alloc<Piece>(PCAP);
   int *npieces = B.alloc<int>(1);
+  CC(hipMemsetAsync(npieces, 0, sizeof(int), B.st));  // read back also without segments
   int4 *info = nullptr, *info2 = nullptr;
   int *swin = nullptr, *W2 = nullptr;
   int seg_passes = 0, npieces_total = 0;
   if (ns > 0) {
     CC(hipMemcpyAsync(seg, segs, sizeof(int2) * ns, hipMemcpyHostToDevice, B.st));
     CC(hipMemsetAsync(done, 0, sizeof(int) * ns, B.st));
-    CC(hipMemsetAsync(npieces, 0, sizeof(int), B.st));
     std::vector<int> hp(ns);
     for (int s = 0; s < ns; s++) hp[s] = s;
     CC(hipMemcpyAsync(pend, hp.data(), sizeof(int) * ns, hipMemcpyHostToDevice, B.st));

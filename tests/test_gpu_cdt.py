@@ -89,3 +89,20 @@ def test_gpu_cdt_feeds_the_refinement(gpu, oracle):
     c = gpu.check_mesh(r.points, r.triangles, r.neighbors, r.segments, points_in=P,
                        segments_in=S, theta=25.0)
     assert gpu.violations(c) == 0, c
+
+
+@pytest.mark.parametrize("n,dist,seed", [(3, 0, 21), (7, 0, 22), (3000, 0, 23), (5001, 3, 24)])
+def test_gpu_cdt_without_segments(gpu, oracle, n, dist, seed):
+    """A bare point set, right after a build with segments whose freed device
+    memory it may be given: only the hull edges come out as segments."""
+    print(f"gpu cdt without segments n={n}", flush=True)
+    Q, S0 = gpu.generate_pslg(3000, 300, L=500.0, maxlen=50.0, dist=0, min_angle=5.0, seed=20)
+    gpu.build_cdt(Q, S0, device=True)
+    P = gpu.generate_pslg(max(n, 40), 1, L=1000.0, maxlen=500.0, dist=dist, min_angle=5.0,
+                          seed=seed)[0][:n]
+    none = np.zeros((0, 2), np.int32)
+    T, N, S = gpu.build_cdt(P, none, device=True)
+    Th, Nh, Sh = gpu.build_cdt(P, none)
+    assert _canon(T) == _canon(Th) and _segset(S) == _segset(Sh)
+    assert len(S) == int((N == -1).sum())
+    _valid(oracle, P, T, N, S)
