@@ -2171,6 +2171,7 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
     __syncthreads();
     if (listed > SR_ENC) st.ne = -1;
     const bool grow = ovf && base.K < a.kmax;
+    st.grow = grow ? 1 : 0;  // also when this pass is the last
     if (seg_pass) {
       st.seg_passes++;
     } else {
@@ -2196,7 +2197,6 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
       }
       st.np_round = st.np;
     }
-    st.grow = grow ? 1 : 0;
     if (grow || st.ne < 0) {
       passes++;
       break;
@@ -3683,6 +3683,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   st.bad_passes += o.bad_passes;
   st.cand_evals += o.cand_evals;
   add_pass_stats(c);
+  if (o.grow) K = std::min(2 * K, opt.cav_cap_max);
   if (o.code == SR_DONE || o.code == SR_ROUNDS) {
     *done = true;
     return true;
@@ -3700,7 +3701,6 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
       *done = after_bad_pass(nseg1, nc1 - nseg1, nwin, nws, prog, of, prev_win, round);
     return true;
   }
-  if (o.grow) K = std::min(2 * K, opt.cav_cap_max);
   return o.passes > 0;
 }
 

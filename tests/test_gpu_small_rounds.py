@@ -91,3 +91,20 @@ def test_located_candidates_equal_inline(gpu, dist, opt):
     assert sa["cand_evals"] > 16384
     assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
     assert np.array_equal(a.triangles, b.triangles) and np.array_equal(a.neighbors, b.neighbors)
+
+
+@pytest.mark.parametrize("n,seed,rounds,cap", [(20, 1, 1, 4), (40, 1, 3, 8), (60, 2, 1, 8),
+                                               (100, 1, 1, 4)])
+def test_cavity_capacity_at_the_round_limit(gpu, n, seed, rounds, cap):
+    """A pass that overflows a cavity and is also the last round: the capacity
+    a run ends with does not depend on the path its last pass took."""
+    print(f"capacity at round limit n={n} rounds={rounds}", flush=True)
+    P, S0 = gpu.generate_pslg(n, max(1, n // 20), L=64.0 * n ** 0.5, maxlen=1280.0, dist=0,
+                              min_angle=5.0, seed=seed)
+    mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    opt = dict(cav_cap0=cap, max_rounds=rounds)
+    a, sa = _run(gpu, mesh, opt, 0)
+    b, sb = _run(gpu, mesh, opt, 1)
+    assert sa["rounds"] == rounds and sa["rej_overflow"] > 0
+    assert {k: sa[k] for k in SAME} == {k: sb[k] for k in SAME}
+    assert np.array_equal(a.triangles, b.triangles)
