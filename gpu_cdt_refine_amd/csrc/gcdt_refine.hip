@@ -1914,6 +1914,10 @@ constexpr int SR_DEL = 64;
 constexpr int SR_ENC = 512;      // encroached subsegments listed
 constexpr int SR_DIRTY = 8192;   // rewritten triangles listed between two bad passes
 constexpr int SR_PASSES = 128;   // passes of one launch
+constexpr int SR_LIST = 512;     // entries of a list built in the dynamic LDS
+static_assert(SR_LIST > SR_CAP && SR_LIST >= SR_ENC &&
+                  SR_LIST <= (SR_THREADS / DEL_G) * DEL_LDS_INTS,
+              "lists fit the smallest dynamic LDS (small_lds)");
 static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
 
 // The lists k_small_rounds keeps as passes change the mesh.
@@ -1993,14 +1997,18 @@ __global__ __launch_bounds__(SR_THREADS) void k_small_rounds(MeshD m, ParamsD pr
       const uint8_t f0 = t0 >= 0 ? m.tflag[t0] : 0;
       if (tid == 0) s_k = 0;
       __syncthreads();
-      if ((f0 & (TF_ALIVE | TF_BAD | TF_GIVEUP | TF_CHECK)) == (TF_ALIVE | TF_BAD))
-        sm[atomicAdd(&s_k, 1)] = t0;
+      // both appends are bounded: waves already at the rewritten triangles may
+      // have counted past the list before another wave stores its survivors
+      if ((f0 & (TF_ALIVE | TF_BAD | TF_GIVEUP | TF_CHECK)) == (TF_ALIVE | TF_BAD)) {
+        const int p = atomicAdd(&s_k, 1);
+        if (p < SR_LIST) sm[p] = t0;
+      }
       for (int q = tid; q < nd; q += SR_THREADS) {
         const int t = a.dirty[q];
         const uint8_t f = mark_bad_one(m, pr, t, m.tflag[t]);
         if ((f & (TF_ALIVE | TF_BAD | TF_GIVEUP)) == (TF_ALIVE | TF_BAD)) {
           const int p = atomicAdd(&s_k, 1);
-          if (p < 2 * SR_CAP) sm[p] = t;
+          if (p < SR_LIST) sm[p] = t;
         }
       }
       __syncthreads();
