@@ -41,8 +41,7 @@ enum : int {
   ST_REJ_ENC = 1,
   ST_REJ_BLOCKED = 2,
   ST_OVERFLOW = 3,
-  ST_GIVEUP = 4,
-  ST_BIG = 5  // cavity larger than the LDS list; recomputed in global memory
+  ST_GIVEUP = 4
 };
 enum : int {
   CNT_MARKS = 0,
@@ -56,7 +55,6 @@ enum : int {
   CNT_EXACT,
   CNT_ERRORS,
   CNT_VALID,
-  CNT_BIG,
   CNT_DD,
   CNT_SLOW,    // candidates deferred to the exact-predicate kernel
   CNT_SEGWIN,  // winners that split a subsegment
@@ -70,7 +68,7 @@ enum : int {
   CNT_DEL,       // vertices deleted
   CNT_FLIPS,     // flips Lawson's algorithm would make for the pass's changes
   CNT_NENC,      // encroached subsegments after the pass (listed behind its apply)
-  CNT_N = 25
+  CNT_N = 24
 };
 
 #define GCDT_WALK_LIMIT (1 << 22)

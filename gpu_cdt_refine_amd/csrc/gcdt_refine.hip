@@ -2612,7 +2612,7 @@ __device__ void ctl_accumulate(Ctl *c, int nwin) {
   c->acc[A_FP64] += n[CNT_FP64];
   c->acc[A_EXACT] += n[CNT_EXACT];
   c->acc[A_DD] += n[CNT_DD];
-  c->acc[A_BIG] += n[CNT_BIG];
+  c->acc[A_BIG] += n[CNT_SLOW];
   c->acc[A_EXAM_SEG] += n[CNT_EXAM_SEG];
   c->acc[A_EXAM_BAD] += n[CNT_EXAM_BAD];
   c->acc[A_WS_SEG] += n[CNT_WS_SEG];
@@ -3754,7 +3754,7 @@ void Refiner::add_pass_stats(const unsigned long long *c) {
   st.pred_fp64 += c[CNT_FP64];
   st.pred_exact += c[CNT_EXACT];
   st.pred_dd += c[CNT_DD];
-  st.big_cavities += c[CNT_BIG];
+  st.big_cavities += c[CNT_SLOW];
   st.tri_examined_seg += c[CNT_EXAM_SEG];
   st.tri_examined_bad += c[CNT_EXAM_BAD];
   st.ws_ints_seg += c[CNT_WS_SEG];

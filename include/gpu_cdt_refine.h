@@ -211,7 +211,8 @@ typedef struct gcdt_stats {
   long long pred_fp32, pred_fp64, pred_exact; /* predicate stage hits */
   long long n_points, n_triangles, n_subsegs;
   long long cand_evals;  /* bad-pass candidates evaluated */
-  long long big_cavities; /* cavity evaluations that left the LDS fast path */
+  long long big_cavities; /* cavity evaluations that left the LDS fast path: a
+                            cavity beyond cav_lds_cap or an undecided sign */
   long long pred_dd;     /* signs decided by the double-double stage */
   long long tri_examined_seg, tri_examined_bad; /* triangle records the cavity
                             kernels examined (walk steps, seeds, conflict

@@ -42,7 +42,7 @@ SAME = ["rounds", "seg_passes", "bad_passes", "status", "seg_splits", "inserted"
         "rej_encroach", "rej_blocked", "rej_overflow", "giveups", "cand_evals", "deleted", "flips",
         "n_points", "n_triangles", "n_subsegs", "final_cav_cap", "pred_fp32", "pred_fp64",
         "pred_exact", "pred_dd", "tri_examined_seg", "tri_examined_bad", "ws_ints_seg",
-        "ws_ints_bad"]
+        "ws_ints_bad", "big_cavities"]
 
 
 def _run(gpu, mesh, opt, log):
@@ -108,3 +108,20 @@ def test_cavity_capacity_at_the_round_limit(gpu, n, seed, rounds, cap):
     assert sa["rounds"] == rounds and sa["rej_overflow"] > 0
     assert {k: sa[k] for k in SAME} == {k: sb[k] for k in SAME}
     assert np.array_equal(a.triangles, b.triangles)
+
+
+def test_evaluations_off_the_fast_path(gpu):
+    """big_cavities: the evaluations left to the exact kernel.  The number
+    does not depend on the path, grows as the fast path's capacity shrinks,
+    and counts undecided signs alone when every cavity fits."""
+    P, S0 = gpu.generate_pslg(800, 40, L=64.0 * 800 ** 0.5, maxlen=1280.0, dist=0, min_angle=5.0,
+                              seed=900)
+    mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    big = {}
+    for cap in (4, 8, 32):
+        opt = dict(CHOSEN, priority=1, mix_below=0, cav_lds_cap=cap, cav_cap0=32)
+        st = [_run(gpu, mesh, opt, log)[1] for log in (0, 1)]
+        st.append(_run(gpu, mesh, dict(opt, graph=1), 0)[1])
+        assert st[0]["big_cavities"] == st[1]["big_cavities"] == st[2]["big_cavities"], cap
+        big[cap] = st[0]["big_cavities"]
+    assert big[4] > big[8] > big[32]
