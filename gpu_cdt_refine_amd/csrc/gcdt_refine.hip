@@ -1905,7 +1905,6 @@ __global__ __launch_bounds__(DEL_BLOCK) void k_del_apply(MeshD m, DelD dd) {
 // ---------------------------------------------------------------------------
 constexpr int SR_WAVES = 8, SR_THREADS = 64 * SR_WAVES;
 constexpr int SR_LG = 16;        // lanes per cavity
-constexpr int SR_K = 32;         // largest cavity held in LDS
 constexpr int SR_CAP = 256;      // candidates of a pass
 // subsegments of a pass that deletes vertices: 32 groups of lanes serve their
 // 2 nominations each, 4 rounds of walks around a vertex (2,999 points in Chew
@@ -1919,6 +1918,10 @@ static_assert(SR_LIST > SR_CAP && SR_LIST >= SR_ENC &&
                   SR_LIST <= (SR_THREADS / DEL_G) * DEL_LDS_INTS,
               "lists fit the smallest dynamic LDS (small_lds)");
 static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
+// dynamic LDS, beside about 20 KiB of lists: cavities of up to 69 triangles.
+// While the caller's capacity (cav_lds_cap, up to the pass's K) does not fit,
+// small passes take the separate kernels, whose blocks of one wave hold it.
+constexpr size_t SR_LDS = 136 * 1024;
 
 // The lists k_small_rounds keeps as passes change the mesh.
 struct ListTrace {
@@ -2790,7 +2793,7 @@ Refiner::Refiner(const gcdt_options &o) : opt(o) {
   for (const void *f : cav)
     HC(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, BIG_LDS_BYTES));
   HC(hipFuncSetAttribute((const void *)k_small_rounds, hipFuncAttributeMaxDynamicSharedMemorySize,
-                         (int)small_lds(SR_K)));
+                         (int)SR_LDS));
 
   dalloc(&d_total, 4);
   dalloc(&d_cnt, CNT_N);
@@ -3604,7 +3607,8 @@ void Refiner::ensure_feat(int nc) {
 // A pass of nc candidates, nseg of them subsegments, that k_small_rounds
 // takes (the training logs need the separate kernels).
 bool Refiner::small_pass(int nc, int nseg) const {
-  return nc > 0 && nc <= SR_CAP && !(del_on && nseg > SR_DEL) && !opt.log_training && (opt.priority != 2 || mlp_params);
+  return nc > 0 && nc <= SR_CAP && !(del_on && nseg > SR_DEL) && !opt.log_training &&
+         (opt.priority != 2 || mlp_params) && small_lds(std::min(K, opt.cav_lds_cap)) <= SR_LDS;
 }
 
 // Rounds from the segment check on, while their passes are small: ne
@@ -3630,7 +3634,6 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   if (!cnt_zero) HC(hipMemsetAsync(d_cnt, 0, CNT_N * sizeof(unsigned long long), stream));
   cnt_zero = true;
   PassD ps = pass_base(K);
-  ps.Kf = std::min(ps.Kf, SR_K);
   SmallArgs a{};
   a.st.np = np;
   a.st.nt = nt;
@@ -3668,7 +3671,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   a.capT = capT;
   a.capS = capS;
   a.out = d_sr_out;
-  const size_t lds = small_lds(std::min(K, ps.Kf));
+  const size_t lds = small_lds(std::min(K, opt.cav_lds_cap));
   tbegin(K_SMALL);
   k_small_rounds<<<1, SR_THREADS, lds, stream>>>(m, pr, ps, a);
   tend(K_SMALL, 0);
