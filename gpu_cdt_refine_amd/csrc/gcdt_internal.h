@@ -55,7 +55,6 @@ enum KernelId {
   K_MLP,
   K_DEL_SCAN,
   K_DEL_APPLY,
-  K_SMALL,
   K_NKERN
 };
 

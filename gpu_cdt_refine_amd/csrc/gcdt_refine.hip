@@ -3167,8 +3167,7 @@ const char *Refiner::kname(int id) {
   static const char *names[] = {"init",       "mark_bad", "compact",
                                 "seg_cavity", "bad_cavity", "claim",
                                 "win",        "apply",      "export",
-                                "mlp",        "del_scan",   "del_apply",
-                                "small_rounds"};
+                                "mlp",        "del_scan",   "del_apply"};
   return names[id];
 }
 
@@ -3605,10 +3604,12 @@ void Refiner::ensure_feat(int nc) {
 }
 
 // A pass of nc candidates, nseg of them subsegments, that k_small_rounds
-// takes (the training logs need the separate kernels).
+// takes (the training logs need the separate kernels, and a profile's rows
+// each hold all of one step's work, as the statistics count it).
 bool Refiner::small_pass(int nc, int nseg) const {
   return nc > 0 && nc <= SR_CAP && !(del_on && nseg > SR_DEL) && !opt.log_training &&
-         (opt.priority != 2 || mlp_params) && small_lds(std::min(K, opt.cav_lds_cap)) <= SR_LDS;
+         !opt.profile && (opt.priority != 2 || mlp_params) &&
+         small_lds(std::min(K, opt.cav_lds_cap)) <= SR_LDS;
 }
 
 // Rounds from the segment check on, while their passes are small: ne
@@ -3672,9 +3673,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   a.capS = capS;
   a.out = d_sr_out;
   const size_t lds = small_lds(std::min(K, opt.cav_lds_cap));
-  tbegin(K_SMALL);
   k_small_rounds<<<1, SR_THREADS, lds, stream>>>(m, pr, ps, a);
-  tend(K_SMALL, 0);
   HC(hipGetLastError());
   HC(hipStreamSynchronize(stream));
   const SmallState &o = sr_out->st;

@@ -123,7 +123,9 @@ typedef struct gcdt_options {
                             conflict degree, higher first (learned_shift) */
   int pred_mode;         /* 0 = FP64 filter + exact; 1 = FP32 semi-static,
                             then FP64, then exact */
-  int profile;           /* 1 = time every kernel launch with HIP events */
+  int profile;           /* 1 = time every kernel launch with HIP events (small
+                            passes then take the separate kernels as well, so
+                            that a step's row holds all of its work) */
   int device;            /* HIP device ordinal */
   int cand_factor;       /* a bad pass evaluates at most max(cand_min,
                             cand_factor * winners of the previous bad pass)

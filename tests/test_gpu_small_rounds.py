@@ -144,3 +144,26 @@ def test_fast_path_capacity_above_the_default(gpu, oracle, k, cap):
     if cap >= k:  # the ring's fan of k - 2 triangles is one cavity: it fits now
         narrow = _run(gpu, mesh, dict(opt, cav_lds_cap=32), 0)[1]
         assert narrow["big_cavities"] > sa["big_cavities"]
+
+
+def test_profile_rows_hold_every_pass(gpu):
+    """profile = 1: the cavity rows time every pass that the statistics count,
+    the small ones too, and profiling does not change the mesh."""
+    P, S0 = gpu.generate_pslg(2000, 100, L=64.0 * 2000 ** 0.5, maxlen=1280.0, dist=0,
+                              min_angle=5.0, seed=400)
+    mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    res = []
+    for profile in (0, 1):
+        s = gpu.Session(*mesh, theta=25.0, mode=1, profile=profile, priority=1, **CHOSEN)
+        try:
+            st = s.run()
+            res.append((st, s.download(), s.kernel_times()))
+        finally:
+            s.close()
+    (sa, a, _), (sb, b, kt) = res
+    assert {k: sa[k] for k in SAME} == {k: sb[k] for k in SAME}
+    assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
+    assert kt["bad_cavity"]["launches"] == sb["bad_passes"]
+    assert kt["bad_cavity"]["items"] == sb["cand_evals"]
+    assert kt["seg_cavity"]["launches"] == sb["seg_passes"]
+    assert kt["apply"]["items"] == sb["inserted"] + sb["seg_splits"]
