@@ -1,6 +1,7 @@
 """GPU refinement vs the CPU oracle: bit-identical meshes, exact invariants,
 run-to-run determinism.  Inputs are seeded PSLGs triangulated by the
-reference's Triangle ("pzQnc", mesh.cpp:397)."""
+reference's Triangle ("pzQnc", mesh.cpp:397), or by the host builder where
+Triangle is not built."""
 import numpy as np
 import pytest
 

@@ -88,9 +88,42 @@ def test_located_candidates_equal_inline(gpu, dist, opt):
     b, sb = _run(gpu, mesh, dict(opt, graph=1, cand_min=1 << 20), 0)
     for k in ("rounds", "inserted", "seg_splits", "giveups", "flips", "cand_evals"):
         assert sa[k] == sb[k], k
-    assert sa["cand_evals"] > 16384
     assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
     assert np.array_equal(a.triangles, b.triangles) and np.array_equal(a.neighbors, b.neighbors)
+    # one round holds one bad pass: the first is large enough to be located
+    first = _run(gpu, mesh, dict(opt, graph=0, cand_min=1 << 20, max_rounds=1), 0)[1]
+    assert first["bad_passes"] == 1 and first["cand_evals"] > 16384
+
+
+def _encroached(P, T, S):
+    """Subsegments with the apex of an adjacent triangle strictly inside their
+    diametral circle."""
+    key = lambda a, b: np.minimum(a, b).astype(np.int64) * len(P) + np.maximum(a, b)
+    want = key(S[:, 0], S[:, 1])
+    hit = []
+    for j in range(3):
+        c, a, b = T[:, j], T[:, (j + 1) % 3], T[:, (j + 2) % 3]
+        inside = ((P[a] - P[c]) * (P[b] - P[c])).sum(1) < 0
+        hit.append(key(a[inside], b[inside]))
+    return int(np.isin(want, np.concatenate(hit)).sum())
+
+
+@pytest.mark.parametrize("opt", [dict(CHOSEN, priority=1, mix_below=0), dict(mode=0)])
+def test_located_subsegments_equal_inline(gpu, opt):
+    """A first segment pass of more than 16,384 subsegments, the same way."""
+    print(f"located subsegments {opt}", flush=True)
+    n = 60000
+    P, S0 = gpu.generate_pslg(n, 40000, L=64.0 * n ** 0.5, maxlen=400.0, dist=0, min_angle=5.0,
+                              seed=78)
+    mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    assert _encroached(P, mesh[1], mesh[3]) > 16384
+    o = dict(opt, theta=20.7)
+    a, sa = _run(gpu, mesh, dict(o, graph=0), 0)
+    b, sb = _run(gpu, mesh, dict(o, graph=1), 0)
+    for k in ("rounds", "seg_passes", "inserted", "seg_splits", "giveups", "flips", "cand_evals"):
+        assert sa[k] == sb[k], k
+    assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
+    assert np.array_equal(a.triangles, b.triangles) and np.array_equal(a.segments, b.segments)
 
 
 @pytest.mark.parametrize("n,seed,rounds,cap", [(20, 1, 1, 4), (40, 1, 3, 8), (60, 2, 1, 8),
@@ -167,3 +200,37 @@ def test_profile_rows_hold_every_pass(gpu):
     assert kt["bad_cavity"]["items"] == sb["cand_evals"]
     assert kt["seg_cavity"]["launches"] == sb["seg_passes"]
     assert kt["apply"]["items"] == sb["inserted"] + sb["seg_splits"]
+
+
+# what does not depend on how many lanes test a triangle at the same time
+LANE_SAME = [k for k in SAME if not k.startswith(("pred_", "tri_examined"))]
+
+
+@pytest.mark.parametrize("case", ["uniform", "overflow", "deferred", "chew", "ring"])
+@pytest.mark.parametrize("lanes", [8, 32, 64])
+def test_lane_groups_equal_the_default(gpu, oracle, case, lanes):
+    """The filtered cavity kernel with 8, 32 and 64 lanes per candidate against
+    16: cavities that overflow the capacity, that leave the fast path, and
+    stars longer than a lane group.  (The training logs keep every pass out of
+    the one-launch rounds, whose group size is fixed.)"""
+    print(f"lane groups {case} {lanes}", flush=True)
+    opt = {"uniform": dict(CHOSEN, priority=1), "overflow": dict(cav_cap0=4),
+           "deferred": dict(CHOSEN, priority=1, cav_lds_cap=6), "chew": dict(mode=0, claim_iters=2),
+           "ring": dict(CHOSEN, priority=1, cav_cap0=128, cav_lds_cap=128)}[case]
+    if case == "ring":
+        from test_gpu_parity import circle_pslg
+        mesh = circle_pslg(oracle)
+    else:
+        P, S0 = gpu.generate_pslg(2500, 125, L=64.0 * 50, maxlen=1280.0, dist=1, min_angle=5.0,
+                                  seed=500)
+        mesh = (P,) + tuple(gpu.build_cdt(P, S0))
+    a, sa = _run(gpu, mesh, opt, 1)
+    b, sb = _run(gpu, mesh, dict(opt, cavity_lanes=lanes), 1)
+    assert {k: sa[k] for k in LANE_SAME} == {k: sb[k] for k in LANE_SAME}
+    if case == "overflow":
+        assert sa["rej_overflow"] > 0
+    if case == "deferred":
+        assert sa["big_cavities"] > 1000
+    assert np.array_equal(a.points.view(np.uint64), b.points.view(np.uint64))
+    for f in ("triangles", "neighbors", "segments", "pstatus", "tstatus"):
+        assert np.array_equal(getattr(a, f), getattr(b, f)), f
