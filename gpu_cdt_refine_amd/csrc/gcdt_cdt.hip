@@ -921,7 +921,8 @@ __global__ __launch_bounds__(SCAN_CHUNK) void k_scan_scatter(const int *f, int n
 // makes no progress the host grows the capacity (fewer segments a pass).
 constexpr int KSEG0 = 512;
 // per-segment workspace for capacity k: region | left chain | right chain |
-// boundary u, v, outer | new triangles (3 ints) | Anglada stack (4 ints)
+// boundary u, v, outer | new triangles (3 ints) | 4 ints: the stack of
+// sub-problems (two an entry), then the sorted slots
 __host__ __device__ constexpr size_t ws_seg(int k) {
   return (size_t)k + 2 * ((size_t)k + 2) + 3 * ((size_t)k + 2) + 3 * (size_t)k + 4 * ((size_t)k + 2);
 }

@@ -29,11 +29,11 @@
 
 namespace gcdt {
 
-// Inference: the weights converted to BF16 once
-// per block and kept in LDS, four waves per block, each wave taking 16 rows
-// at a time; layer 2 on the 16x16x32 MFMA.  Same roundings as the training
-// forward (inputs, weights and hidden activations in BF16, FP32 accumulate);
-// only layer 2's accumulation order differs.
+// Inference: the weights converted to BF16 once per block and kept in LDS,
+// four waves per block, each wave taking 16 rows at a time; layer 2 on the
+// 16x16x32 MFMA.  The gradient kernel's forward pass makes the same products
+// and roundings (inputs, weights and hidden activations in BF16, FP32
+// accumulate).
 constexpr int INF_WAVES = 4;
 __global__ __launch_bounds__(64 * INF_WAVES) void k_mlp_infer(const float *X, int n,
                                                               const float *P, float *y,

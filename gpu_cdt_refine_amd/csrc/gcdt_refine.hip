@@ -452,10 +452,6 @@ __device__ __forceinline__ void flush_stats(unsigned long long *cnt,
   if (st.dd_hits) atomicAdd(&cnt[CNT_DD], (unsigned long long)st.dd_hits);
 }
 
-__device__ __forceinline__ void mark_enc(const MeshD &m, int s,
-                                         unsigned long long *cnt) {
-  if (atomicCAS(&m.senc[s], 0, 1) == 0) atomicAdd(&cnt[CNT_MARKS], 1ull);
-}
 // Marks subsegment s encroached; true if this call marked it.
 __device__ __forceinline__ bool mark_enc_local(const MeshD &m, int s) {
   return atomicCAS(&m.senc[s], 0, 1) == 0;
@@ -534,9 +530,11 @@ constexpr int EXACT_GRID = 512;
 // boundary / disk / orientation checks, the ring and the encroachment test
 // run lane-parallel over the cavity's edges.  Loops that contain a barrier or
 // a ballot run a group-uniform number of times.  Large passes are bound by
-// instruction issue (an evaluation is a few thousand wave instructions, and 5
-// waves per SIMD hide most of the gathers), small ones by the length of the
-// chain of gathers and LDS round trips; both want fewer, wider steps.
+// the gathers and the instructions together: at 10^6 points a wave waits 59%
+// of its cycles and issues 32%, and 3.5 waves on a SIMD keep its vector ALU
+// busy about half of the time (rocprofv3 counters).  Small ones are bound by
+// the length of the chain of gathers and LDS round trips.  Both want fewer,
+// wider steps.
 // On 10^6 points the work list, the lane-per-candidate location and the star
 // order by pointer doubling took bad cavities from 63.4 to 48.3 ms and segment
 // cavities from 23.1 to 17.2 ms (three refinements, small passes left out).
@@ -1886,7 +1884,7 @@ __global__ __launch_bounds__(DEL_BLOCK) void k_del_apply(MeshD m, DelD dd) {
 // Small passes: whole rounds in one launch of one block.
 //
 // A pass over few candidates is a chain of 8 to 16 dependent launches (about
-// 4 us each for almost no work) and a host round trip.  Here one block of 16
+// 4 us each for almost no work) and a host round trip.  Here one block of 8
 // waves runs the same steps with block barriers between them, pass after
 // pass, while every pass has at most SR_CAP candidates.  Steps and order are
 // the separate kernels' (the same device functions), so the mesh is the same

@@ -29,8 +29,8 @@ __device__ __forceinline__ floatx4 mfma(bf16x4 a, bf16x4 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-// gfx950's double-K BF16 MFMA (v_mfma_f32_16x16x32_bf16), used by the
-// inference kernel's 64-wide hidden layer: two instructions per 16x16 output
+// gfx950's double-K BF16 MFMA (v_mfma_f32_16x16x32_bf16), used for the 64-wide
+// hidden layer by inference and by the gradient kernel: two instructions per 16x16 output
 // block instead of four.  Operand layout (checked by k_mfma_probe32 against a
 // host product): A[16][32]: lane l holds row l%16, k = 8*(l/16) + 0..7;
 // B[32][16]: lane l holds col l%16, k = 8*(l/16) + 0..7; D as for 16x16x16.

@@ -152,7 +152,8 @@ typedef struct gcdt_options {
   int cavity_lanes;      /* lanes per candidate in the cavity kernel: 8, 16,
                             32 or 64 (a wave evaluates 64/cavity_lanes
                             candidates at once; default 16; widened when the
-                            groups' LDS would not fit) */
+                            groups' LDS would not fit; always 16 in the
+                            one-launch rounds of small passes) */
   int cav_lds_cap;       /* cavities of up to this many triangles are built
                             in the filtered kernel's LDS; larger ones (and
                             undecided signs) go to the exact kernel, which

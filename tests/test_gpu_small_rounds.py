@@ -1,7 +1,8 @@
 """Runs of small passes in one launch (k_small_rounds) against the separate
-kernels.  The training logs need the separate kernels, so the same options
-with log_training = 1 never take the one-launch path: mesh and statistics have
-to be equal bit for bit.  The inputs cross the limits of the path: passes of
+kernels, and the separate kernels' own variants against each other.  The
+training logs need the separate kernels, so the same options with log_training
+= 1 never take the one-launch path: mesh and statistics have to be equal bit
+for bit.  The inputs cross the limits of the path: passes of
 more and fewer candidates than it takes, cavities beyond its LDS and undecided
 signs (left to the exact kernel inside a pass), capacity doubling and mesh
 growth, the selection by priority, a round limit, and lists reallocated while
