@@ -1898,8 +1898,11 @@ __global__ __launch_bounds__(DEL_BLOCK) void k_del_apply(MeshD m, DelD dd) {
 // Bound by the chain of gathers and LDS round trips of the cavities (about half
 // of a pass), on one CU.  A pass of a 300-point refinement takes 50 us, where
 // its launches took 85 to 110 with the round trip.  8 waves with 256 registers:
-// 41,003 points 22.1 ms a call, 22.8 with 16 waves and spills.  SR_CAP: a few
-// batches of cavities on the one CU still cost less than the launches saved.
+// 41,003 points 22.1 ms a call, 22.8 with 16 waves and spills.  SR_CAP 128 /
+// 256 / 384 / 512: 2.80 / 2.91 / 3.20 / 3.97 ms a call at 300 points, 10.7 /
+// 10.8 / 11.1 / 11.2 at 2,999 (Chew mode), 18.6 / 18.6 / 18.9 / 19.5 at 41,003:
+// beyond 256 candidates the one CU's batches of cavities cost more than the
+// launches they save.
 // ---------------------------------------------------------------------------
 constexpr int SR_WAVES = 8, SR_THREADS = 64 * SR_WAVES;
 constexpr int SR_LG = 16;        // lanes per cavity
