@@ -1919,10 +1919,13 @@ static_assert(SR_LIST > SR_CAP && SR_LIST >= SR_ENC &&
                   SR_LIST <= (SR_THREADS / DEL_G) * DEL_LDS_INTS,
               "lists fit the smallest dynamic LDS (small_lds)");
 static_assert(SR_CAP <= SR_THREADS && SR_ENC <= SR_THREADS, "one list entry per thread");
-// dynamic LDS, beside about 20 KiB of lists: cavities of up to 69 triangles.
-// While the caller's capacity (cav_lds_cap, up to the pass's K) does not fit,
-// small passes take the separate kernels, whose blocks of one wave hold it.
-constexpr size_t SR_LDS = 136 * 1024;
+// Largest cavity held in the launch's LDS: 136 KiB for 32 groups of lanes, beside
+// about 20 KiB of lists.  Larger ones go to the exact kernel even if the caller's
+// capacity (cav_lds_cap) allows them: with a capacity of 128, inputs of 100 and
+// 60,000 points take 2.9 and 14.6 ms a run that way, 3.6 and 15.5 with only as
+// many waves as the capacity leaves room for, 4.6 and 16.1 with the separate
+// kernels.
+constexpr int SR_K = 69;
 
 // The lists k_small_rounds keeps as passes change the mesh.
 struct ListTrace {
@@ -2794,7 +2797,7 @@ Refiner::Refiner(const gcdt_options &o) : opt(o) {
   for (const void *f : cav)
     HC(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, BIG_LDS_BYTES));
   HC(hipFuncSetAttribute((const void *)k_small_rounds, hipFuncAttributeMaxDynamicSharedMemorySize,
-                         (int)SR_LDS));
+                         (int)small_lds(SR_K)));
 
   dalloc(&d_total, 4);
   dalloc(&d_cnt, CNT_N);
@@ -3609,8 +3612,7 @@ void Refiner::ensure_feat(int nc) {
 // each hold all of one step's work, as the statistics count it).
 bool Refiner::small_pass(int nc, int nseg) const {
   return nc > 0 && nc <= SR_CAP && !(del_on && nseg > SR_DEL) && !opt.log_training &&
-         !opt.profile && (opt.priority != 2 || mlp_params) &&
-         small_lds(std::min(K, opt.cav_lds_cap)) <= SR_LDS;
+         !opt.profile && (opt.priority != 2 || mlp_params);
 }
 
 // Rounds from the segment check on, while their passes are small: ne
@@ -3636,6 +3638,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   if (!cnt_zero) HC(hipMemsetAsync(d_cnt, 0, CNT_N * sizeof(unsigned long long), stream));
   cnt_zero = true;
   PassD ps = pass_base(K);
+  ps.Kf = std::min(ps.Kf, SR_K);
   SmallArgs a{};
   a.st.np = np;
   a.st.nt = nt;
@@ -3673,7 +3676,7 @@ bool Refiner::run_small(const int *enc, int ne, const int *bad, int nb, int *rou
   a.capT = capT;
   a.capS = capS;
   a.out = d_sr_out;
-  const size_t lds = small_lds(std::min(K, opt.cav_lds_cap));
+  const size_t lds = small_lds(std::min(K, ps.Kf));
   k_small_rounds<<<1, SR_THREADS, lds, stream>>>(m, pr, ps, a);
   HC(hipGetLastError());
   HC(hipStreamSynchronize(stream));

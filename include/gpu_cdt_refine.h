@@ -157,7 +157,8 @@ typedef struct gcdt_options {
   int cav_lds_cap;       /* cavities of up to this many triangles are built
                             in the filtered kernel's LDS; larger ones (and
                             undecided signs) go to the exact kernel, which
-                            holds cav_cap triangles (default 32) */
+                            holds cav_cap triangles (default 32; at most 69
+                            count in the one-launch rounds of small passes) */
   int learned_shift;     /* learned priority: claims compare shortest-edge
                             buckets coarsened by 2^learned_shift half-octaves,
                             then the predicted conflict degree (higher first);
